@@ -17,6 +17,7 @@ extern "C" {
 #define FMB_MAXLEV 12 /* levels 0..11; the reference caps at 10 (octree.c:637) */
 #define FMB_NOFF 343  /* offset codes (dx+3)*49+(dy+3)*7+(dz+3)               */
 #define FMB_NDIST 15  /* distinct |offset|^2 among M2L offsets                */
+#define FMB_NCLASS 34 /* (|dz|, dx^2 + dy^2) classes of the M2L offsets        */
 
 struct fmb_mesh {
   int nv, nf;
@@ -75,6 +76,10 @@ typedef struct fmb_opset {
                         hi and lo parts [nbeta][2][hb_half]                 */
   size_t hb_half;
   int gws_grid;      /* persistent workgroups sharing d_gws                  */
+  /* target-stationary M2L: rotation tables per offset class [34][ts_hstride]
+   * and phases [343][2][ts_P] of the forward and the transposed pass        */
+  void *d_ts_H, *d_ts_phase[2];
+  int ts_hstride, ts_P;
 } fmb_opset;
 
 /* one translation kind at one level on the matrix cores */
@@ -93,6 +98,12 @@ typedef struct fmb_rcr_tab {
   size_t cpad_stride;   /* complex values per coaxial matrix in d_Cpad     */
   int hlen;             /* values of the padded rotation blocks n < P      */
   int tiled;            /* M2L: chunks in tile-major order (else offset-major) */
+  /* target-stationary M2L, per opset (ts_slots 0: not set up): sums of a
+   * workgroup, two pair lists by (group, class) with their boxes per group,
+   * unit schedule, coaxial tables                                          */
+  int ts_slots[2], ts_tgrp[2][2], ts_cstride[2];
+  void *d_ts_pairs[2][2], *d_ts_C[2];
+  int *d_ts_seg[2][2], *d_ts_sched[2];
 } fmb_rcr_tab;
 
 struct fmb_plan {
@@ -108,6 +119,9 @@ struct fmb_plan {
   int off_beta[FMB_NOFF];
   double off_phi[FMB_NOFF];
   int off_dist[FMB_NOFF];
+  /* M2L offset classes: offsets that differ by a rotation about z or the
+   * reflection z -> -z share a polar angle (dz >= 0) and a distance        */
+  int off_class[FMB_NOFF], class_beta[FMB_NCLASS], class_dist[FMB_NCLASS];
   /* octant o of a child: child centre - parent centre = (bits - 1/2) side */
   int m2m_beta[8], l2l_beta[8]; /* t = parent - child, t = child - parent  */
   double m2m_phi[8], l2l_phi[8];

@@ -141,6 +141,41 @@ int fmbh_split_rot(const double *d_H64, int nbeta, int Pmax, const int *d_hboff,
 int fmbh_pad_coax(int prec, const void *d_C, int ncoax, int P, int pin,
                   int pout, const int *d_coff, size_t pstride, void *d_Cp,
                   void *stream);
+/* ---- target-stationary M2L of low orders (rcr_ts.hip) */
+#define FMBH_TS_PMAX 16    /* largest order                                 */
+#define FMBH_TS_WAVES64 16 /* waves of a workgroup in the FP64 pass         */
+#define FMBH_TS_WAVES32 8  /* in the FP32 pass                              */
+typedef struct fmbh_ts_job {
+  const void *pairs; /* int2 {source box, place of the target in its group |
+                        offset code << 8}, by (group, class)                */
+  const int *seg;    /* [group][class] first pair, and the end              */
+  int npairs, ngroups, tgrp, nbox; /* tgrp: boxes of a group                */
+  int slots;         /* target vectors that a workgroup sums                */
+  int p;
+  const void *phase; /* [offset code][parity of n][pstride]                 */
+  int pstride;
+  const void *H;     /* rotation tables of the classes                      */
+  int hstride;
+  const void *C;     /* coaxial tables of the distances                     */
+  int cstride;
+  const int *cdist;  /* host: distance of each class                        */
+  const int *sched;
+  const void *in;
+  void *out;
+} fmbh_ts_job;
+/* LDS of a workgroup */
+size_t fmbh_ts_lds_bytes(int p, int prec, int slots);
+int fmbh_ts_run(const fmbh_ts_job *j, int prec, int nrhs, void *stream);
+/* level l's pairs by (group of tgrp targets, class), allocated here; h_cls:
+ * class of each offset code */
+int fmbh_ts_lists(const fmb_tree *t, int l, int tgrp, const int *h_cls, void **d_pairs,
+                  int **d_seg, void *stream);
+/* operator tables (layouts there) from the FP64 rotation blocks and the
+ * opset's scaled coaxial matrices */
+int fmbh_ts_rot(int prec, const double *d_H64, int Pmax, int P, const int *d_cbeta,
+                const int *d_hoff, int hstride, void *out, void *stream);
+int fmbh_ts_coax(int prec, const void *d_C, int p, const int *d_coff, int cstride, void *out,
+                 void *stream);
 int fmbh_l2l(const fmb_plan *pl, int op, int l, int nrhs, void *stream);
 int fmbh_l2p_near(const fmb_plan *pl, int op, int nrhs, int parts,
                   void *stream);

@@ -2,6 +2,9 @@
 #ifndef FMB_HOST_H
 #define FMB_HOST_H
 #include "../fmb_internal.h"
+/* defaults of m2l_tile and m2l_tile_min_mb */
+#define RCR_TILE 256
+#define RCR_TILE_MIN_MB 256
 void fmbx_gauss_legendre(int n, double *x, double *w);
 int fmbx_tri_rule(int rule, int order, double **out);
 void fmbx_abs_hn(int nmax, double x, double *out);

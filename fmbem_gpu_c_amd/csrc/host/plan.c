@@ -38,8 +38,8 @@ void fmb_plan_params_default(fmb_plan_params *p) {
   p->near_ratio = 2.0;
   p->nedge = 24;
   p->nrhs_max = 1;
-  p->m2l_tile = 256; /* measured: level-7 M2L 70.0 -> 66.5 ms (FP32), 128 -> 116 ms (FP64) */
-  p->m2l_tile_min_mb = 256;
+  p->m2l_tile = RCR_TILE; /* measured: level-7 M2L 70.0 -> 66.5 ms (FP32), 128 -> 116 ms (FP64) */
+  p->m2l_tile_min_mb = RCR_TILE_MIN_MB;
 }
 
 static const int k_dist2[FMB_NDIST] = {4, 5, 6, 8, 9, 10, 11, 12,
@@ -150,6 +150,13 @@ static void opset_free_rot(fmb_opset *o) {
     fmbh_free(o->d_phase_c[i]);
     o->d_phase[i] = o->d_phase_c[i] = NULL;
   }
+  fmbh_free(o->d_ts_H);
+  for (int i = 0; i < 2; i++) {
+    fmbh_free(o->d_ts_phase[i]);
+    o->d_ts_phase[i] = NULL;
+  }
+  o->d_ts_H = NULL;
+  o->ts_P = 0;
   o->hpad_stride = 0;
 }
 
@@ -225,6 +232,20 @@ static int plan_geometry(fmb_plan *pl, void *stream) {
     pl->off_beta[o] = beta_of(pl, dz / sqrt((double)d2));
     pl->off_dist[o] = dist_class(d2);
     pl->off_phi[o] = atan2((double)dy, (double)dx);
+  }
+  int ncls = 0, key[FMB_NCLASS];
+  for (int o = 0; o < FMB_NOFF; o++) {
+    int dx = o / 49 - 3, dy = (o / 7) % 7 - 3, dz = o % 7 - 3, c = 0;
+    pl->off_class[o] = 0;
+    if (pl->off_beta[o] < 0) continue;
+    int id = (dx * dx + dy * dy) * 4 + abs(dz);
+    while (c < ncls && key[c] != id) c++;
+    if (c == ncls) {
+      key[ncls++] = id;
+      pl->class_beta[c] = pl->off_beta[fmb_off_code(dx, dy, abs(dz))];
+      pl->class_dist[c] = pl->off_dist[o];
+    }
+    pl->off_class[o] = c;
   }
   for (int oct = 0; oct < 8; oct++) {
     double d[3] = {((oct >> 2) & 1) - 0.5, ((oct >> 1) & 1) - 0.5, (oct & 1) - 0.5};

@@ -371,6 +371,229 @@ static int plan_tab(fmb_plan *pl, fmb_rcr_tab *tb, int pin, int pout,
   return rc;
 }
 
+/* ---- target-stationary M2L of low orders (csrc/hip/rcr_ts.hip) ---- */
+
+/* offsets of the table blocks of one class (rotations of degrees n < p) or
+ * one distance (coaxial |m| < p), in values; returns their total.  Layouts:
+ * k_ts_rot and k_ts_coax. */
+static int ts_blocks(int prec, int rot, int p, int *off) {
+  int o = 0;
+  for (int i = 0; i < p; i++) {
+    const int rg = ((rot ? i + 1 : p - i) + 3) / 4; /* row groups */
+    off[i] = o;
+    if (prec == FMB_FP64)
+      o += (rot ? 2 : 4) * rg * 64;
+    else
+      o += rot ? (rg + 1) / 2 * 256 : 512;
+  }
+  return o;
+}
+
+/* rotation tables and phases of opset o, orders up to FMBH_TS_PMAX */
+static int ts_rot_setup(fmb_plan *pl, fmb_opset *o, void *stream) {
+  const int P = pl->Pmax < FMBH_TS_PMAX ? pl->Pmax : FMBH_TS_PMAX;
+  int hoff[FMBH_TS_PMAX], *d_hoff = NULL, *d_cb = NULL, rc;
+  o->ts_P = P;
+  o->ts_hstride = ts_blocks(o->prec, 1, P, hoff);
+  size_t bytes = o->csz / 2 * (size_t)o->ts_hstride * FMB_NCLASS;
+  if ((rc = fmbh_malloc(&o->d_ts_H, bytes))) return rc;
+  pl->bytes += bytes;
+  rc = fmbh_malloc((void **)&d_hoff, sizeof(int) * P);
+  if (!rc) rc = fmbh_malloc((void **)&d_cb, sizeof(int) * FMB_NCLASS);
+  if (!rc) rc = fmbh_h2d(d_hoff, hoff, sizeof(int) * P, stream);
+  if (!rc) rc = fmbh_h2d(d_cb, pl->class_beta, sizeof(int) * FMB_NCLASS, stream);
+  if (!rc)
+    rc = fmbh_ts_rot(o->prec, (const double *)pl->ops[0].d_H, pl->Pmax, P, d_cb, d_hoff,
+                     o->ts_hstride, o->d_ts_H, stream);
+  /* row (offset, parity of n): e^{i m phi} s^(m + n), s = -1 for an offset
+   * below its class's direction (dz < 0): the reflection z -> -z multiplies
+   * coefficient (n, m) by (-1)^(n + m).  The transposed pass takes the pair
+   * of the opposite offset backwards: that offset's angles, conjugated. */
+  const size_t n = (size_t)FMB_NOFF * 2 * P;
+  double *w = (double *)malloc(sizeof(double) * 2 * n);
+  float *f = (float *)malloc(sizeof(float) * 2 * n);
+  if (!rc && (!w || !f)) rc = fmb_set_error(FMB_ERR_NOMEM, "phase tables");
+  for (int tr = 0; tr < 2 && !rc; tr++) {
+    for (int off = 0; off < FMB_NOFF; off++) {
+      const int dx = off / 49 - 3, dy = (off / 7) % 7 - 3, dz = off % 7 - 3;
+      const double phi = pl->off_phi[tr ? fmb_off_code(-dx, -dy, -dz) : off];
+      const int below = tr ? dz > 0 : dz < 0;
+      for (int par = 0; par < 2; par++)
+        for (int m = 0; m < P; m++) {
+          const double s = below && ((m + par) & 1) ? -1.0 : 1.0;
+          const size_t i = 2 * (((size_t)off * 2 + par) * P + m);
+          w[i] = s * cos(m * phi);
+          w[i + 1] = s * (tr ? -sin(m * phi) : sin(m * phi));
+        }
+    }
+    for (size_t i = 0; i < 2 * n; i++) f[i] = (float)w[i];
+    if ((rc = fmbh_malloc(&o->d_ts_phase[tr], o->csz * n))) break;
+    pl->bytes += o->csz * n;
+    rc = fmbh_h2d(o->d_ts_phase[tr], o->prec == FMB_FP64 ? (const void *)w : (const void *)f,
+                  o->csz * n, stream);
+  }
+  free(w);
+  free(f);
+  if (!rc) rc = fmbh_sync(stream);
+  fmbh_free(d_hoff);
+  fmbh_free(d_cb);
+  return rc;
+}
+
+/* schedule: {first, end} of every wave's rotation units, then of its coaxial
+ * units, then the units {degree or |m|, table offset}.  Units go by
+ * decreasing cost to the least-loaded SIMD (waves w, w + 4, ... share one),
+ * and there to the least-loaded wave. */
+static int ts_sched(int prec, int p, int **d_out, void *stream) {
+  const int nw = prec == FMB_FP64 ? FMBH_TS_WAVES64 : FMBH_TS_WAVES32;
+  int off[FMBH_TS_PMAX], h[4 * FMBH_TS_WAVES64 + 4 * FMBH_TS_PMAX], q = 2 * nw, rc;
+  unit_t u[FMBH_TS_PMAX];
+  const int c1 = prec == FMB_FP64 ? 16 : 8; /* cycles of 4 rows x 1 column */
+  for (int st = 0; st < 2; st++) {
+    ts_blocks(prec, !st, p, off);
+    for (int i = 0; i < p; i++) {
+      const int s = st ? p - i : i + 1, rg = (s + 3) / 4;
+      u[i].code = i;
+      u[i].aoff = off[i];
+      /* cycles: the products of both rotations and the rows' loads, phases
+       * and sums; the products of the coaxial block */
+      u[i].cost = st ? 2 * c1 * rg * s + 20 * s + 100 : 2 * c1 * rg * s + 300 * rg + 300;
+    }
+    int simd[4] = {0}, load[FMBH_TS_WAVES64] = {0};
+    qsort(u, p, sizeof(unit_t), by_cost);
+    for (int i = 0; i < p; i++) {
+      int b = 0;
+      for (int k = 1; k < 4; k++)
+        if (simd[k] < simd[b]) b = k;
+      int w = b;
+      for (int k = b; k < nw; k += 4)
+        if (load[k] < load[w]) w = k;
+      simd[b] += u[i].cost;
+      load[w] += u[i].cost;
+      u[i].w = w;
+    }
+    for (int w = 0; w < nw; w++) {
+      h[2 * (st * nw + w)] = q;
+      for (int i = 0; i < p; i++)
+        if (u[i].w == w) {
+          h[2 * q] = u[i].code;
+          h[2 * q + 1] = u[i].aoff;
+          q++;
+        }
+      h[2 * (st * nw + w) + 1] = q;
+    }
+  }
+  rc = fmbh_malloc((void **)d_out, sizeof(int) * 2 * q);
+  if (!rc) rc = fmbh_h2d(*d_out, h, sizeof(int) * 2 * q, stream);
+  return rc;
+}
+
+/* Whether an M2L of order p over npairs pairs and nrhs right-hand sides runs
+ * target-stationary.  Measured against the offset-batched kernels on the
+ * 20,480-triangle sphere, speedup at 1 / 3 / 16 right-hand sides:
+ *   FP64, 170,400 and 400,056 pairs: order 14 1.32 / 1.45 / 1.9, order 16
+ *     1.1-1.2 / 1.29 / 1.46, orders 2 to 12 1.2-1.7; 9,744 pairs: 1.2-1.5;
+ *     2,504 pairs 0.9-1.2.  Order 18 (327,680 triangles) 0.78.
+ *   FP32: order 14 1.15-1.2 / 1.25 / 1.6-1.8, order 16 0.92 / 1.0 / 1.3,
+ *     orders 2 to 12 1.15-1.6; at or under 36,192 vectors 0.85-1.1.
+ * (Above order 16 the batch and the sums no longer fit the LDS at a useful
+ * size.) */
+static int ts_use(int prec, int p, int npairs, int nrhs) {
+  if (p > FMBH_TS_PMAX) return 0;
+  if (prec == FMB_FP64) return 1;
+  return (p <= 14 || nrhs >= 16) && (double)npairs * nrhs >= 40000;
+}
+
+/* sums of a workgroup: at most 32 target vectors in 160 KB of LDS, or in the
+ * FP32 pass in 80 KB, so that two workgroups share a CU */
+static int ts_slots(int prec, int p) {
+  const size_t cap = (prec == FMB_FP64 ? 160 : 80) * 1024;
+  int s = 32;
+  while (s > 1 && fmbh_ts_lds_bytes(p, prec, s) > cap) s--;
+  return s;
+}
+
+/* schedule, pair lists and coaxial tables of the target-stationary M2L at
+ * level l, where its shape was not requested otherwise.  Two lists: groups of
+ * as many targets as fill the slots at nrhs_max right-hand sides, and at one
+ * (passes with fewer right-hand sides than the plan holds). */
+static int ts_setup(fmb_plan *pl, int l, fmb_rcr_tab *tb, int op, void *stream) {
+  const fmb_tree *t = pl->tree;
+  const fmb_plan_params *prm = &pl->prm;
+  fmb_opset *o = &pl->ops[op];
+  const int p = pl->p[l];
+  int rc, coff[FMBH_TS_PMAX], *d_coff = NULL;
+  /* 32-bit buffer offsets into the coefficients */
+  if ((size_t)t->nbox[l] * pl->nrhs_max * p * p * o->csz >= (1ull << 32)) return FMB_OK;
+  if (prm->rcr_mode || prm->waves || prm->ldso || (prm->split_bf16 && op == 1) ||
+      prm->m2l_tile != RCR_TILE || prm->m2l_tile_min_mb != RCR_TILE_MIN_MB)
+    return FMB_OK;
+  if (!t->npairs[l] || !ts_use(o->prec, p, t->npairs[l], pl->nrhs_max)) return FMB_OK;
+  const int S = ts_slots(o->prec, p);
+  tb->ts_slots[op] = S;
+  for (int i = 0; i < (pl->nrhs_max > 1 ? 2 : 1); i++) {
+    const int R = i || pl->nrhs_max == 1 ? 1 : (pl->nrhs_max < S ? pl->nrhs_max : S);
+    tb->ts_tgrp[op][i] = S / R;
+    const size_t bytes = sizeof(int) * (2 * (size_t)t->npairs[l] +
+                                        (size_t)FMB_NCLASS * (t->nbox[l] / (S / R) + 1));
+    if ((rc = fmbh_ts_lists(t, l, S / R, pl->off_class, &tb->d_ts_pairs[op][i],
+                            &tb->d_ts_seg[op][i], stream)))
+      return rc;
+    pl->bytes += bytes;
+  }
+  if ((rc = ts_sched(o->prec, p, &tb->d_ts_sched[op], stream))) return rc;
+  tb->ts_cstride[op] = ts_blocks(o->prec, 0, p, coff);
+  const size_t cb = o->csz / 2 * (size_t)tb->ts_cstride[op] * FMB_NDIST;
+  if ((rc = fmbh_malloc(&tb->d_ts_C[op], cb))) return rc;
+  pl->bytes += cb;
+  rc = fmbh_malloc((void **)&d_coff, sizeof(int) * p);
+  if (!rc) rc = fmbh_h2d(d_coff, coff, sizeof(int) * p, stream);
+  if (!rc)
+    rc = fmbh_ts_coax(o->prec, o->d_Csr[l], p, d_coff, tb->ts_cstride[op], tb->d_ts_C[op], stream);
+  if (!rc) rc = fmbh_sync(stream);
+  fmbh_free(d_coff);
+  return rc;
+}
+
+static int ts_run(const fmb_plan *pl, int op, int l, int trans, int nrhs, void *stream) {
+  const fmb_rcr_tab *tb = &pl->rcr[0][l];
+  const fmb_opset *o = &pl->ops[op];
+  const int S = tb->ts_slots[op];
+  /* the list of one right-hand side per group where the other would leave
+   * over a quarter of the slots empty */
+  int i = 0;
+  if (tb->d_ts_pairs[op][1]) {
+    const int T = tb->ts_tgrp[op][0], R = S / T < nrhs ? S / T : nrhs;
+    i = 4 * T * R < 3 * S && R < 16;
+  }
+  fmbh_ts_job j;
+  j.pairs = tb->d_ts_pairs[op][i];
+  j.seg = tb->d_ts_seg[op][i];
+  j.npairs = pl->tree->npairs[l];
+  j.tgrp = tb->ts_tgrp[op][i];
+  j.nbox = pl->tree->nbox[l];
+  j.ngroups = (j.nbox + j.tgrp - 1) / j.tgrp;
+  j.slots = S;
+  j.p = pl->p[l];
+  j.phase = o->d_ts_phase[trans];
+  j.pstride = o->ts_P;
+  j.H = o->d_ts_H;
+  j.hstride = o->ts_hstride;
+  j.C = tb->d_ts_C[op];
+  j.cstride = tb->ts_cstride[op];
+  j.cdist = pl->class_dist;
+  j.sched = tb->d_ts_sched[op];
+  j.in = trans ? o->d_L[l] : o->d_M[l];
+  j.out = trans ? o->d_M[l] : o->d_L[l];
+  return fmbh_ts_run(&j, o->prec, nrhs, stream);
+}
+
+/* the target-stationary M2L was set up for this pass */
+static int ts_ready(const fmb_plan *pl, int op, int l, int nrhs) {
+  return pl->rcr[0][l].ts_slots[op] &&
+         ts_use(pl->ops[op].prec, pl->p[l], pl->tree->npairs[l], nrhs);
+}
+
 int fmbx_rcr_rot_setup(fmb_plan *pl, void *stream) {
   if (pl->prm.rcr_path == FMB_RCR_VALU) return FMB_OK;
   int rc = FMB_OK;
@@ -409,6 +632,7 @@ int fmbx_rcr_rot_setup(fmb_plan *pl, void *stream) {
     }
     free(ph);
   }
+  for (int op = 0; op < pl->nops && !rc; op++) rc = ts_rot_setup(pl, &pl->ops[op], stream);
   if (rc) return rc;
   /* padded rotation blocks of every polar angle, per opset */
   int *hoff = (int *)malloc(sizeof(int) * (pl->Pmax + 1)), *d_hoff = NULL;
@@ -858,6 +1082,11 @@ int fmbx_rcr_setup(fmb_plan *pl, void *stream) {
   if (pl->prm.autotune && pl->prm.rcr_path != FMB_RCR_VALU)
     for (int op = 0; op < pl->nops; op++)
       if ((rc = autotune(pl, op, stream))) return rc;
+  /* (last: the autotuner times the offset-batched shapes) */
+  if (pl->prm.rcr_path != FMB_RCR_VALU)
+    for (int op = 0; op < pl->nops; op++)
+      for (int l = 2; l <= L; l++)
+        if ((rc = ts_setup(pl, l, &pl->rcr[0][l], op, stream))) return rc;
   return FMB_OK;
 }
 
@@ -871,6 +1100,12 @@ void fmbx_rcr_free(fmb_plan *pl) {
       for (int op = 0; op < 2; op++) {
         fmbh_free(tb->d_sched[op]);
         fmbh_free(tb->d_Cpad[op]);
+        for (int i = 0; i < 2; i++) {
+          fmbh_free(tb->d_ts_pairs[op][i]);
+          fmbh_free(tb->d_ts_seg[op][i]);
+        }
+        fmbh_free(tb->d_ts_sched[op]);
+        fmbh_free(tb->d_ts_C[op]);
       }
       memset(tb, 0, sizeof(*tb));
     }
@@ -895,6 +1130,7 @@ int fmbx_rcr_run(const fmb_plan *pl, int op, int kind, int l, int nrhs,
     if (kind == 1) return fmbh_m2m(pl, op, l, nrhs, stream);
     return fmbh_l2l(pl, op, l, nrhs, stream);
   }
+  if (kind == 0 && ts_ready(pl, op, l, nrhs)) return ts_run(pl, op, l, 0, nrhs, stream);
   const fmb_tree *t = pl->tree;
   const fmb_opset *o = &pl->ops[op];
   const fmb_rcr_tab *pairs = kind == 0 ? tb : &pl->rcr[1][l];
@@ -968,6 +1204,7 @@ int fmbx_rcr_run_t(const fmb_plan *pl, int op, int kind, int l, int nrhs,
   if (!tb->mode[op])
     return fmb_set_error(FMB_ERR_ARG,
                          "transposed translations need the matrix-core kernels");
+  if (kind == 0 && ts_ready(pl, op, l, nrhs)) return ts_run(pl, op, l, 1, nrhs, stream);
   const fmb_tree *t = pl->tree;
   const fmb_opset *o = &pl->ops[op];
   const fmb_rcr_tab *pairs = kind == 0 ? tb : &pl->rcr[1][l];

@@ -255,7 +255,10 @@ int fmb_plan_retune(fmb_plan *pl, double k, const fmb_c64 *robin, void *stream);
  * tiles per batch nt (8 nt vectors), row tiles per unit mt, waves per
  * workgroup nw (4 or 8), bf = 1 where the rotations run in split-BF16, and
  * with autotune the timed milliseconds of one launch (else 0).  Any output
- * pointer may be NULL. */
+ * pointer may be NULL.  For M2L this is the shape of the offset-batched
+ * kernel; levels of order 16 and less whose shape is left to the rule or the
+ * autotuner (rcr_mode, waves, ldso and m2l_tile at their defaults) run
+ * target-stationary instead where that is faster (csrc/hip/rcr_ts.hip). */
 int fmb_plan_tile_shape(const fmb_plan *pl, int kind, int level, int prec, int *mode,
                         int *nt, int *mt, int *nw, int *bf, double *ms);
 /* Wavenumber of the operator the plan holds (0 after a failed retune). */
