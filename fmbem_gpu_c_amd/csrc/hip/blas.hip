@@ -1,116 +1,160 @@
 // blas.hip -- FP64 complex vector kernels for GMRES (batched over right-hand
-// sides) and the plane-wave right-hand side.  Reductions are two-stage with
-// a fixed chunk count so results do not depend on scheduling.
+// sides) and the plane-wave right-hand side.  Reductions sum the partial sums
+// of a number of blocks fixed by N, in block order, so results do not depend
+// on scheduling.
 #include "fmb_device.h"
 
 namespace {
 
-constexpr int CHUNKS = 128;
 constexpr int BS = 256;
+// blocks per inner product and per vector update at most: an inner product has nv nrhs rows of
+// blocks beside each other, an update only nrhs
+constexpr int DOT_CHUNKS = 128, UPD_CHUNKS = 2048;
 
+// sum of v over the block in a fixed order, in every thread
 __device__ __forceinline__ double block_sum(double v, double *sh) {
-  sh[threadIdx.x] = v;
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
   __syncthreads();
-  for (int s = BS / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-    __syncthreads();
-  }
-  double r = sh[0];
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
+  double r = 0.0;
+  for (int i = 0; i < BS / 64; i++) r += sh[i];
   return r;
 }
 
-// partial[(j*nrhs + r)*CHUNKS + c] = sum over chunk c of conj(V_j^r) w^r
+// Whether this block is the last of the n of reduction q to arrive: it then reads the others'
+// partial sums and completes the reduction, so a reduction takes one launch and its order does
+// not depend on which block is last.  Leaves the counter at 0.
+__device__ __forceinline__ bool last_block(unsigned *cnt, int q, unsigned n) {
+  __shared__ unsigned seen;
+  if (threadIdx.x == 0) {
+    __threadfence();
+    seen = atomicAdd(cnt + q, 1u);
+    if (seen == n - 1) cnt[q] = 0u;
+    __threadfence();
+  }
+  __syncthreads();
+  return seen == n - 1;
+}
+
+// elements [i0, i1) of chunk c of C
+__device__ __forceinline__ void chunk_range(int N, int c, int C, int &i0, int &i1) {
+  const int per = (N + C - 1) / C;
+  i0 = min(per * c, N);
+  i1 = min(i0 + per, N);
+}
+
+// h[j nrhs + r] = <V_j^r, w^r>, also to hp (host memory): grid (chunks, vectors x right-hand
+// sides)
 __global__ void __launch_bounds__(BS)
-    k_zdots_part(const double2 *__restrict__ V, int nrhs, int N,
-                 const double2 *__restrict__ w, double2 *__restrict__ part) {
-  __shared__ double sh[BS];
-  int c = blockIdx.x, jr = blockIdx.y;
-  int j = jr / nrhs, r = jr % nrhs;
-  const double2 *v = V + ((size_t)j * nrhs + r) * N;
-  const double2 *x = w + (size_t)r * N;
-  size_t per = ((size_t)N + CHUNKS - 1) / CHUNKS;
-  size_t i0 = per * c, i1 = i0 + per < (size_t)N ? i0 + per : (size_t)N;
+    k_dots(const double2 *__restrict__ V, int nrhs, int N, const double2 *__restrict__ w,
+           double2 *__restrict__ part, unsigned *__restrict__ cnt, double2 *__restrict__ h,
+           double2 *__restrict__ hp) {
+  __shared__ double sh[BS / 64];
+  const int C = gridDim.x, c = blockIdx.x, jr = blockIdx.y, r = jr % nrhs;
+  const double2 *v = V + (size_t)jr * N, *x = w + (size_t)r * N;
+  int i0, i1;
+  chunk_range(N, c, C, i0, i1);
   double sr = 0, si = 0;
-  for (size_t i = i0 + threadIdx.x; i < i1; i += BS) {
-    double2 a = v[i], b = x[i];
+  for (int i = i0 + threadIdx.x; i < i1; i += BS) {
+    const double2 a = v[i], b = x[i];
     sr += a.x * b.x + a.y * b.y;
     si += a.x * b.y - a.y * b.x;
   }
   sr = block_sum(sr, sh);
   si = block_sum(si, sh);
-  if (threadIdx.x == 0) part[(size_t)jr * CHUNKS + c] = make_double2(sr, si);
+  if (C > 1) {
+    if (threadIdx.x == 0) part[(size_t)jr * C + c] = make_double2(sr, si);
+    if (!last_block(cnt, jr, C)) return;
+    double2 t = make_double2(0.0, 0.0);
+    if (threadIdx.x < C) t = part[(size_t)jr * C + threadIdx.x];
+    sr = block_sum(t.x, sh);
+    si = block_sum(t.y, sh);
+  }
+  if (threadIdx.x == 0) h[jr] = hp[jr] = make_double2(sr, si);
 }
 
-__global__ void k_sum_chunks(const double2 *__restrict__ part, int n,
-                             double2 *__restrict__ out) {
-  int jr = blockIdx.x * blockDim.x + threadIdx.x;
-  if (jr >= n) return;
-  double sr = 0, si = 0;
-  for (int c = 0; c < CHUNKS; c++) {
-    double2 v = part[(size_t)jr * CHUNKS + c];
-    sr += v.x;
-    si += v.y;
-  }
-  out[jr] = make_double2(sr, si);
-}
-
-__global__ void __launch_bounds__(BS)
-    k_znorm_part(const double2 *__restrict__ w, int N, double *__restrict__ part) {
-  __shared__ double sh[BS];
-  int c = blockIdx.x, r = blockIdx.y;
-  const double2 *x = w + (size_t)r * N;
-  size_t per = ((size_t)N + CHUNKS - 1) / CHUNKS;
-  size_t i0 = per * c, i1 = i0 + per < (size_t)N ? i0 + per : (size_t)N;
-  double s = 0;
-  for (size_t i = i0 + threadIdx.x; i < i1; i += BS) {
-    double2 a = x[i];
-    s += a.x * a.x + a.y * a.y;
-  }
+// |w|^2 of the block's chunk -> norm of right-hand side r
+__device__ __forceinline__ void norm_end(double s, double *sh, double *part, unsigned *cnt, int r,
+                                         double *nrm, double *hp) {
+  const int C = gridDim.x, c = blockIdx.x;
   s = block_sum(s, sh);
-  if (threadIdx.x == 0) part[(size_t)r * CHUNKS + c] = s;
-}
-
-__global__ void k_norm_final(const double *__restrict__ part, int n,
-                             double *__restrict__ out) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  double s = 0;
-  for (int c = 0; c < CHUNKS; c++) s += part[(size_t)r * CHUNKS + c];
-  out[r] = sqrt(s);
-}
-
-__global__ void k_gemv(const double2 *__restrict__ V, int nv,
-                       const double2 *__restrict__ h, double2 *__restrict__ w,
-                       int nrhs, int N, double sign) {
-  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)N * nrhs) return;
-  int r = (int)(t / N);
-  size_t i = t % N;
-  double sr = 0, si = 0;
-  for (int j = 0; j < nv; j++) {
-    double2 a = h[(size_t)j * nrhs + r], v = V[((size_t)j * nrhs + r) * N + i];
-    sr += a.x * v.x - a.y * v.y;
-    si += a.x * v.y + a.y * v.x;
+  if (C > 1) {
+    if (threadIdx.x == 0) part[(size_t)r * C + c] = s;
+    if (!last_block(cnt, r, C)) return;
+    s = 0.0;
+    for (int i = threadIdx.x; i < C; i += BS) s += part[(size_t)r * C + i];
+    s = block_sum(s, sh);
   }
-  w[t].x += sign * sr;
-  w[t].y += sign * si;
+  if (threadIdx.x == 0) nrm[r] = hp[r] = sqrt(s);
 }
 
-__global__ void k_axpby(const double2 *__restrict__ a, const double2 *__restrict__ x,
-                        const double2 *__restrict__ b, double2 *__restrict__ y,
-                        int nrhs, int N) {
-  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)N * nrhs) return;
-  int r = (int)(t / N);
-  double2 av = a[r], xv = x[t];
-  double2 res = make_double2(av.x * xv.x - av.y * xv.y, av.x * xv.y + av.y * xv.x);
-  if (b) {
-    double2 bv = b[r], yv = y[t];
-    res.x += bv.x * yv.x - bv.y * yv.y;
-    res.y += bv.x * yv.y + bv.y * yv.x;
+// w^r += sign sum_j h[j nrhs + r] V_j^r, and with NORM |w^r|: grid (chunks, right-hand sides)
+template <bool NORM>
+__global__ void __launch_bounds__(BS)
+    k_gemv(const double2 *__restrict__ V, int nv, const double2 *__restrict__ h,
+           double2 *__restrict__ w, int nrhs, int N, double sign, double *__restrict__ part,
+           unsigned *__restrict__ cnt, double *__restrict__ nrm, double *__restrict__ hp) {
+  __shared__ double sh[BS / 64];
+  const int r = blockIdx.y;
+  int i0, i1;
+  chunk_range(N, blockIdx.x, gridDim.x, i0, i1);
+  double s = 0.0;
+  for (int i = i0 + threadIdx.x; i < i1; i += BS) {
+    double sr = 0, si = 0;
+#pragma unroll 8
+    for (int j = 0; j < nv; j++) {
+      const double2 a = h[(size_t)j * nrhs + r], v = V[((size_t)j * nrhs + r) * N + i];
+      sr += a.x * v.x - a.y * v.y;
+      si += a.x * v.y + a.y * v.x;
+    }
+    double2 y = w[(size_t)r * N + i];
+    y.x += sign * sr;
+    y.y += sign * si;
+    w[(size_t)r * N + i] = y;
+    s += y.x * y.x + y.y * y.y;
   }
-  y[t] = res;
+  if constexpr (NORM) norm_end(s, sh, part, cnt, r, nrm, hp);
+}
+
+// r = b - w (w NULL: r = b; r NULL: only the norm) and |r|
+__global__ void __launch_bounds__(BS)
+    k_resid(const double2 *__restrict__ b, const double2 *__restrict__ w, double2 *__restrict__ res,
+            int N, double *__restrict__ part, unsigned *__restrict__ cnt,
+            double *__restrict__ nrm, double *__restrict__ hp) {
+  __shared__ double sh[BS / 64];
+  const size_t o = (size_t)blockIdx.y * N;
+  int i0, i1;
+  chunk_range(N, blockIdx.x, gridDim.x, i0, i1);
+  double s = 0.0;
+  for (int i = i0 + threadIdx.x; i < i1; i += BS) {
+    double2 y = b[o + i];
+    if (w) {
+      const double2 v = w[o + i];
+      y.x -= v.x;
+      y.y -= v.y;
+    }
+    if (res) res[o + i] = y;
+    s += y.x * y.x + y.y * y.y;
+  }
+  norm_end(s, sh, part, cnt, blockIdx.y, nrm, hp);
+}
+
+// y^r = x^r / nrm[r] (0 for a zero norm)
+__global__ void __launch_bounds__(BS)
+    k_unit(const double2 *__restrict__ x, const double *__restrict__ nrm, double2 *__restrict__ y,
+           int nrhs, int N) {
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (size_t)N * nrhs) return;
+  const double n = nrm[t / N], f = n > 0 ? 1.0 / n : 0.0;
+  y[t] = make_double2(f * x[t].x, f * x[t].y);
+}
+
+// y += x
+__global__ void __launch_bounds__(BS)
+    k_add(const double2 *__restrict__ x, double2 *__restrict__ y, size_t n) {
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) y[t] = make_double2(y[t].x + x[t].x, y[t].y + x[t].y);
 }
 
 __global__ void k_rhs_plane(const double *__restrict__ geo,
@@ -171,65 +215,99 @@ inline int nblk(size_t n, int b = 256) { return (int)((n + b - 1) / b); }
 
 }  // namespace
 
-extern "C" int fmbh_zdots(const fmb_c64 *d_V, int nv, const fmb_c64 *d_w,
-                          int nrhs, int N, fmb_c64 *d_h, void *stream) {
+// blocks over N elements: one element a thread up to the limit
+static int chunks_for(int N, int limit) {
+  const int c = (N + BS - 1) / BS;
+  return c < 1 ? 1 : (c > limit ? limit : c);
+}
+
+// Layout of the vector workspace: partial sums, counters, h1, h2, norms; the host mirror holds
+// h1, h2, norms
+static size_t ws_part(int nv, int nrhs, int N) {
+  const size_t d = sizeof(double2) * chunks_for(N, DOT_CHUNKS) * (size_t)nv * nrhs;
+  const size_t u = (sizeof(double) * chunks_for(N, UPD_CHUNKS) * (size_t)nrhs + 15) & ~(size_t)15;
+  return d > u ? d : u;
+}
+static size_t ws_cnt(int nv, int nrhs) {
+  return (sizeof(unsigned) * (size_t)nv * nrhs + 15) & ~(size_t)15;
+}
+
+extern "C" size_t fmbh_vecws_host_bytes(int nv, int nrhs) {
+  return sizeof(double2) * 2 * (size_t)nv * nrhs + sizeof(double) * (size_t)nrhs;
+}
+extern "C" size_t fmbh_vecws_bytes(int nv, int nrhs, int N) {
+  return ws_part(nv, nrhs, N) + ws_cnt(nv, nrhs) + fmbh_vecws_host_bytes(nv, nrhs);
+}
+
+extern "C" int fmbh_vecws_init(fmbh_vecws *ws, void *dev, void *host, int nv, int nrhs, int N,
+                               void *stream) {
+  char *d = (char *)dev + ws_part(nv, nrhs, N);
+  ws->part = dev;
+  ws->cnt = (unsigned *)d;
+  ws->h1 = (fmb_c64 *)(d + ws_cnt(nv, nrhs));
+  ws->h2 = ws->h1 + (size_t)nv * nrhs;
+  ws->nrm = (double *)(ws->h2 + (size_t)nv * nrhs);
+  ws->hp1 = (fmb_c64 *)host;
+  ws->hp2 = ws->hp1 + (size_t)nv * nrhs;
+  ws->hpn = (double *)(ws->hp2 + (size_t)nv * nrhs);
+  return fmbh_memset(ws->cnt, 0, ws_cnt(nv, nrhs), stream);
+}
+
+// One Arnoldi step: w -= V (V^H w) twice (classical Gram-Schmidt with one reorthogonalisation),
+// |w|, V_nv = w / |w|.  The inner products of both passes and the norms reach the host mirror; the
+// caller waits for the stream once.  A small solve is bound by launches and waits: five launches and
+// no transfers take 0.06 ms a step beside the product at 1,280 triangles, ten launches, six
+// transfers, three allocations and eleven waits took 0.19 ms (its whole solve 7.5 ms then, 4.2
+// now; 0.5 ms of the difference are M2L's).
+extern "C" int fmbh_arnoldi(fmb_c64 *d_V, int nv, fmb_c64 *d_w, int nrhs, int N,
+                            const fmbh_vecws *ws, void *stream) {
   hipStream_t st = (hipStream_t)stream;
-  double2 *part;
-  int rc = fmbh_malloc((void **)&part, sizeof(double2) * CHUNKS * nv * nrhs);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_zdots_part, dim3(CHUNKS, nv * nrhs), dim3(BS), 0, st,
-                     (const double2 *)d_V, nrhs, N, (const double2 *)d_w, part);
+  double2 *V = (double2 *)d_V, *w = (double2 *)d_w, *part = (double2 *)ws->part;
+  const dim3 gd(chunks_for(N, DOT_CHUNKS), nv * nrhs), gv(chunks_for(N, UPD_CHUNKS), nrhs), blk(BS);
+  hipLaunchKernelGGL(k_dots, gd, blk, 0, st, V, nrhs, N, w, part, ws->cnt, (double2 *)ws->h1,
+                     (double2 *)ws->hp1);
   FMB_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_chunks, dim3(nblk(nv * nrhs)), dim3(256), 0, st,
-                     part, nv * nrhs, (double2 *)d_h);
+  hipLaunchKernelGGL(k_gemv<false>, gv, blk, 0, st, V, nv, (const double2 *)ws->h1, w, nrhs, N,
+                     -1.0, nullptr, nullptr, nullptr, nullptr);
   FMB_LAUNCH_CHECK();
-  FMB_HIP_CHECK(hipStreamSynchronize(st));
-  fmbh_free(part);
-  return FMB_OK;
+  hipLaunchKernelGGL(k_dots, gd, blk, 0, st, V, nrhs, N, w, part, ws->cnt, (double2 *)ws->h2,
+                     (double2 *)ws->hp2);
+  FMB_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_gemv<true>, gv, blk, 0, st, V, nv, (const double2 *)ws->h2, w, nrhs, N,
+                     -1.0, (double *)ws->part, ws->cnt, ws->nrm, ws->hpn);
+  FMB_LAUNCH_CHECK();
+  return fmbh_unit(d_w, ws->nrm, d_V + (size_t)nv * nrhs * N, nrhs, N, stream);
 }
 
-extern "C" int fmbh_znorms(const fmb_c64 *d_w, int nrhs, int N, double *d_nrm,
-                           void *stream) {
-  hipStream_t st = (hipStream_t)stream;
-  double *part;
-  int rc = fmbh_malloc((void **)&part, sizeof(double) * CHUNKS * nrhs);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_znorm_part, dim3(CHUNKS, nrhs), dim3(BS), 0, st,
-                     (const double2 *)d_w, N, part);
-  FMB_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_norm_final, dim3(nblk(nrhs)), dim3(256), 0, st, part,
-                     nrhs, d_nrm);
-  FMB_LAUNCH_CHECK();
-  FMB_HIP_CHECK(hipStreamSynchronize(st));
-  fmbh_free(part);
-  return FMB_OK;
-}
-
-extern "C" int fmbh_zgemv_sub(const fmb_c64 *d_V, int nv, const fmb_c64 *d_h,
-                              fmb_c64 *d_w, int nrhs, int N, void *stream) {
-  hipLaunchKernelGGL(k_gemv, dim3(nblk((size_t)N * nrhs)), dim3(256), 0,
-                     (hipStream_t)stream, (const double2 *)d_V, nv,
-                     (const double2 *)d_h, (double2 *)d_w, nrhs, N, -1.0);
+extern "C" int fmbh_resid(const fmb_c64 *d_b, const fmb_c64 *d_w, fmb_c64 *d_r, int nrhs, int N,
+                          const fmbh_vecws *ws, void *stream) {
+  hipLaunchKernelGGL(k_resid, dim3(chunks_for(N, UPD_CHUNKS), nrhs), dim3(BS), 0, (hipStream_t)stream,
+                     (const double2 *)d_b, (const double2 *)d_w, (double2 *)d_r, N,
+                     (double *)ws->part, ws->cnt, ws->nrm, ws->hpn);
   FMB_LAUNCH_CHECK();
   return FMB_OK;
 }
 
-extern "C" int fmbh_zgemv_add(const fmb_c64 *d_V, int nv, const fmb_c64 *d_y,
-                              fmb_c64 *d_x, int nrhs, int N, void *stream) {
-  hipLaunchKernelGGL(k_gemv, dim3(nblk((size_t)N * nrhs)), dim3(256), 0,
-                     (hipStream_t)stream, (const double2 *)d_V, nv,
-                     (const double2 *)d_y, (double2 *)d_x, nrhs, N, 1.0);
+extern "C" int fmbh_unit(const fmb_c64 *d_x, const double *d_nrm, fmb_c64 *d_y, int nrhs, int N,
+                         void *stream) {
+  hipLaunchKernelGGL(k_unit, dim3(nblk((size_t)N * nrhs)), dim3(BS), 0, (hipStream_t)stream,
+                     (const double2 *)d_x, d_nrm, (double2 *)d_y, nrhs, N);
   FMB_LAUNCH_CHECK();
   return FMB_OK;
 }
 
-extern "C" int fmbh_zaxpby(const fmb_c64 *d_a, const fmb_c64 *d_x,
-                           const fmb_c64 *d_b, fmb_c64 *d_y, int nrhs, int N,
-                           void *stream) {
-  hipLaunchKernelGGL(k_axpby, dim3(nblk((size_t)N * nrhs)), dim3(256), 0,
-                     (hipStream_t)stream, (const double2 *)d_a,
-                     (const double2 *)d_x, (const double2 *)d_b, (double2 *)d_y,
-                     nrhs, N);
+extern "C" int fmbh_zgemv_add(const fmb_c64 *d_V, int nv, const fmb_c64 *d_y, fmb_c64 *d_x,
+                              int nrhs, int N, void *stream) {
+  hipLaunchKernelGGL(k_gemv<false>, dim3(chunks_for(N, UPD_CHUNKS), nrhs), dim3(BS), 0, (hipStream_t)stream,
+                     (const double2 *)d_V, nv, (const double2 *)d_y, (double2 *)d_x, nrhs, N, 1.0,
+                     nullptr, nullptr, nullptr, nullptr);
+  FMB_LAUNCH_CHECK();
+  return FMB_OK;
+}
+
+extern "C" int fmbh_zadd(const fmb_c64 *d_x, fmb_c64 *d_y, size_t n, void *stream) {
+  hipLaunchKernelGGL(k_add, dim3(nblk(n)), dim3(BS), 0, (hipStream_t)stream,
+                     (const double2 *)d_x, (double2 *)d_y, n);
   FMB_LAUNCH_CHECK();
   return FMB_OK;
 }

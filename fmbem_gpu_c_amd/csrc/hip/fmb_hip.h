@@ -19,6 +19,9 @@ int fmbh_init(void);
 int fmbh_device_tag(char *buf, int n);
 int fmbh_malloc(void **p, size_t bytes);
 int fmbh_free(void *p);
+int fmbh_host_malloc(void **p, size_t bytes); /* page-locked, device-visible */
+int fmbh_host_free(void *p);
+int fmbh_h2d_async(void *dst, const void *pinned, size_t bytes, void *stream);
 int fmbh_h2d(void *dst, const void *src, size_t bytes, void *stream);
 int fmbh_d2h(void *dst, const void *src, size_t bytes, void *stream);
 int fmbh_d2d(void *dst, const void *src, size_t bytes, void *stream);
@@ -214,21 +217,35 @@ int fmbh_sweep_guess(const fmb_plan *pl, double dk, const fmb_c64 *d_x,
                      const double *h_dirs, int nrhs, fmb_c64 *d_x0, void *stream);
 int fmbh_rhs_plane(const fmb_plan *pl, const double *h_dirs, int nrhs,
                    fmb_c64 *d_b, void *stream);
-/* h[j*nrhs + r] = <V_j^r, w^r> for j < nv ; V: [nv][nrhs][N] */
-int fmbh_zdots(const fmb_c64 *d_V, int nv, const fmb_c64 *d_w, int nrhs,
-               int N, fmb_c64 *d_h, void *stream);
-/* w^r -= sum_j h[j*nrhs+r] V_j^r */
-int fmbh_zgemv_sub(const fmb_c64 *d_V, int nv, const fmb_c64 *d_h,
-                   fmb_c64 *d_w, int nrhs, int N, void *stream);
-/* nrm[r] = ||w^r|| */
-int fmbh_znorms(const fmb_c64 *d_w, int nrhs, int N, double *d_nrm,
-                void *stream);
-/* y^r = a[r] x^r + b[r] y^r  (a, b device complex per rhs; NULL b = 0) */
-int fmbh_zaxpby(const fmb_c64 *d_a, const fmb_c64 *d_x, const fmb_c64 *d_b,
-                fmb_c64 *d_y, int nrhs, int N, void *stream);
-/* x^r += sum_j y[j*nrhs+r] V_j^r  (y on device) */
-int fmbh_zgemv_add(const fmb_c64 *d_V, int nv, const fmb_c64 *d_y,
-                   fmb_c64 *d_x, int nrhs, int N, void *stream);
+/* GMRES vector operations (blas.hip).  V: [nv][nrhs][N].  Workspace of up to
+ * nv basis vectors: one device block, and one page-locked host block that the
+ * kernels write h1, h2 (the two Gram-Schmidt passes, [j*nrhs + r]) and the
+ * norms to; the host reads it after waiting for the stream. */
+typedef struct fmbh_vecws {
+  void *part;
+  unsigned *cnt;
+  fmb_c64 *h1, *h2;
+  double *nrm;
+  fmb_c64 *hp1, *hp2;
+  double *hpn;
+} fmbh_vecws;
+size_t fmbh_vecws_bytes(int nv, int nrhs, int N); /* sizes in multiples of 8 */
+size_t fmbh_vecws_host_bytes(int nv, int nrhs);
+int fmbh_vecws_init(fmbh_vecws *ws, void *dev, void *host, int nv, int nrhs, int N,
+                    void *stream);
+/* w orthogonalised against V_0 .. V_{nv-1}, V_nv = w / |w| */
+int fmbh_arnoldi(fmb_c64 *d_V, int nv, fmb_c64 *d_w, int nrhs, int N, const fmbh_vecws *ws,
+                 void *stream);
+/* r = b - w (w NULL: r = b; r NULL: not stored) and the norms |r| */
+int fmbh_resid(const fmb_c64 *d_b, const fmb_c64 *d_w, fmb_c64 *d_r, int nrhs, int N,
+               const fmbh_vecws *ws, void *stream);
+/* y^r = x^r / nrm[r], 0 for a zero norm (nrm on the device) */
+int fmbh_unit(const fmb_c64 *d_x, const double *d_nrm, fmb_c64 *d_y, int nrhs, int N,
+              void *stream);
+/* x^r += sum_j y[j*nrhs+r] V_j^r  (y on the device) */
+int fmbh_zgemv_add(const fmb_c64 *d_V, int nv, const fmb_c64 *d_y, fmb_c64 *d_x, int nrhs, int N,
+                   void *stream);
+int fmbh_zadd(const fmb_c64 *d_x, fmb_c64 *d_y, size_t n, void *stream); /* y += x */
 
 #ifdef __cplusplus
 }

@@ -41,6 +41,27 @@ extern "C" int fmbh_free(void *p) {
   return FMB_OK;
 }
 
+extern "C" int fmbh_host_malloc(void **p, size_t bytes) {
+  *p = nullptr;
+  hipError_t e = hipHostMalloc(p, bytes ? bytes : 64, hipHostMallocDefault);
+  if (e != hipSuccess)
+    return fmb_set_error(FMB_ERR_NOMEM, "hipHostMalloc(%zu) failed: %s", bytes,
+                         hipGetErrorString(e));
+  return FMB_OK;
+}
+
+extern "C" int fmbh_host_free(void *p) {
+  if (p) FMB_HIP_CHECK(hipHostFree(p));
+  return FMB_OK;
+}
+
+/* src page-locked and left alone until the stream has passed the copy */
+extern "C" int fmbh_h2d_async(void *dst, const void *src, size_t bytes, void *stream) {
+  if (!bytes) return FMB_OK;
+  FMB_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, (hipStream_t)stream));
+  return FMB_OK;
+}
+
 extern "C" int fmbh_h2d(void *dst, const void *src, size_t bytes,
                         void *stream) {
   if (!bytes) return FMB_OK;

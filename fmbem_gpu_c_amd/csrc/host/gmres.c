@@ -185,11 +185,58 @@ static void sys_free(sys_t *S) {
   memset(S, 0, sizeof(*S));
 }
 
+/* Device vectors and scratch of a solve in one block, and the page-locked
+ * host block that the vector kernels write their inner products and norms to
+ * (then y): made once for a solve, also for all cycles of a refined one. */
+typedef struct {
+  void *dev, *host;
+  fmb_c64 *dV, *dw, *dr, *dy; /* m + 1 Arnoldi vectors; w; r; y            */
+  fmb_c64 *hy;                /* y on the host                             */
+  fmbh_vecws v;
+} gws_t;
+
+static int gws_init(gws_t *W, int m, int nrhs, int N, void *stream) {
+  memset(W, 0, sizeof(*W));
+  const size_t nvec = (size_t)N * nrhs, ny = (size_t)m * nrhs;
+  int rc = fmbh_malloc(&W->dev, sizeof(fmb_c64) * (nvec * (m + 3) + ny) +
+                                    fmbh_vecws_bytes(m, nrhs, N));
+  if (!rc) rc = fmbh_host_malloc(&W->host, sizeof(fmb_c64) * ny + fmbh_vecws_host_bytes(m, nrhs));
+  if (rc) return rc;
+  W->dV = (fmb_c64 *)W->dev;
+  W->dw = W->dV + nvec * (m + 1);
+  W->dr = W->dw + nvec;
+  W->dy = W->dr + nvec;
+  W->hy = (fmb_c64 *)W->host;
+  return fmbh_vecws_init(&W->v, W->dy + ny, W->hy + ny, m, nrhs, N, stream);
+}
+
+static void gws_free(gws_t *W) {
+  fmbh_free(W->dev);
+  fmbh_host_free(W->host);
+  memset(W, 0, sizeof(*W));
+}
+
+/* norms of x -> W's first inner products' place, of b -> norms, r = b */
+static int first_norms(const gws_t *W, const fmb_c64 *b, const fmb_c64 *x, fmb_c64 *r, int nrhs,
+                       int N, const double **xn, const double **bn, void *stream) {
+  fmbh_vecws vx = W->v;
+  vx.nrm = (double *)W->v.h1;
+  vx.hpn = (double *)W->v.hp1;
+  int rc = fmbh_resid(x, NULL, NULL, nrhs, N, &vx, stream);
+  if (!rc) rc = fmbh_resid(b, NULL, r, nrhs, N, &W->v, stream);
+  if (!rc) rc = fmbh_sync(stream);
+  *xn = vx.hpn;
+  *bn = W->v.hpn;
+  return rc;
+}
+
 /* x += V y over the first j Arnoldi vectors, y from the triangular solve of
  * the rotated Hessenberg systems, for the columns with sel[r] (others y = 0) */
-static int update_x(const zc *Hh, const zc *g, zc *yv, fmb_c64 *hh, int m, int nrhs,
-                    int j, const int *sel, const fmb_c64 *dV, fmb_c64 *dy, fmb_c64 *x,
-                    int N, void *stream) {
+static int update_x(const gws_t *W, const zc *Hh, const zc *g, zc *yv, int m, int nrhs, int j,
+                    const int *sel, fmb_c64 *x, int N, void *stream) {
+  fmb_c64 *hh = W->hy;
+  int rc = fmbh_sync(stream); /* an earlier update may still read hy */
+  if (rc) return rc;
 #define HQ(r, i, c) Hh[((size_t)(r) * m + (c)) * (m + 1) + (i)]
   for (int r = 0; r < nrhs; r++) {
     for (int q = j - 1; q >= 0; q--) {
@@ -201,18 +248,18 @@ static int update_x(const zc *Hh, const zc *g, zc *yv, fmb_c64 *hh, int m, int n
     for (int q = 0; q < j; q++) hh[(size_t)q * nrhs + r] = fromz(yv[(size_t)r * (m + 1) + q]);
   }
 #undef HQ
-  int rc = fmbh_h2d(dy, hh, sizeof(fmb_c64) * j * nrhs, stream);
-  if (!rc) rc = fmbh_zgemv_add(dV, j, dy, x, nrhs, N, stream);
-  if (!rc) rc = fmbh_sync(stream); /* hh is reused at once */
+  rc = fmbh_h2d_async(W->dy, hh, sizeof(fmb_c64) * j * nrhs, stream);
+  if (!rc) rc = fmbh_zgemv_add(W->dV, j, W->dy, x, nrhs, N, stream);
   return rc;
 }
 
 /* est_stop: a cycle whose estimated residuals all meet the tolerance ends
  * the solve without the FP64 true residual (for a caller that checks the
- * result itself); relres then holds those estimates */
+ * result itself); relres then holds those estimates.  W: the workspace, or
+ * NULL to make one for this solve. */
 static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, int graph,
                      const fmb_c64 *b, fmb_c64 *x, int restart, double tol, int maxit,
-                     int est_stop, fmb_gmres_info *info, void *stream) {
+                     int est_stop, gws_t *W, fmb_gmres_info *info, void *stream) {
   if (!b || !x || restart < 1 || !(tol > 0) || maxit < 1)
     return fmb_set_error(FMB_ERR_ARG, "fmb_gmres: invalid arguments");
   sys_t S;
@@ -227,56 +274,49 @@ static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, in
   const int N = pl->tree->nelem, m = restart;
   const int work = pl->work_prec;
   const double itol = work == FMB_MIXED ? 0.5 * tol : tol; /* Arnoldi stop */
-  size_t vbytes = sizeof(fmb_c64) * (size_t)N * nrhs;
-  fmb_c64 *dV = NULL, *dw = NULL, *dr = NULL, *dh = NULL, *dh2 = NULL, *dy = NULL;
-  double *dn = NULL;
+  gws_t own;
+  memset(&own, 0, sizeof(own));
   zc *Hh = NULL, *cs = NULL, *sn = NULL, *g = NULL, *yv = NULL;
-  fmb_c64 *hh = NULL, *hh2 = NULL;
-  double *bn = NULL, *rn = NULL, *hn = NULL, *rsave = NULL;
+  double *bn = NULL, *rn = NULL, *rsave = NULL;
+  const double *hx, *hb;
   int *active = NULL, *sel = NULL;
   int iters = 0, mv64 = 0, mvw = 0, restarts = 0, conv = 0;
-  if ((rc = fmbh_malloc((void **)&dV, vbytes * (m + 1)))) goto done;
-  if ((rc = fmbh_malloc((void **)&dw, vbytes))) goto done;
-  if ((rc = fmbh_malloc((void **)&dr, vbytes))) goto done;
-  if ((rc = fmbh_malloc((void **)&dh, sizeof(fmb_c64) * (m + 1) * nrhs))) goto done;
-  if ((rc = fmbh_malloc((void **)&dh2, sizeof(fmb_c64) * (m + 1) * nrhs))) goto done;
-  if ((rc = fmbh_malloc((void **)&dy, sizeof(fmb_c64) * (m + 1) * nrhs))) goto done;
-  if ((rc = fmbh_malloc((void **)&dn, sizeof(double) * nrhs))) goto done;
+  if (!W) {
+    W = &own;
+    if ((rc = gws_init(W, m, nrhs, N, stream))) goto done;
+  }
+  fmb_c64 *dV = W->dV, *dw = W->dw, *dr = W->dr;
+  const fmb_c64 *hh = W->v.hp1, *hh2 = W->v.hp2;
+  const double *hn = W->v.hpn;
   if (graph && (rc = sys_graph_init(&S, dw))) goto done;
   Hh = (zc *)calloc((size_t)(m + 1) * m * nrhs, sizeof(zc));
   cs = (zc *)calloc((size_t)m * nrhs, sizeof(zc));
   sn = (zc *)calloc((size_t)m * nrhs, sizeof(zc));
   g = (zc *)calloc((size_t)(m + 1) * nrhs, sizeof(zc));
   yv = (zc *)calloc((size_t)(m + 1) * nrhs, sizeof(zc));
-  hh = (fmb_c64 *)malloc(sizeof(fmb_c64) * (m + 1) * nrhs);
-  hh2 = (fmb_c64 *)malloc(sizeof(fmb_c64) * (m + 1) * nrhs);
   bn = (double *)malloc(sizeof(double) * nrhs);
   rn = (double *)malloc(sizeof(double) * nrhs);
-  hn = (double *)malloc(sizeof(double) * nrhs);
   rsave = (double *)malloc(sizeof(double) * nrhs);
   active = (int *)malloc(sizeof(int) * nrhs);
   sel = (int *)malloc(sizeof(int) * nrhs);
-  if (!Hh || !cs || !sn || !g || !yv || !hh || !hh2 || !bn || !rn || !hn || !rsave || !active ||
-      !sel) {
+  if (!Hh || !cs || !sn || !g || !yv || !bn || !rn || !rsave || !active || !sel) {
     rc = fmb_set_error(FMB_ERR_NOMEM, "GMRES host workspace");
     goto done;
   }
 #define HH(r, i, j) Hh[((size_t)(r) * m + (j)) * (m + 1) + (i)]
-  if ((rc = fmbh_znorms(x, nrhs, N, dn, stream))) goto done;
-  if ((rc = fmbh_d2h(bn, dn, sizeof(double) * nrhs, stream))) goto done;
+  if ((rc = first_norms(W, b, x, dr, nrhs, N, &hx, &hb, stream))) goto done;
   int x_zero = 1;
   for (int r = 0; r < nrhs; r++) {
     /* a NaN compares false with every tolerance and would read as
      * converged: non-finite inputs are refused */
-    if (!isfinite(bn[r])) {
+    if (!isfinite(hx[r])) {
       rc = fmb_set_error(FMB_ERR_ARG, "fmb_gmres: initial guess %d holds NaN or Inf", r);
       goto done;
     }
-    x_zero &= bn[r] == 0.0;
+    x_zero &= hx[r] == 0.0;
   }
-  if ((rc = fmbh_znorms(b, nrhs, N, dn, stream))) goto done;
-  if ((rc = fmbh_d2h(bn, dn, sizeof(double) * nrhs, stream))) goto done;
   for (int r = 0; r < nrhs; r++) {
+    bn[r] = hb[r];
     if (!isfinite(bn[r])) {
       rc = fmb_set_error(FMB_ERR_ARG, "fmb_gmres: right-hand side %d holds NaN or Inf", r);
       goto done;
@@ -284,30 +324,17 @@ static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, in
     if (bn[r] == 0.0) bn[r] = 1.0;
   }
   while (1) {
-    /* true residual r = b - A x in FP64 (A x = 0 for a zero first guess) */
+    /* true residual r = b - A x in FP64 (r = b, as set above, for a zero first
+     * guess) */
     if (x_zero) {
-      if ((rc = fmbh_memset(dw, 0, vbytes, stream))) goto done;
       x_zero = 0;
     } else {
       if ((rc = apply(&S, FMB_FP64, x, dw, stream))) goto done;
       mv64++;
+      if ((rc = fmbh_resid(b, dw, dr, nrhs, N, &W->v, stream))) goto done;
+      if ((rc = fmbh_sync(stream))) goto done;
     }
-    {
-      fmb_c64 *one = hh, *mone = hh2;
-      for (int r = 0; r < nrhs; r++) {
-        one[r].re = 1.0;
-        one[r].im = 0.0;
-        mone[r].re = -1.0;
-        mone[r].im = 0.0;
-      }
-      if ((rc = fmbh_h2d(dh, one, sizeof(fmb_c64) * nrhs, stream))) goto done;
-      if ((rc = fmbh_h2d(dh2, mone, sizeof(fmb_c64) * nrhs, stream))) goto done;
-      if ((rc = fmbh_d2d(dr, b, vbytes, stream))) goto done;
-      /* r = 1*b + (-1)*w  ->  zaxpby(a=-1, x=w, b=1, y=r) */
-      if ((rc = fmbh_zaxpby(dh2, dw, dh, dr, nrhs, N, stream))) goto done;
-    }
-    if ((rc = fmbh_znorms(dr, nrhs, N, dn, stream))) goto done;
-    if ((rc = fmbh_d2h(rn, dn, sizeof(double) * nrhs, stream))) goto done;
+    memcpy(rn, hn, sizeof(double) * nrhs);
     /* plans out of the graphs are not applied any more: their residuals are
      * the ones they converged with (their x no longer changes) */
     for (int p = 0; p < np; p++)
@@ -342,14 +369,10 @@ static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, in
     if (restarts > 0 || iters > 0) restarts++;
     /* V_0 = r / |r| */
     for (int r = 0; r < nrhs; r++) {
-      double s = rn[r] > 0 ? 1.0 / rn[r] : 0.0;
-      hh[r].re = s;
-      hh[r].im = 0.0;
       g[(size_t)r * (m + 1)] = rn[r];
       for (int i = 1; i <= m; i++) g[(size_t)r * (m + 1) + i] = 0.0;
     }
-    if ((rc = fmbh_h2d(dh, hh, sizeof(fmb_c64) * nrhs, stream))) goto done;
-    if ((rc = fmbh_zaxpby(dh, dr, NULL, dV, nrhs, N, stream))) goto done;
+    if ((rc = fmbh_unit(dr, W->v.nrm, dV, nrhs, N, stream))) goto done;
     int j, cyc_done = 0;
     for (j = 0; j < m && iters < maxit; j++) {
       fmb_c64 *Vj = dV + (size_t)j * N * nrhs;
@@ -359,24 +382,14 @@ static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, in
       else
         mv64++;
       iters++;
-      /* two passes of classical Gram-Schmidt */
-      for (int pass = 0; pass < 2; pass++) {
-        fmb_c64 *hbuf = pass ? hh2 : hh;
-        if ((rc = fmbh_zdots(dV, j + 1, dw, nrhs, N, dh, stream))) goto done;
-        if ((rc = fmbh_zgemv_sub(dV, j + 1, dh, dw, nrhs, N, stream))) goto done;
-        if ((rc = fmbh_d2h(hbuf, dh, sizeof(fmb_c64) * (j + 1) * nrhs, stream)))
-          goto done;
-      }
-      if ((rc = fmbh_znorms(dw, nrhs, N, dn, stream))) goto done;
-      if ((rc = fmbh_d2h(hn, dn, sizeof(double) * nrhs, stream))) goto done;
+      /* two passes of classical Gram-Schmidt, V_{j+1} = w / |w| */
+      if ((rc = fmbh_arnoldi(dV, j + 1, dw, nrhs, N, &W->v, stream))) goto done;
+      if ((rc = fmbh_sync(stream))) goto done;
       int all_done = 1;
       for (int r = 0; r < nrhs; r++) {
         for (int i = 0; i <= j; i++)
           HH(r, i, j) = toz(hh[(size_t)i * nrhs + r]) + toz(hh2[(size_t)i * nrhs + r]);
         HH(r, j + 1, j) = hn[r];
-        double s = hn[r] > 0 ? 1.0 / hn[r] : 0.0;
-        hh[r].re = s;
-        hh[r].im = 0.0;
         /* apply previous rotations and form the new one */
         for (int i = 0; i < j; i++) {
           zc h0 = HH(r, i, j), h1 = HH(r, i + 1, j);
@@ -397,10 +410,6 @@ static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, in
         if (active[r] && cabs(g[(size_t)r * (m + 1) + j + 1]) / bn[r] > itol)
           all_done = 0;
       }
-      if ((rc = fmbh_h2d(dh, hh, sizeof(fmb_c64) * nrhs, stream))) goto done;
-      if ((rc = fmbh_zaxpby(dh, dw, NULL, dV + (size_t)(j + 1) * N * nrhs, nrhs,
-                            N, stream)))
-        goto done;
       /* a batch retires a plan as soon as its estimated residuals meet the
        * tolerance: its columns of x take this step's update, its FP64 true
        * residual is checked, and it leaves the pass (a plan that fails the
@@ -415,7 +424,7 @@ static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, in
         if (!S.live[p] || !any || !ok) continue;
         for (int r = 0; r < nrhs; r++)
           sel[r] = r >= S.off[p] && r < S.off[p + 1] && active[r];
-        if ((rc = update_x(Hh, g, yv, hh, m, nrhs, j + 1, sel, dV, dy, x, N, stream)))
+        if ((rc = update_x(W, Hh, g, yv, m, nrhs, j + 1, sel, x, N, stream)))
           goto done;
         for (int r = S.off[p]; r < S.off[p + 1]; r++) active[r] = 0;
         const size_t o = (size_t)S.off[p] * N;
@@ -433,19 +442,8 @@ static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, in
         /* w's columns of p are free (V_{j+1} is formed): A x_p there */
         if ((rc = plan_apply(S.pl[p], trans, FMB_FP64, x + o, dw + o, nq, stream))) goto done;
         mv64++;
-        if ((rc = fmbh_d2d(dr + o, b + o, sizeof(fmb_c64) * nq * (size_t)N, stream))) goto done;
-        for (int r = 0; r < nq; r++) {
-          hh[r].re = 1.0;
-          hh[r].im = 0.0;
-          hh2[r].re = -1.0;
-          hh2[r].im = 0.0;
-        }
-        if ((rc = fmbh_h2d(dh, hh, sizeof(fmb_c64) * nq, stream))) goto done;
-        if ((rc = fmbh_h2d(dh2, hh2, sizeof(fmb_c64) * nq, stream))) goto done;
-        /* r_p = 1 * b_p + (-1) * A x_p */
-        if ((rc = fmbh_zaxpby(dh2, dw + o, dh, dr + o, nq, N, stream))) goto done;
-        if ((rc = fmbh_znorms(dr + o, nq, N, dn, stream))) goto done;
-        if ((rc = fmbh_d2h(hn, dn, sizeof(double) * nq, stream))) goto done;
+        if ((rc = fmbh_resid(b + o, dw + o, dr + o, nq, N, &W->v, stream))) goto done;
+        if ((rc = fmbh_sync(stream))) goto done;
         int pass = 1;
         for (int r = 0; r < nq; r++) pass &= hn[r] / bn[S.off[p] + r] <= tol;
         if (!pass) continue;
@@ -461,7 +459,7 @@ static int gmres_run(fmb_plan *const *pls, const int *nrs, int np, int trans, in
       }
     }
     /* x += V y, y from the triangular solve (inactive rhs get y = 0) */
-    if ((rc = update_x(Hh, g, yv, hh, m, nrhs, j, active, dV, dy, x, N, stream))) goto done;
+    if ((rc = update_x(W, Hh, g, yv, m, nrhs, j, active, x, N, stream))) goto done;
     if (est_stop && cyc_done) {
       for (int r = 0; r < nrhs; r++)
         if (active[r]) rn[r] = cabs(g[(size_t)r * (m + 1) + j]);
@@ -492,23 +490,14 @@ done:
     for (int p = 0; p < np; p++) info[p].seconds = now_s() - t0;
   fmbh_sync(stream);
   sys_free(&S);
-  fmbh_free(dV);
-  fmbh_free(dw);
-  fmbh_free(dr);
-  fmbh_free(dh);
-  fmbh_free(dh2);
-  fmbh_free(dy);
-  fmbh_free(dn);
+  gws_free(&own);
   free(Hh);
   free(cs);
   free(sn);
   free(g);
   free(yv);
-  free(hh);
-  free(hh2);
   free(bn);
   free(rn);
-  free(hn);
   free(rsave);
   free(active);
   free(sel);
@@ -518,19 +507,22 @@ done:
 int fmb_gmres(fmb_plan *pl, const fmb_c64 *b, fmb_c64 *x, int nrhs,
               int restart, double tol, int maxit, fmb_gmres_info *info,
               void *stream) {
-  return gmres_run(&pl, &nrhs, 1, 0, 0, b, x, restart, tol, maxit, 0, info, stream);
+  return gmres_run(&pl, &nrhs, 1, 0, 0, b, x, restart, tol, maxit, 0, NULL, info,
+                   stream);
 }
 
 int fmb_gmres_transpose(fmb_plan *pl, const fmb_c64 *b, fmb_c64 *x, int nrhs,
                         int restart, double tol, int maxit, fmb_gmres_info *info,
                         void *stream) {
-  return gmres_run(&pl, &nrhs, 1, 1, 0, b, x, restart, tol, maxit, 0, info, stream);
+  return gmres_run(&pl, &nrhs, 1, 1, 0, b, x, restart, tol, maxit, 0, NULL, info,
+                   stream);
 }
 
 int fmb_gmres_batch(fmb_plan *const *plans, const int *nrhs, int nplans, int graph,
                     const fmb_c64 *b, fmb_c64 *x, int restart, double tol, int maxit,
                     fmb_gmres_info *info, void *stream) {
-  return gmres_run(plans, nrhs, nplans, 0, graph, b, x, restart, tol, maxit, 0, info, stream);
+  return gmres_run(plans, nrhs, nplans, 0, graph, b, x, restart, tol, maxit, 0, NULL, info,
+                   stream);
 }
 
 /* Robin coefficients of two plans on one tree agree (both rigid or equal) */
@@ -596,54 +588,41 @@ static int refined_run(fmb_plan *const *outers, fmb_plan *const *inners, const i
   const int N = outers[0]->tree->nelem;
   double t0 = now_s();
   const size_t vbytes = sizeof(fmb_c64) * (size_t)N * nrhs;
-  fmb_c64 *dw = NULL, *dr = NULL, *dd = NULL, *dh = NULL, *dh2 = NULL;
-  double *dn = NULL, *bn = NULL, *rn = NULL, *tn = NULL;
-  fmb_c64 *one = NULL, *mone = NULL;
+  fmb_c64 *dw = NULL, *dr = NULL, *dd = NULL;
+  double *bn = NULL, *rn = NULL;
+  const double *hx, *hb;
+  gws_t W; /* of the inner solves; its norms serve the outer residuals too */
+  memset(&W, 0, sizeof(W));
   fmb_gmres_info *ii = NULL;
   int *off = NULL, *pdone = NULL, *mvin = NULL, *mv64 = NULL;
   int iters = 0, cycles = 0, conv = 0, x_zero = 1;
   if ((rc = fmbh_malloc((void **)&dw, vbytes))) goto done;
   if ((rc = fmbh_malloc((void **)&dr, vbytes))) goto done;
   if ((rc = fmbh_malloc((void **)&dd, vbytes))) goto done;
-  if ((rc = fmbh_malloc((void **)&dh, sizeof(fmb_c64) * nrhs))) goto done;
-  if ((rc = fmbh_malloc((void **)&dh2, sizeof(fmb_c64) * nrhs))) goto done;
-  if ((rc = fmbh_malloc((void **)&dn, sizeof(double) * nrhs))) goto done;
+  if ((rc = gws_init(&W, restart, nrhs, N, stream))) goto done;
   bn = (double *)malloc(sizeof(double) * nrhs);
   rn = (double *)malloc(sizeof(double) * nrhs);
-  tn = (double *)malloc(sizeof(double) * nrhs);
-  one = (fmb_c64 *)malloc(sizeof(fmb_c64) * nrhs);
-  mone = (fmb_c64 *)malloc(sizeof(fmb_c64) * nrhs);
   ii = (fmb_gmres_info *)calloc((size_t)np, sizeof(fmb_gmres_info));
   off = (int *)malloc(sizeof(int) * (np + 1));
   pdone = (int *)calloc((size_t)np, sizeof(int));
   mvin = (int *)calloc((size_t)np, sizeof(int));
   mv64 = (int *)calloc((size_t)np, sizeof(int));
-  if (!bn || !rn || !tn || !one || !mone || !ii || !off || !pdone || !mvin || !mv64) {
+  if (!bn || !rn || !ii || !off || !pdone || !mvin || !mv64) {
     rc = fmb_set_error(FMB_ERR_NOMEM, "fmb_gmres_refined host workspace");
     goto done;
   }
   off[0] = 0;
   for (int p = 0; p < np; p++) off[p + 1] = off[p] + nrs[p];
+  if ((rc = first_norms(&W, b, x, dr, nrhs, N, &hx, &hb, stream))) goto done;
   for (int r = 0; r < nrhs; r++) {
-    one[r].re = 1.0;
-    one[r].im = 0.0;
-    mone[r].re = -1.0;
-    mone[r].im = 0.0;
-  }
-  if ((rc = fmbh_h2d(dh, one, sizeof(fmb_c64) * nrhs, stream))) goto done;
-  if ((rc = fmbh_h2d(dh2, mone, sizeof(fmb_c64) * nrhs, stream))) goto done;
-  if ((rc = fmbh_znorms(x, nrhs, N, dn, stream))) goto done;
-  if ((rc = fmbh_d2h(rn, dn, sizeof(double) * nrhs, stream))) goto done;
-  for (int r = 0; r < nrhs; r++) {
-    if (!isfinite(rn[r])) {
+    if (!isfinite(hx[r])) {
       rc = fmb_set_error(FMB_ERR_ARG, "fmb_gmres_refined: initial guess %d holds NaN or Inf", r);
       goto done;
     }
-    x_zero &= rn[r] == 0.0;
+    x_zero &= hx[r] == 0.0;
   }
-  if ((rc = fmbh_znorms(b, nrhs, N, dn, stream))) goto done;
-  if ((rc = fmbh_d2h(bn, dn, sizeof(double) * nrhs, stream))) goto done;
   for (int r = 0; r < nrhs; r++) {
+    bn[r] = hb[r];
     if (!isfinite(bn[r])) {
       rc = fmb_set_error(FMB_ERR_ARG, "fmb_gmres_refined: right-hand side %d holds NaN or Inf",
                          r);
@@ -652,26 +631,24 @@ static int refined_run(fmb_plan *const *outers, fmb_plan *const *inners, const i
     if (bn[r] == 0.0) bn[r] = 1.0;
   }
   while (1) {
-    /* r = b - A_out x in FP64 (r = b for a zero first guess); converged
-     * plans keep r = 0 */
-    if ((rc = fmbh_d2d(dr, b, vbytes, stream))) goto done;
-    if (!x_zero) {
-      for (int p = 0; p < np; p++) {
-        if (pdone[p]) continue;
-        const size_t o = (size_t)off[p] * N;
-        if ((rc = plan_apply(outers[p], trans, FMB_FP64, x + o, dw + o, nrs[p], stream)))
-          goto done;
-        mv64[p]++;
-        if ((rc = fmbh_zaxpby(dh2 + off[p], dw + o, dh + off[p], dr + o, nrs[p], N, stream)))
-          goto done;
-      }
+    /* r = b - A_out x in FP64 (r = b, as set above, for a zero first guess);
+     * finished plans keep the norms they converged with and r = 0 */
+    if (x_zero) memcpy(rn, hb, sizeof(double) * nrhs);
+    for (int p = 0; p < np && !x_zero; p++) {
+      const size_t o = (size_t)off[p] * N;
+      if (pdone[p]) continue;
+      if ((rc = plan_apply(outers[p], trans, FMB_FP64, x + o, dw + o, nrs[p], stream))) goto done;
+      mv64[p]++;
+      fmbh_vecws v = W.v;
+      v.hpn += off[p];
+      if ((rc = fmbh_resid(b + o, dw + o, dr + o, nrs[p], N, &v, stream))) goto done;
     }
-    if ((rc = fmbh_znorms(dr, nrhs, N, dn, stream))) goto done;
-    if ((rc = fmbh_d2h(tn, dn, sizeof(double) * nrhs, stream))) goto done;
-    /* finished plans keep the norms they converged with */
-    for (int p = 0; p < np; p++)
-      if (!pdone[p])
-        for (int r = off[p]; r < off[p + 1]; r++) rn[r] = tn[r];
+    if (!x_zero) {
+      if ((rc = fmbh_sync(stream))) goto done;
+      for (int p = 0; p < np; p++)
+        if (!pdone[p])
+          for (int r = off[p]; r < off[p + 1]; r++) rn[r] = W.v.hpn[r];
+    }
     conv = 1;
     for (int r = 0; r < nrhs; r++)
       if (!isfinite(rn[r])) {
@@ -694,13 +671,13 @@ static int refined_run(fmb_plan *const *outers, fmb_plan *const *inners, const i
     if ((rc = fmbh_memset(dd, 0, vbytes, stream))) goto done;
     memset(ii, 0, sizeof(fmb_gmres_info) * np);
     rc = gmres_run(inners, nrs, np, trans, graph, dr, dd, restart, inner_tol, maxit - iters, 1,
-                   ii, stream);
+                   &W, ii, stream);
     if (rc && rc != FMB_ERR_NOCONV) goto done;
     iters += ii[0].iters;
     for (int p = 0; p < np; p++) mvin[p] += ii[p].matvecs_fp64 + ii[p].matvecs_work;
     cycles++;
-    /* x = 1 * d + 1 * x */
-    if ((rc = fmbh_zaxpby(dh, dd, dh, x, nrhs, N, stream))) goto done;
+    /* x += d */
+    if ((rc = fmbh_zadd(dd, x, (size_t)N * nrhs, stream))) goto done;
     x_zero = 0;
   }
   rc = conv ? FMB_OK
@@ -723,14 +700,9 @@ done:
   fmbh_free(dw);
   fmbh_free(dr);
   fmbh_free(dd);
-  fmbh_free(dh);
-  fmbh_free(dh2);
-  fmbh_free(dn);
+  gws_free(&W);
   free(bn);
   free(rn);
-  free(tn);
-  free(one);
-  free(mone);
   free(ii);
   free(off);
   free(pdone);
