@@ -142,6 +142,7 @@ __device__ inline void dev_sph_jn(int nmax, double x, double *j) {
   double ax = fabs(x);
   double top = nk > ax ? (double)nk : ax;
   int nst = (int)ceil(top) + 40 + (int)ceil(6.0 * cbrt(top));
+  const double ix = 1.0 / x;
   double fp1 = 0.0, fc = 1.0, sum = 0.0, f0 = 0.0, f1 = 0.0;
   for (int n = nst; n >= 0; n--) {
     if (n <= nmax) j[n] = fc;
@@ -149,7 +150,7 @@ __device__ inline void dev_sph_jn(int nmax, double x, double *j) {
     if (n == 1) f1 = fc;
     sum += (2.0 * n + 1.0) * fc * fc;
     if (n == 0) break;
-    double fm1 = (2.0 * n + 1.0) / x * fc - fp1;
+    double fm1 = (2.0 * n + 1.0) * ix * fc - fp1;
     fp1 = fc;
     fc = fm1;
     if (fabs(fc) > 1e100) {
@@ -200,17 +201,19 @@ __device__ inline void panel_sum(double k, const double *x, const double *nx,
     double s, c;
     sincos(k * r, &s, &c);
     double w = qq[3] * area;
-    double g0 = 1.0 / (4.0 * M_PI * r);
+    // one division a point (81,920 panels at 32 points: 120 us, 142 with six)
+    double ir = 1.0 / r;
+    double g0 = (1.0 / (4.0 * M_PI)) * ir;
     double gr = c * g0, gi = s * g0;
-    double rnx = (d[0] * nx[0] + d[1] * nx[1] + d[2] * nx[2]) / r;
-    double rny = -(d[0] * ny[0] + d[1] * ny[1] + d[2] * ny[2]) / r;
+    double rnx = (d[0] * nx[0] + d[1] * nx[1] + d[2] * nx[2]) * ir;
+    double rny = -(d[0] * ny[0] + d[1] * ny[1] + d[2] * ny[2]) * ir;
     // gp = g (-1/r + i k)
-    double gpr = -gr / r - k * gi, gpi = -gi / r + k * gr;
+    double gpr = -gr * ir - k * gi, gpi = -gi * ir + k * gr;
     double nn = nx[0] * ny[0] + nx[1] * ny[1] + nx[2] * ny[2];
     // d2G = e/(4 pi r^3) [ (3 - k^2 r^2 - 3ikr) rnx rny + (1 - ikr) nn ]
     double ar = (3.0 - k * k * r * r) * rnx * rny + nn;
     double ai = -3.0 * k * r * rnx * rny - k * r * nn;
-    double h0 = g0 / (r * r);
+    double h0 = g0 * ir * ir;
     double hr = h0 * (c * ar - s * ai), hi = h0 * (c * ai + s * ar);
     out[0].x += w * gr;
     out[0].y += w * gi;
@@ -227,147 +230,243 @@ __device__ inline void panel_sum(double k, const double *x, const double *nx,
  * contour integrals over its three edges (integral.cu:202-249, 666-751):
  *   S = (1/4pi) oint (e^{ik rho}-1)/(ik) dtheta
  *   T = -(1/4pi) [ oint (e^{ik rho}-1)/rho dtheta + oint dtheta/rho - 2 pi i k ]
- * with nedge Gauss points per edge (edge: {x, w} pairs on [-1,1]). */
+ * with nedge Gauss points per edge (edge: {x, w} pairs on [-1,1]).  By a
+ * whole wavefront, one point a lane, the result in every lane: by one lane
+ * while 63 wait, the 72 points of a panel took longer than its row of near
+ * entries. */
+__device__ __forceinline__ double wave_all_sum(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
 __device__ inline void self_terms(double k, const double *tri, const double *c,
-                           const double *edge, int nedge, double2 &S,
+                           const double *edge, int nedge, int lane, double2 &S,
                            double2 &T) {
-  double sSr = 0, sSi = 0, sTr = 0, sTi = 0, sinv = 0;
-  for (int e = 0; e < 3; e++) {
-    const double *P = tri + 3 * e, *Q = tri + 3 * ((e + 1) % 3);
-    double ev[3], L = 0;
-    for (int i = 0; i < 3; i++) {
-      ev[i] = Q[i] - P[i];
-      L += ev[i] * ev[i];
+  double sSr = 0, sSi = 0, sTr = 0, sTi = 0;
+  for (int i = lane; i < 3 * nedge; i += 64) {
+    const int e = i / nedge, q = i - e * nedge;
+    double P[3], Q[3], ev[3], L = 0;
+    for (int a = 0; a < 3; a++) {
+      P[a] = e == 0 ? tri[a] : e == 1 ? tri[3 + a] : tri[6 + a];
+      Q[a] = e == 0 ? tri[3 + a] : e == 1 ? tri[6 + a] : tri[a];
+      ev[a] = Q[a] - P[a];
+      L += ev[a] * ev[a];
     }
     L = sqrt(L);
     double tp = 0;
-    for (int i = 0; i < 3; i++) {
-      ev[i] /= L;
-      tp += (c[i] - P[i]) * ev[i];
+    for (int a = 0; a < 3; a++) {
+      ev[a] /= L;
+      tp += (c[a] - P[a]) * ev[a];
     }
     double h = 0;
-    for (int i = 0; i < 3; i++) {
-      double f = P[i] + tp * ev[i] - c[i];
+    for (int a = 0; a < 3; a++) {
+      double f = P[a] + tp * ev[a] - c[a];
       h += f * f;
     }
     h = sqrt(h);
     double thP = atan2(-tp, h), thQ = atan2(L - tp, h);
-    sinv += (sin(thQ) - sin(thP)) / h;
+    if (q == 0) sTr += (sin(thQ) - sin(thP)) / h;
     double half = 0.5 * (thQ - thP), mid = 0.5 * (thQ + thP);
-    for (int q = 0; q < nedge; q++) {
-      double th = mid + half * edge[2 * q];
-      double rho = h / cos(th);
-      double w = half * edge[2 * q + 1];
-      double s2, c2;
-      sincos(0.5 * k * rho, &s2, &c2);
-      // gs = 2 sin(k rho/2) e^{i k rho/2} / k
-      double gr, gi;
-      if (k == 0.0) {
-        gr = rho;
-        gi = 0;
-      } else {
-        gr = 2.0 * s2 * c2 / k;
-        gi = 2.0 * s2 * s2 / k;
-      }
-      sSr += w * gr;
-      sSi += w * gi;
-      // i k gs / rho
-      sTr += w * (-k * gi / rho);
-      sTi += w * (k * gr / rho);
+    double th = mid + half * edge[2 * q];
+    double rho = h / cos(th);
+    double w = half * edge[2 * q + 1];
+    double s2, c2;
+    sincos(0.5 * k * rho, &s2, &c2);
+    // gs = 2 sin(k rho/2) e^{i k rho/2} / k
+    double gr, gi;
+    if (k == 0.0) {
+      gr = rho;
+      gi = 0;
+    } else {
+      gr = 2.0 * s2 * c2 / k;
+      gi = 2.0 * s2 * s2 / k;
     }
+    sSr += w * gr;
+    sSi += w * gi;
+    // i k gs / rho
+    sTr += w * (-k * gi / rho);
+    sTi += w * (k * gr / rho);
   }
+  sSr = wave_all_sum(sSr);
+  sSi = wave_all_sum(sSi);
+  sTr = wave_all_sum(sTr);
+  sTi = wave_all_sum(sTi);
   const double f = 1.0 / (4.0 * M_PI);
   S = make_double2(f * sSr, f * sSi);
-  T = make_double2(-f * (sTr + sinv), -f * (sTi - 2.0 * M_PI * k));
+  T = make_double2(-f * sTr, -f * (sTi - 2.0 * M_PI * k));
 }
-
 
 /* ---- spherical basis tables (P2M / L2P bases, shape sensitivities) ---- */
+
+/* degree and order of entry f of a table of n = 0, 1, ..., m = 0 .. n */
 __device__ __forceinline__ int tri_idx(int n, int m) { return n * (n + 1) / 2 + m; }
+__device__ __forceinline__ void tri_nm(int f, int &n, int &m) {
+  n = (int)((sqrtf(8.0f * f + 1.0f) - 1.0f) * 0.5f);
+  n -= tri_idx(n, 0) > f;
+  n += tri_idx(n + 1, 0) <= f;
+  m = f - tri_idx(n, 0);
+}
 
-// Fill Rt[(n,m)] = R_n^m(v), n <= nm, in LDS, in a workgroup of one
-// 64-lane wavefront.  Scratch in LDS as given.
-__device__ inline void r_table(int nm, double k, const double *v, double *jn,
-                        double *diag, double *Pt, double2 *ph, double2 *Rt,
-                        double *geo) {
-  int lane = threadIdx.x;
-  if (lane == 0) {
-    double rho2 = v[0] * v[0] + v[1] * v[1];
-    double r = sqrt(rho2 + v[2] * v[2]);
-    double ct = 1.0, st = 0.0, phi = 0.0;
-    if (r > 0) {
-      ct = v[2] / r;
-      st = sqrt(rho2) / r;
-      phi = atan2(v[1], v[0]);
+/* R_n^m(v), n <= nm, m >= 0 (R_n^{-m} is its conjugate), of one wavefront's
+ * points in LDS: Rs the sum over the points with weights, R1 one more point.
+ * The points' serial parts (the Bessel recurrence, its 70 steps the longest
+ * chain here) run side by side, a point a lane; then a lane runs column m of
+ * the Legendre functions up for one point, 1, 2 or 4 points at a time by the
+ * order.  With a point after the other and one lane at the recurrences of
+ * each, a table cost 20,000 cycles. */
+constexpr int kRPts = 16; /* points of a pass */
+struct r_lds {
+  double2 *Rs, *R1, *leg; /* nt entries each; leg: recurrence factors      */
+  double2 *part;          /* further sums, a table each                    */
+  double *pt, *jn;        /* cos, sin, azimuth, weight; j_n of each point  */
+};
+static inline __host__ __device__ int r_slots(int nm) { return nm < 16 ? 4 : nm < 32 ? 2 : 1; }
+static inline __host__ __device__ size_t r_lds_bytes(int nm, int one) {
+  const size_t nt = (size_t)(nm + 1) * (nm + 2) / 2;
+  return 16 * nt * (1 + r_slots(nm) + (one ? 1 : 0)) + 8 * (size_t)kRPts * (nm + 5);
+}
+__device__ __forceinline__ r_lds r_lds_at(void *p, int nm, int one) {
+  const int nt = (nm + 1) * (nm + 2) / 2;
+  r_lds t;
+  t.leg = (double2 *)p;
+  t.Rs = t.leg + nt;
+  t.part = t.Rs + nt;
+  t.R1 = t.part + (r_slots(nm) - 1) * nt;
+  t.pt = (double *)(t.R1 + (one ? nt : 0));
+  t.jn = t.pt + 4 * kRPts;
+  return t;
+}
+
+/* np points with weights (point(q, v, w)), then, with one set, point np for
+ * R1; np >= 1 */
+template <typename F>
+__device__ inline void r_tables(int nm, double k, int np, int one, F point, const r_lds &t) {
+  const int lane = threadIdx.x, nt = (nm + 1) * (nm + 2) / 2;
+  for (int f = lane; f < nt; f += 64) {
+    int n, m;
+    tri_nm(f, n, m);
+    double a, b = 0.0;
+    if (n == m) { /* P_m^m = a sin^m */
+      a = 1.0 / (4.0 * M_PI);
+      for (int i = 1; i <= m; i++) a *= (2.0 * i + 1.0) / (2.0 * i);
+      a = sqrt(a);
+    } else { /* P_n^m = a (cos P_{n-1}^m - b P_{n-2}^m) */
+      a = sqrt((4.0 * n * n - 1.0) / ((double)n * n - (double)m * m));
+      if (n > m + 1)
+        b = sqrt((((double)(n - 1) * (n - 1)) - (double)m * m) /
+                 (4.0 * (n - 1) * (n - 1) - 1.0));
     }
-    geo[0] = ct;
-    geo[1] = st;
-    geo[2] = phi;
-    dev_sph_jn(nm, k * r, jn);
-    double d = 1.0 / sqrt(4.0 * M_PI);
-    diag[0] = d;
-    for (int m = 1; m <= nm; m++) {
-      d *= sqrt((2.0 * m + 1.0) / (2.0 * m)) * st;
-      diag[m] = d;
-    }
+    t.leg[f] = make_double2(a, b);
   }
-  __syncthreads();
-  double ct = geo[0], phi = geo[2];
-  for (int m = lane; m <= nm; m += 64) {
-    double p2 = 0.0, p1 = diag[m];
-    Pt[tri_idx(m, m)] = p1;
-    for (int n = m + 1; n <= nm; n++) {
-      double pv;
-      if (n == m + 1)
-        pv = sqrt(2.0 * m + 3.0) * ct * p1;
-      else {
-        double a = sqrt((4.0 * n * n - 1.0) / ((double)n * n - (double)m * m));
-        double b = sqrt((((double)(n - 1) * (n - 1)) - (double)m * m) /
-                        (4.0 * (n - 1) * (n - 1) - 1.0));
-        pv = a * (ct * p1 - b * p2);
+  const int slots = r_slots(nm), wd = 64 / slots, slot = lane / wd, lm = lane % wd;
+  double2 *Rp = slot ? t.part + (slot - 1) * nt : t.Rs;
+  const int all = np + (one ? 1 : 0);
+  for (int q0 = 0; q0 < all; q0 += kRPts) {
+    const int nq = min(kRPts, all - q0);
+    __syncthreads();
+    if (lane < nq) {
+      double v[3], w;
+      point(q0 + lane, v, w);
+      double rho2 = v[0] * v[0] + v[1] * v[1];
+      double r = sqrt(rho2 + v[2] * v[2]);
+      double ct = 1.0, st = 0.0, phi = 0.0;
+      if (r > 0) {
+        ct = v[2] / r;
+        st = sqrt(rho2) / r;
+        phi = atan2(v[1], v[0]);
       }
-      Pt[tri_idx(n, m)] = pv;
-      p2 = p1;
-      p1 = pv;
+      double *pt = t.pt + 4 * lane;
+      pt[0] = ct;
+      pt[1] = st;
+      pt[2] = phi;
+      pt[3] = w;
+      dev_sph_jn(nm, k * r, t.jn + lane * (nm + 1));
     }
-    double s, c;
-    sincos(m * phi, &s, &c);
-    ph[m] = make_double2(c, s);
+    __syncthreads();
+    for (int i = slot; i < nq; i += slots) {
+      const int q = q0 + i;
+      const double ct = t.pt[4 * i], st = t.pt[4 * i + 1], phi = t.pt[4 * i + 2];
+      const double w = q < np ? t.pt[4 * i + 3] : 1.0;
+      const double *jn = t.jn + i * (nm + 1);
+      double2 *R = q < np ? Rp : t.R1;
+      const bool add = q < np && q >= slots;
+      for (int m = lm; m <= nm; m += wd) {
+        double pw = 1.0, base = st;
+        for (int e = m; e > 0; e >>= 1) {
+          if (e & 1) pw *= base;
+          base *= base;
+        }
+        double s, c;
+        sincos(m * phi, &s, &c);
+        c *= w;
+        s *= w;
+        double p1 = t.leg[tri_idx(m, m)].x * pw, p2 = 0.0;
+        for (int n = m; n <= nm; n++) {
+          const int f = tri_idx(n, m);
+          if (n > m) {
+            const double2 ab = t.leg[f];
+            const double pv = ab.x * (ct * p1 - ab.y * p2);
+            p2 = p1;
+            p1 = pv;
+          }
+          const double a = jn[n] * p1;
+          double2 v = make_double2(a * c, a * s);
+          if (add) {
+            v.x += R[f].x;
+            v.y += R[f].y;
+          }
+          R[f] = v;
+        }
+      }
+    }
   }
   __syncthreads();
-  for (int f = lane; f < (nm + 1) * (nm + 1); f += 64) {
-    int n = (int)sqrt((double)f);
-    while (n * n > f) n--;
-    while ((n + 1) * (n + 1) <= f) n++;
-    int m = f - n * n - n, am = m < 0 ? -m : m;
-    double a = jn[n] * Pt[tri_idx(n, am)];
-    double2 e = ph[am];
-    Rt[f] = make_double2(a * e.x, m < 0 ? -a * e.y : a * e.y);
+  const int ns = min(slots, np);
+  if (ns > 1) {
+    for (int f = lane; f < nt; f += 64) {
+      double2 v = t.Rs[f];
+      for (int s = 1; s < ns; s++) {
+        v.x += t.part[(s - 1) * nt + f].x;
+        v.y += t.part[(s - 1) * nt + f].y;
+      }
+      t.Rs[f] = v;
+    }
+    __syncthreads();
   }
-  __syncthreads();
 }
 
-__device__ __forceinline__ double2 rget(const double2 *Rt, int n, int m) {
-  if (n < 0 || (m < 0 ? -m : m) > n) return make_double2(0.0, 0.0);
-  return Rt[n * n + n + m];
+/* dR_n^m/dn, m >= 0, of a table of m >= 0 (integral.cu:284-331); f: its
+ * factors, which depend on n and m only */
+struct dr_fac {
+  double f0, f1, f2, f3, f4, f5;
+};
+__device__ __forceinline__ dr_fac dr_factors(int n, int m) {
+  dr_fac f;
+  f.f0 = bcoef(n + 1, -m - 1);
+  f.f1 = bcoef(n, m);
+  f.f2 = bcoef(n + 1, m - 1);
+  f.f3 = bcoef(n, -m);
+  f.f4 = acoef(n - 1, m);
+  f.f5 = acoef(n, m);
+  return f;
 }
-
-// dR_n^m/dn (integral.cu:284-331)
-__device__ __forceinline__ double2 dRdn(const double2 *Rt, int n, int m,
+__device__ __forceinline__ double2 r_get(const double2 *R, int n, int m) {
+  if (m > n || n < 0) return make_double2(0.0, 0.0);
+  if (m >= 0) return R[tri_idx(n, m)];
+  if (-m > n) return make_double2(0.0, 0.0);
+  const double2 v = R[tri_idx(n, -m)];
+  return make_double2(v.x, -v.y);
+}
+__device__ __forceinline__ double2 dRdn(const double2 *R, int n, int m, const dr_fac &f,
                                         double k, const double *nr) {
-  double2 a1 = rget(Rt, n + 1, m + 1), a2 = rget(Rt, n - 1, m + 1);
-  double2 b1 = rget(Rt, n + 1, m - 1), b2 = rget(Rt, n - 1, m - 1);
-  double2 c1 = rget(Rt, n - 1, m), c2 = rget(Rt, n + 1, m);
-  double f0 = bcoef(n + 1, -m - 1), f1 = bcoef(n, m);
-  double f2 = bcoef(n + 1, m - 1), f3 = bcoef(n, -m);
-  double f4 = acoef(n - 1, m), f5 = acoef(n, m);
-  double t0r = f0 * a1.x - f1 * a2.x, t0i = f0 * a1.y - f1 * a2.y;
-  double t1r = f2 * b1.x - f3 * b2.x, t1i = f2 * b1.y - f3 * b2.y;
-  double t2r = f4 * c1.x - f5 * c2.x, t2i = f4 * c1.y - f5 * c2.y;
+  double2 a1 = r_get(R, n + 1, m + 1), a2 = r_get(R, n - 1, m + 1);
+  double2 b1 = r_get(R, n + 1, m - 1), b2 = r_get(R, n - 1, m - 1);
+  double2 c1 = r_get(R, n - 1, m), c2 = r_get(R, n + 1, m);
+  double t0r = f.f0 * a1.x - f.f1 * a2.x, t0i = f.f0 * a1.y - f.f1 * a2.y;
+  double t1r = f.f2 * b1.x - f.f3 * b2.x, t1i = f.f2 * b1.y - f.f3 * b2.y;
+  double t2r = f.f4 * c1.x - f.f5 * c2.x, t2i = f.f4 * c1.y - f.f5 * c2.y;
   double hx = 0.5 * k * nr[0], hy = 0.5 * k * nr[1], kz = k * nr[2];
   return make_double2(hx * t0r + hy * t0i + hx * t1r - hy * t1i + kz * t2r,
                       hx * t0i - hy * t0r + hx * t1i + hy * t1r + kz * t2i);
 }
-
 
 #endif
