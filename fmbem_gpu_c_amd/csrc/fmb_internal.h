@@ -93,6 +93,10 @@ typedef struct fmb_rcr_tab {
   int bf[2];            /* per opset: split-BF16 rotations                 */
   int *d_sched[2];      /* per opset: unit schedule                        */
   int sched_len[2];     /* ints in d_sched                                 */
+  /* per opset: the form with 8 waves (d_sched8 NULL: none), for launches of
+   * few workgroups; wide8: for every launch                               */
+  int nt8[2], mt8[2], wide8[2], sched8_len[2];
+  int *d_sched8[2];
   void *d_Cpad[2];      /* per opset: zero-padded coaxial blocks           */
   float tuned_ms[2];    /* per opset: autotuned time of one launch (0: not tuned) */
   size_t cpad_stride;   /* complex values per coaxial matrix in d_Cpad     */

@@ -306,6 +306,70 @@ static int octant_pairs(const fmb_tree *t, int l, fmb_rcr_tab *tb, void *stream)
   return rc;
 }
 
+/* The form with 8 waves beside a shape of the fixed rule (4 waves), for the
+ * launches that leave a CU with too few waves to cover the operators' loads.
+ * That is, first, every launch of an order whose batches leave room for one
+ * workgroup (FP64) or two (FP32) on a CU's LDS: M2L of 327,680 triangles, FP32
+ * with nine right-hand sides, 4 -> 8 waves: order 23 39.7 -> 31.7 ms, 31 24.8
+ * -> 18.3, 42 19.6 -> 13.4, but 18 62.1 -> 65.1; FP64 with one: 31 5.5 -> 4.8,
+ * but 23 8.1 -> 10.5 (an FP64 product occupies its matrix core twice as
+ * long).  In the global workspace, FP64 alone, with 8 vectors a batch and
+ * blocks in one piece: order 94 3.7 -> 2.7 ms, 62 3.1 -> 2.9, 42 4.8 -> 3.9
+ * (FP32 order 62 13.2 -> 13.4).  Second (job_shape), launches that leave half
+ * of the 256 CUs empty: FP64 M2M of 16 workgroups, order 16, 21 -> 17 us, of
+ * 64, order 23, 36 -> 33, but of 204 41 -> 42. */
+static int wide_form(fmb_plan *pl, fmb_rcr_tab *tb, int op, const int *hoff, const int *coff,
+                     void *stream) {
+  const int prec = pl->ops[op].prec, P = tb->P, mode = tb->mode[op];
+  if (pl->prm.waves || pl->prm.autotune || tb->bf[op] ||
+      (mode != FMBH_RCR_LDS && mode != FMBH_RCR_GWS))
+    return FMB_OK;
+  int nt = tb->nt[op], mt = tb->mt[op], wide, rc;
+  if (mode == FMBH_RCR_GWS) {
+    if (prec != FMB_FP64 || pl->prm.rcr_mode == FMB_RCR_MODE_GWS) return FMB_OK;
+    nt = 1;
+    mt = fmbh_rcr_mt_lds(P, 0) ? fmbh_rcr_mt_lds(P, 0) : 6;
+    wide = 1;
+  } else {
+    const size_t b = fmbh_rcr_lds_bytes(P, prec, nt, tb->sched_len[op]);
+    wide = 160 * 1024 / b <= (prec == FMB_FP64 ? 1 : 2);
+  }
+  int *sched = NULL, slen = 0;
+  if ((rc = build_sched(tb->pin, tb->pout, P, mode, mt, 8, hoff, 0, coff, &sched, &slen, stream)))
+    return rc;
+  if (mode == FMBH_RCR_LDS && fmbh_rcr_lds_bytes(P, prec, nt, slen) > 160 * 1024) {
+    fmbh_free(sched);
+    return FMB_OK;
+  }
+  tb->nt8[op] = nt;
+  tb->mt8[op] = mt;
+  tb->wide8[op] = wide;
+  tb->d_sched8[op] = sched;
+  tb->sched8_len[op] = slen;
+  return FMB_OK;
+}
+
+/* tile shape of one launch */
+static void job_shape(const fmb_rcr_tab *tb, int op, int nrhs, fmbh_rcr_job *j) {
+  j->mode = tb->mode[op];
+  j->bf = tb->bf[op];
+  const int v = 8 * tb->nt[op];
+  const long wgs = (long)j->nchunks * ((j->chunk_pairs * nrhs + v - 1) / v);
+  if (tb->d_sched8[op] && (tb->wide8[op] || wgs <= 128)) {
+    j->nt = tb->nt8[op];
+    j->mt = tb->mt8[op];
+    j->nw = 8;
+    j->sched = tb->d_sched8[op];
+    j->sched_len = tb->sched8_len[op];
+    return;
+  }
+  j->nt = tb->nt[op];
+  j->mt = tb->mt[op];
+  j->nw = tb->nw[op];
+  j->sched = tb->d_sched[op];
+  j->sched_len = tb->sched_len[op];
+}
+
 /* tile shapes, schedules and padded coaxial blocks of one translation;
  * C: the scaled coaxial matrices of each opset (ncoax of them, order P) */
 static int plan_tab(fmb_plan *pl, fmb_rcr_tab *tb, int pin, int pout,
@@ -354,6 +418,7 @@ static int plan_tab(fmb_plan *pl, fmb_rcr_tab *tb, int pin, int pout,
                           tb->bf[op] ? hboff : hoff, tb->bf[op], coff, &tb->d_sched[op],
                           &tb->sched_len[op], stream)))
       break;
+    if ((rc = wide_form(pl, tb, op, hoff, coff, stream))) break;
     if (!d_coff) {
       if ((rc = fmbh_malloc((void **)&d_coff, sizeof(int) * (mn + 1)))) break;
       if ((rc = fmbh_h2d(d_coff, coff, sizeof(int) * (mn + 1), stream))) break;
@@ -1099,6 +1164,7 @@ void fmbx_rcr_free(fmb_plan *pl) {
       fmbh_free(tb->d_chi);
       for (int op = 0; op < 2; op++) {
         fmbh_free(tb->d_sched[op]);
+        fmbh_free(tb->d_sched8[op]);
         fmbh_free(tb->d_Cpad[op]);
         for (int i = 0; i < 2; i++) {
           fmbh_free(tb->d_ts_pairs[op][i]);
@@ -1136,17 +1202,13 @@ int fmbx_rcr_run(const fmb_plan *pl, int op, int kind, int l, int nrhs,
   const fmb_rcr_tab *pairs = kind == 0 ? tb : &pl->rcr[1][l];
   fmbh_rcr_job j;
   memset(&j, 0, sizeof(j));
-  j.mode = tb->mode[op];
-  j.nt = tb->nt[op];
-  j.mt = tb->mt[op];
-  j.nw = tb->nw[op];
-  j.bf = tb->bf[op];
   j.Hb = o->d_Hb;
   j.hbstride = 2 * o->hb_half;
   j.hbhalf = o->hb_half;
   j.chunks = pairs->d_chunks;
   j.nchunks = pairs->nchunks;
   j.chunk_pairs = RCR_CHUNK;
+  job_shape(tb, op, nrhs, &j);
   j.H = o->d_Hpad;
   j.hstride = o->hpad_stride;
   j.C = tb->d_Cpad[op];
@@ -1154,8 +1216,6 @@ int fmbx_rcr_run(const fmb_plan *pl, int op, int kind, int l, int nrhs,
   j.P = tb->P;
   j.pin = tb->pin;
   j.pout = tb->pout;
-  j.sched = tb->d_sched[op];
-  j.sched_len = tb->sched_len[op];
   j.hlen = tb->hlen;
   j.xcd = kind == 0 && tb->tiled && j.mode == FMBH_RCR_LDS;
   j.gws = (pl->aux && stream == pl->aux) ? (char *)o->d_gws + o->gws_slot : o->d_gws;
@@ -1210,17 +1270,13 @@ int fmbx_rcr_run_t(const fmb_plan *pl, int op, int kind, int l, int nrhs,
   const fmb_rcr_tab *pairs = kind == 0 ? tb : &pl->rcr[1][l];
   fmbh_rcr_job j;
   memset(&j, 0, sizeof(j));
-  j.mode = tb->mode[op];
-  j.nt = tb->nt[op];
-  j.mt = tb->mt[op];
-  j.nw = tb->nw[op];
-  j.bf = tb->bf[op];
   j.Hb = o->d_Hb;
   j.hbstride = 2 * o->hb_half;
   j.hbhalf = o->hb_half;
   j.chunks = pairs->d_chunks;
   j.nchunks = pairs->nchunks;
   j.chunk_pairs = RCR_CHUNK;
+  job_shape(tb, op, nrhs, &j);
   j.H = o->d_Hpad;
   j.hstride = o->hpad_stride;
   j.C = tb->d_Cpad[op];
@@ -1228,8 +1284,6 @@ int fmbx_rcr_run_t(const fmb_plan *pl, int op, int kind, int l, int nrhs,
   j.P = tb->P;
   j.pin = tb->pin;
   j.pout = tb->pout;
-  j.sched = tb->d_sched[op];
-  j.sched_len = tb->sched_len[op];
   j.hlen = tb->hlen;
   j.xcd = kind == 0 && tb->tiled && j.mode == FMBH_RCR_LDS;
   j.gws = o->d_gws;

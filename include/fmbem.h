@@ -258,7 +258,10 @@ int fmb_plan_retune(fmb_plan *pl, double k, const fmb_c64 *robin, void *stream);
  * pointer may be NULL.  For M2L this is the shape of the offset-batched
  * kernel; levels of order 16 and less whose shape is left to the rule or the
  * autotuner (rcr_mode, waves, ldso and m2l_tile at their defaults) run
- * target-stationary instead where that is faster (csrc/hip/rcr_ts.hip). */
+ * target-stationary instead where that is faster (csrc/hip/rcr_ts.hip).  A
+ * shape of the fixed rule (autotune and waves 0) names the 4-wave form: high
+ * orders and launches of few workgroups run its 8-wave form
+ * (csrc/host/rcr.c). */
 int fmb_plan_tile_shape(const fmb_plan *pl, int kind, int level, int prec, int *mode,
                         int *nt, int *mt, int *nw, int *bf, double *ms);
 /* Wavenumber of the operator the plan holds (0 after a failed retune). */
