@@ -64,7 +64,7 @@ typedef struct fmb_opset {
   void *d_L2P;  /* [N][pL^2] complex                                        */
   void *d_near; /* near blocks, complex                                     */
   void *d_M[FMB_MAXLEV], *d_L[FMB_MAXLEV]; /* [nbox][nrhs][p^2] complex      */
-  void *d_xs, *d_ys; /* sorted-order vectors [nrhs][N] complex                */
+  void *d_xs; /* the caller's vectors in element order [nrhs][N], complex       */
   void *d_gws;       /* global workspace of the GWS-mode translations: one
                         slot per stream the plan launches them on         */
   size_t gws_bytes, gws_slot;

@@ -23,6 +23,13 @@
 
 #define FMB_LAUNCH_CHECK() FMB_HIP_CHECK(hipGetLastError())
 
+/* Block i of n with each of the 8 XCDs (workgroups go round them in turn)
+ * taking a contiguous range: neighbours share an L2. */
+__device__ __forceinline__ int xcd_block(int i, int n) {
+  const int x = i & 7, q = n >> 3, r = n & 7;
+  return x * q + min(x, r) + (i >> 3);
+}
+
 template <typename T> struct cplx {
   T re, im;
 };

@@ -79,11 +79,14 @@ int fmbh_near_assemble(fmb_plan *pl, int op, const fmb_c64 *d_robin_sorted,
 int fmbh_near_layout(fmb_plan *pl, void *stream);
 
 /* ---- FMM pass (fmm.hip) */
-int fmbh_gather(const fmb_plan *pl, int op, const fmb_c64 *x, int nrhs,
-                void *stream);
-int fmbh_scatter(const fmb_plan *pl, int op, fmb_c64 *y, int nrhs,
-                 void *stream);
-int fmbh_p2m(const fmb_plan *pl, int op, int nrhs, void *stream);
+/* start of a pass: the caller's x to element order; by what, its P2M
+ * (transposed L2P) and the cleared coefficient arrays of a product, its
+ * transpose, or an upward pass alone */
+#define FMBH_BEGIN_FWD 0
+#define FMBH_BEGIN_T 1
+#define FMBH_BEGIN_UP 2
+#define FMBH_BEGIN_NEAR 3 /* x only */
+int fmbh_begin(const fmb_plan *pl, int op, int what, const fmb_c64 *x, int nrhs, void *stream);
 int fmbh_m2m(const fmb_plan *pl, int op, int l, int nrhs, void *stream);
 int fmbh_m2l(const fmb_plan *pl, int op, int l, int nrhs, void *stream);
 /* matrix-core RCR translations (rcr_kernels.h, rcr_mfma.hip) */
@@ -180,7 +183,7 @@ int fmbh_ts_rot(int prec, const double *d_H64, int Pmax, int P, const int *d_cbe
 int fmbh_ts_coax(int prec, const void *d_C, int p, const int *d_coff, int cstride, void *out,
                  void *stream);
 int fmbh_l2l(const fmb_plan *pl, int op, int l, int nrhs, void *stream);
-int fmbh_l2p_near(const fmb_plan *pl, int op, int nrhs, int parts,
+int fmbh_l2p_near(const fmb_plan *pl, int op, fmb_c64 *y, int nrhs, int parts,
                   void *stream);
 int fmbh_mmajor_table(int p, int **d_tab, void *stream);
 
@@ -196,8 +199,7 @@ int fmbh_field_tree(const fmb_plan *pl, int op, const fmb_c64 *x, int nrhs,
                     const double *d_dirs, fmb_c64 *out, void *stream);
 /* transposed pass pieces: (-1)^n L2P^T into L[lmax]; near^T + P2M^T into
  * ys with the given near blocks / P2M basis (NULL: the opset's own) */
-int fmbh_l2p_t(const fmb_plan *pl, int op, int nrhs, void *stream);
-int fmbh_near_t(const fmb_plan *pl, int op, const void *near, const void *basis,
+int fmbh_near_t(const fmb_plan *pl, int op, const void *near, const void *basis, fmb_c64 *y,
                 int nrhs, int parts, void *stream);
 /* sigma-derivative tables for the adjoint: P2M basis of dA/dsigma_j's
  * column factor ([N][pL^2]) and its near blocks (near layout) */

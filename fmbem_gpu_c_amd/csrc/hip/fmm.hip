@@ -1,6 +1,6 @@
-// fmm.hip -- the FMM pass on gfx950: gather/scatter between caller and
-// Morton element order, P2M, M2M ("SS"), M2L ("SR"), L2L ("RR"), L2P fused
-// with the near-field block product.
+// fmm.hip -- the FMM pass on gfx950: its start (caller to Morton element
+// order, P2M, cleared sums) and the VALU translations M2M ("SS"), M2L ("SR"),
+// L2L ("RR").
 //
 // Translations are rotate-coaxial-rotate (translation.cu:1711-1808,
 // 3461-3759): with t = (|t|, theta, phi),
@@ -219,44 +219,75 @@ __global__ void __launch_bounds__(GS)
   }
 }
 
-// P2M: one block per leaf box, M[b][r][f] = sum_{e in b} B[e][f] xs[r][e].
-// FLIP multiplies coefficient f = (n, m) by (-1)^n: with B = the L2P basis
-// it is the transposed L2P of the transposed pass.
-template <typename T, bool FLIP>
-__global__ void k_p2m(const int *__restrict__ bstart,
-                      const cplx<T> *__restrict__ B, const cplx<T> *__restrict__ xs,
-                      int N, int ps, cplx<T> *__restrict__ M, int nrhs) {
-  int b = blockIdx.x;
-  int e0 = bstart[b], e1 = bstart[b + 1];
-  for (int r = 0; r < nrhs; r++)
-    for (int f = threadIdx.x; f < ps; f += blockDim.x) {
-      cplx<T> s = cmk<T>(0, 0);
-      for (int e = e0; e < e1; e++)
-        cfma(s, B[(size_t)e * ps + f], xs[(size_t)r * N + e]);
-      if (FLIP && (isqrt_fix(f) & 1)) s = cmk<T>(-s.re, -s.im);
-      M[((size_t)b * nrhs + r) * ps + f] = s;
+// Start of a pass, one launch: a block per leaf box moves the box's elements
+// from the caller's order to xs and sums M[b][r][f] = sum_{e in b} B[e][f]
+// xs[r][e] (B NULL: only moves them); the blocks after those clear the
+// coefficient arrays that the translations add into.  FLIP multiplies
+// coefficient f = (n, m) by (-1)^n: with B = the L2P basis it is the
+// transposed L2P of the transposed pass.  As a gather, a P2M and up to eight
+// fills the start took 24 of the 123 us of a 1,280-triangle product, now 5.
+struct Clear {
+  int n;
+  size_t end[2 * FMB_MAXLEV];  // running 8-byte words
+  double *p[2 * FMB_MAXLEV];
+};
+constexpr int kBegin = 256, kBeginE = 32;
+
+template <typename T, bool FLIP, int RC>
+__global__ void __launch_bounds__(kBegin)
+    k_begin(const int *__restrict__ bstart, const int *__restrict__ perm,
+            const cplx<T> *__restrict__ B, const double2 *__restrict__ x, int N, int ps,
+            cplx<T> *__restrict__ xs, cplx<T> *__restrict__ M, int nrhs, int nbox, Clear cl) {
+  __shared__ cplx<T> xl[RC][kBeginE];
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x >= nbox) {
+    const size_t step = (size_t)(gridDim.x - nbox) * kBegin;
+    size_t i = (size_t)(blockIdx.x - nbox) * kBegin + tid, base = 0;
+    for (int s = 0; s < cl.n; s++) {
+      for (; i < cl.end[s]; i += step) cl.p[s][i - base] = 0.0;
+      base = cl.end[s];
     }
-}
-
-template <typename T>
-__global__ void k_gather(const int *__restrict__ perm, const double2 *__restrict__ x,
-                         int N, int nrhs, cplx<T> *__restrict__ xs) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)N * nrhs) return;
-  int r = (int)(i / N), e = (int)(i % N);
-  double2 v = x[(size_t)r * N + perm[e]];
-  xs[i] = cmk<T>((T)v.x, (T)v.y);
-}
-
-template <typename T>
-__global__ void k_scatter(const int *__restrict__ perm,
-                          const cplx<T> *__restrict__ ys, int N, int nrhs,
-                          double2 *__restrict__ y) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)N * nrhs) return;
-  int r = (int)(i / N), e = (int)(i % N);
-  cplx<T> v = ys[i];
-  y[(size_t)r * N + perm[e]] = make_double2((double)v.re, (double)v.im);
+    return;
+  }
+  const int b = xcd_block(blockIdx.x, nbox);
+  const int e0 = bstart[b], e1 = bstart[b + 1];
+  for (int r0 = 0; r0 < nrhs; r0 += RC) {
+    const int nr = min(RC, nrhs - r0);
+    for (int f0 = 0; f0 < ps; f0 += kBegin) {
+      const int f = f0 + tid;
+      cplx<T> s[RC];
+#pragma unroll
+      for (int r = 0; r < RC; r++) s[r] = cmk<T>(0, 0);
+      for (int c0 = e0; c0 < e1; c0 += kBeginE) {
+        const int ne = min(kBeginE, e1 - c0);
+        __syncthreads();
+        if (tid < RC * kBeginE) {
+          const int r = tid / kBeginE, e = tid % kBeginE;
+          if (r < nr && e < ne) {
+            const double2 v = x[(size_t)(r0 + r) * N + perm[c0 + e]];
+            const cplx<T> z = cmk<T>((T)v.x, (T)v.y);
+            xl[r][e] = z;
+            if (f0 == 0) xs[(size_t)(r0 + r) * N + c0 + e] = z;
+          }
+        }
+        __syncthreads();
+        if (!B || f >= ps) continue;
+#pragma unroll 4
+        for (int e = 0; e < ne; e++) {
+          const cplx<T> be = B[(size_t)(c0 + e) * ps + f];
+#pragma unroll
+          for (int r = 0; r < RC; r++) cfma(s[r], be, xl[r][e]);
+        }
+      }
+      if (!B) break;
+      if (f >= ps) continue;
+      const bool neg = FLIP && (isqrt_fix(f) & 1);
+#pragma unroll
+      for (int r = 0; r < RC; r++)
+        if (r < nr)
+          M[((size_t)b * nrhs + r0 + r) * ps + f] = neg ? cmk<T>(-s[r].re, -s[r].im) : s[r];
+    }
+  }
 }
 
 inline int nblk(size_t n, int b = 256) { return (int)((n + b - 1) / b); }
@@ -306,79 +337,52 @@ extern "C" int fmbh_mmajor_table(int p, int **d_tab, void *stream) {
   return rc;
 }
 
-extern "C" int fmbh_gather(const fmb_plan *pl, int op, const fmb_c64 *x,
-                           int nrhs, void *stream) {
+template <typename T, bool FLIP>
+static int launch_begin(const fmb_plan *pl, const fmb_opset *o, const fmb_c64 *x, int nrhs,
+                        const void *B, void *M, const Clear &cl, hipStream_t st) {
   const fmb_tree *t = pl->tree;
-  size_t n = (size_t)t->nelem * nrhs;
-  hipStream_t st = (hipStream_t)stream;
-  if (pl->ops[op].prec == FMB_FP64)
-    hipLaunchKernelGGL(k_gather<double>, dim3(nblk(n)), dim3(256), 0, st,
-                       t->d_perm, (const double2 *)x, t->nelem, nrhs,
-                       (cplx<double> *)pl->ops[op].d_xs);
-  else
-    hipLaunchKernelGGL(k_gather<float>, dim3(nblk(n)), dim3(256), 0, st,
-                       t->d_perm, (const double2 *)x, t->nelem, nrhs,
-                       (cplx<float> *)pl->ops[op].d_xs);
+  const int nb = t->nbox[t->lmax], ps = pl->p[t->lmax] * pl->p[t->lmax];
+  const size_t w = cl.n ? cl.end[cl.n - 1] : 0;
+  size_t zb = (w + 4 * kBegin - 1) / (4 * kBegin);
+  if (zb > 2048) zb = 2048;
+  // the basis is read once for up to eight right-hand sides
+  auto kern = nrhs == 1   ? k_begin<T, FLIP, 1>
+              : nrhs == 2 ? k_begin<T, FLIP, 2>
+              : nrhs <= 4 ? k_begin<T, FLIP, 4>
+                          : k_begin<T, FLIP, 8>;
+  hipLaunchKernelGGL(kern, dim3(nb + (unsigned)zb), dim3(kBegin), 0, st, t->d_box_start, t->d_perm,
+                     (const cplx<T> *)B, (const double2 *)x, t->nelem, ps, (cplx<T> *)o->d_xs,
+                     (cplx<T> *)M, nrhs, nb, cl);
   FMB_LAUNCH_CHECK();
   return FMB_OK;
 }
 
-extern "C" int fmbh_scatter(const fmb_plan *pl, int op, fmb_c64 *y, int nrhs,
-                            void *stream) {
+extern "C" int fmbh_begin(const fmb_plan *pl, int op, int what, const fmb_c64 *x, int nrhs,
+                          void *stream) {
   const fmb_tree *t = pl->tree;
-  size_t n = (size_t)t->nelem * nrhs;
-  hipStream_t st = (hipStream_t)stream;
-  if (pl->ops[op].prec == FMB_FP64)
-    hipLaunchKernelGGL(k_scatter<double>, dim3(nblk(n)), dim3(256), 0, st,
-                       t->d_perm, (const cplx<double> *)pl->ops[op].d_ys,
-                       t->nelem, nrhs, (double2 *)y);
-  else
-    hipLaunchKernelGGL(k_scatter<float>, dim3(nblk(n)), dim3(256), 0, st,
-                       t->d_perm, (const cplx<float> *)pl->ops[op].d_ys,
-                       t->nelem, nrhs, (double2 *)y);
-  FMB_LAUNCH_CHECK();
-  return FMB_OK;
-}
-
-extern "C" int fmbh_p2m(const fmb_plan *pl, int op, int nrhs, void *stream) {
-  const fmb_tree *t = pl->tree;
-  int L = t->lmax, pL = pl->p[L];
-  hipStream_t st = (hipStream_t)stream;
   const fmb_opset *o = &pl->ops[op];
-  int bs = pL * pL >= 256 ? 256 : (pL * pL >= 128 ? 128 : 64);
-  if (o->prec == FMB_FP64)
-    hipLaunchKernelGGL((k_p2m<double, false>), dim3(t->nbox[L]), dim3(bs), 0, st,
-                       t->d_box_start, (const cplx<double> *)o->d_P2M,
-                       (const cplx<double> *)o->d_xs, t->nelem, pL * pL,
-                       (cplx<double> *)o->d_M[L], nrhs);
-  else
-    hipLaunchKernelGGL((k_p2m<float, false>), dim3(t->nbox[L]), dim3(bs), 0, st,
-                       t->d_box_start, (const cplx<float> *)o->d_P2M,
-                       (const cplx<float> *)o->d_xs, t->nelem, pL * pL,
-                       (cplx<float> *)o->d_M[L], nrhs);
-  FMB_LAUNCH_CHECK();
-  return FMB_OK;
-}
-
-// transposed L2P: L'[L] = (-1)^n L2P^T xs, the start of the transposed pass
-extern "C" int fmbh_l2p_t(const fmb_plan *pl, int op, int nrhs, void *stream) {
-  const fmb_tree *t = pl->tree;
-  int L = t->lmax, pL = pl->p[L];
+  const int L = t->lmax, trans = what == FMBH_BEGIN_T;
   hipStream_t st = (hipStream_t)stream;
-  const fmb_opset *o = &pl->ops[op];
-  int bs = pL * pL >= 256 ? 256 : (pL * pL >= 128 ? 128 : 64);
+  // parents receive the translations of their children as sums, and every
+  // level those of the interaction lists
+  Clear cl;
+  cl.n = 0;
+  size_t end = 0;
+  for (int l = 2; l <= L && what != FMBH_BEGIN_NEAR; l++) {
+    const size_t words = (size_t)t->nbox[l] * nrhs * pl->p[l] * pl->p[l] * o->csz / 8;
+    for (int out = 0; out < 2; out++) {
+      if (out ? what == FMBH_BEGIN_UP : l == L) continue;
+      cl.p[cl.n] = (double *)(out != trans ? o->d_L[l] : o->d_M[l]);
+      cl.end[cl.n++] = end += words;
+    }
+  }
+  void *M = trans ? o->d_L[L] : o->d_M[L];
+  const void *B = what == FMBH_BEGIN_NEAR ? NULL : trans ? o->d_L2P : o->d_P2M;
   if (o->prec == FMB_FP64)
-    hipLaunchKernelGGL((k_p2m<double, true>), dim3(t->nbox[L]), dim3(bs), 0, st,
-                       t->d_box_start, (const cplx<double> *)o->d_L2P,
-                       (const cplx<double> *)o->d_xs, t->nelem, pL * pL,
-                       (cplx<double> *)o->d_L[L], nrhs);
-  else
-    hipLaunchKernelGGL((k_p2m<float, true>), dim3(t->nbox[L]), dim3(bs), 0, st,
-                       t->d_box_start, (const cplx<float> *)o->d_L2P,
-                       (const cplx<float> *)o->d_xs, t->nelem, pL * pL,
-                       (cplx<float> *)o->d_L[L], nrhs);
-  FMB_LAUNCH_CHECK();
-  return FMB_OK;
+    return trans ? launch_begin<double, true>(pl, o, x, nrhs, B, M, cl, st)
+                 : launch_begin<double, false>(pl, o, x, nrhs, B, M, cl, st);
+  return trans ? launch_begin<float, true>(pl, o, x, nrhs, B, M, cl, st)
+               : launch_begin<float, false>(pl, o, x, nrhs, B, M, cl, st);
 }
 
 template <typename T, int GS, int R>

@@ -145,122 +145,210 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
-// L2P + near: one block per leaf box, one wavefront per (row, rhs) job
-template <typename T>
+// L2P + near: one block per leaf box, one wavefront per (row, RC right-hand
+// sides) job, the result in the caller's order.  The neighbourhood is read a box a lane and
+// its columns listed by all threads (by one thread, with a launch of its own
+// for the caller's order, 14 us of a 1,280-triangle product, 9 now); with
+// several right-hand sides a row is read once for four (60,500 triangles, 64
+// right-hand sides, FP32: 1.93 -> 1.74 ms).  Neighbouring boxes share an XCD,
+// since they read the same elements and write to the same cache lines.
+template <typename T, int RC>
 __global__ void __launch_bounds__(256)
     k_l2p_near(const int *__restrict__ bstart, const int *__restrict__ nstart,
                const int *__restrict__ nbox, const int *__restrict__ ncols,
                const unsigned long long *__restrict__ boff,
                const cplx<T> *__restrict__ A, const cplx<T> *__restrict__ E,
                const cplx<T> *__restrict__ Lc, const cplx<T> *__restrict__ xs,
-               cplx<T> *__restrict__ ys, int N, int ps, int nrhs, int parts) {
+               const int *__restrict__ perm, double2 *__restrict__ y, int N, int ps, int nrhs,
+               int parts) {
   extern __shared__ int colj[];
-  int b = blockIdx.x;
-  int r0 = bstart[b], nr = bstart[b + 1] - r0, nc = ncols[b];
-  if (threadIdx.x == 0) {
-    int c = 0;
-    for (int q = nstart[b]; q < nstart[b + 1]; q++) {
-      int o = nbox[q];
-      for (int e = bstart[o]; e < bstart[o + 1]; e++) colj[c++] = e;
+  __shared__ int cpre[28], cfirst[27];
+  const int b = xcd_block(blockIdx.x, gridDim.x);
+  const int r0 = bstart[b], nr = bstart[b + 1] - r0, nc = ncols[b];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int q0 = nstart[b], ncb = nstart[b + 1] - q0;
+  if (wave == 0) {
+    int f = 0, cnt = 0;
+    if (lane < ncb) {
+      const int o = nbox[q0 + lane];
+      f = bstart[o];
+      cnt = bstart[o + 1] - f;
     }
+    int pre = cnt;
+    for (int o = 1; o < 32; o <<= 1) {
+      const int v = __shfl_up(pre, o, 64);
+      if (lane >= o) pre += v;
+    }
+    if (lane < ncb) {
+      cfirst[lane] = f;
+      cpre[lane + 1] = pre;
+    }
+    if (lane == 0) cpre[0] = 0;
   }
   __syncthreads();
-  int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int c = threadIdx.x; c < nc; c += blockDim.x) {
+    int q = 0;
+    while (q + 1 < ncb && cpre[q + 1] <= c) q++;
+    colj[c] = cfirst[q] + (c - cpre[q]);
+  }
+  __syncthreads();
   const cplx<T> *Ab = A + boff[b];
-  for (int job = wave; job < nr * nrhs; job += (blockDim.x >> 6)) {
-    int r = job % nr, rh = job / nr;
-    int i = r0 + r;
-    T sr = 0, si = 0;
+  const int ng = (nrhs + RC - 1) / RC;
+  for (int job = wave; job < nr * ng; job += (blockDim.x >> 6)) {
+    const int r = job % nr, h0 = job / nr * RC, i = r0 + r, to = perm[i];
+    T sr[RC], si[RC];
+    const cplx<T> *x[RC], *l[RC];
+#pragma unroll
+    for (int h = 0; h < RC; h++) {
+      // (right-hand sides beyond the last repeat it: no branch between loads)
+      const int rh = min(h0 + h, nrhs - 1);
+      sr[h] = si[h] = 0;
+      x[h] = xs + (size_t)rh * N;
+      l[h] = Lc + ((size_t)b * nrhs + rh) * ps;
+    }
     const cplx<T> *arow = Ab + (size_t)r * nc;
-    const cplx<T> *x = xs + (size_t)rh * N;
+#pragma unroll 2
     for (int c = (parts & 1) ? lane : nc; c < nc; c += 64) {
-      cplx<T> a = arow[c], v = x[colj[c]];
-      sr += a.re * v.re - a.im * v.im;
-      si += a.re * v.im + a.im * v.re;
+      const cplx<T> a = arow[c];
+      const int j = colj[c];
+#pragma unroll
+      for (int h = 0; h < RC; h++) {
+        const cplx<T> v = x[h][j];
+        sr[h] += a.re * v.re - a.im * v.im;
+        si[h] += a.re * v.im + a.im * v.re;
+      }
     }
     const cplx<T> *e = E + (size_t)i * ps;
-    const cplx<T> *l = Lc + ((size_t)b * nrhs + rh) * ps;
+#pragma unroll 4
     for (int f = (parts & 2) ? lane : ps; f < ps; f += 64) {
-      cplx<T> a = e[f], v = l[f];
-      sr += a.re * v.re - a.im * v.im;
-      si += a.re * v.im + a.im * v.re;
+      const cplx<T> a = e[f];
+#pragma unroll
+      for (int h = 0; h < RC; h++) {
+        const cplx<T> v = l[h][f];
+        sr[h] += a.re * v.re - a.im * v.im;
+        si[h] += a.re * v.im + a.im * v.re;
+      }
     }
-    sr = wave_sum(sr);
-    si = wave_sum(si);
-    if (lane == 0) ys[(size_t)rh * N + i] = cmk<T>(sr, si);
+#pragma unroll
+    for (int h = 0; h < RC; h++) {
+      if (h0 + h >= nrhs) break;
+      const T vr = wave_sum(sr[h]), vi = wave_sum(si[h]);
+      if (lane == 0)
+        y[(size_t)(h0 + h) * N + to] = make_double2((double)vr, (double)vi);
+    }
   }
 }
 
 // Transposed near field + transposed P2M: one block per leaf box c, one
-// wavefront per (element j of c, right-hand side) job.  Column j of A lies in
-// the blocks of the boxes b of c's neighbourhood (neighbourhoods are
-// symmetric), at the columns where b's block lists box c.  Far part:
+// wavefront per (element j of c, right-hand side) job, the result in the
+// caller's order.  Column j of A lies in the blocks of the boxes b of c's
+// neighbourhood (neighbourhoods are symmetric), at the columns where b's
+// block lists box c: found by eight threads a box (by one thread for all,
+// 29 us at 5,120 triangles, 19 now).  Far part:
 // sum_f B[j][f] (-1)^n M'[c][r][f], the transposed pass's coefficients being
 // kept multiplied by (-1)^n.
-template <typename T>
+template <typename T, int RC>
 __global__ void __launch_bounds__(256)
     k_near_t(const int *__restrict__ bstart, const int *__restrict__ nstart,
              const int *__restrict__ nbox, const int *__restrict__ ncols,
              const unsigned long long *__restrict__ boff,
              const cplx<T> *__restrict__ A, const cplx<T> *__restrict__ B,
              const cplx<T> *__restrict__ Mc, const cplx<T> *__restrict__ xs,
-             cplx<T> *__restrict__ ys, int N, int ps, int nrhs, int parts) {
-  __shared__ int nb_first[27], nb_row0[28], nb_col[27], nb_nc[27];
-  __shared__ unsigned long long nb_off[27];
-  __shared__ int nnb;
-  const int c = blockIdx.x;
+             const int *__restrict__ perm, double2 *__restrict__ y, int N, int ps, int nrhs,
+             int parts) {
+  __shared__ int nb_first[32], nb_row0[33], nb_col[32], nb_nc[32];
+  __shared__ unsigned long long nb_off[32];
+  const int c = xcd_block(blockIdx.x, gridDim.x);
   const int e0 = bstart[c], nj = bstart[c + 1] - e0;
-  if (threadIdx.x == 0) {
-    int q0 = nstart[c], q1 = nstart[c + 1], acc = 0, k = 0;
-    for (int q = q0; q < q1 && k < 27; q++) {
-      int b = nbox[q], co = 0, found = 0;
-      for (int qq = nstart[b]; qq < nstart[b + 1]; qq++) {
-        int o = nbox[qq];
-        if (o == c) {
-          found = 1;
-          break;
+  const int q0 = nstart[c], nnb = nstart[c + 1] - q0;
+  {
+    const int q = threadIdx.x >> 3, sub = threadIdx.x & 7;
+    int cnt[4] = {0, 0, 0, 0}, pos = 32, b = -1;
+    if (q < nnb) {
+      b = nbox[q0 + q];
+      const int s0 = nstart[b], s1 = nstart[b + 1];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int s = s0 + sub + 8 * i;
+        if (s < s1) {
+          const int o = nbox[s];
+          cnt[i] = bstart[o + 1] - bstart[o];
+          if (o == c) pos = sub + 8 * i;
         }
-        co += bstart[o + 1] - bstart[o];
       }
-      if (!found) continue; /* not reached: neighbourhoods are symmetric */
-      nb_first[k] = bstart[b];
-      nb_row0[k] = acc;
-      nb_col[k] = co;
-      nb_nc[k] = ncols[b];
-      nb_off[k] = boff[b];
-      acc += bstart[b + 1] - bstart[b];
-      k++;
     }
-    nb_row0[k] = acc;
-    nnb = k;
+    for (int o = 1; o < 8; o <<= 1) pos = min(pos, __shfl_xor(pos, o, 64));
+    int co = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) co += sub + 8 * i < pos ? cnt[i] : 0;
+    for (int o = 1; o < 8; o <<= 1) co += __shfl_xor(co, o, 64);
+    if (sub == 0) {
+      nb_row0[q + 1] = 0;
+      if (b >= 0 && pos < 32) {
+        nb_first[q] = bstart[b];
+        nb_row0[q + 1] = bstart[b + 1] - bstart[b];
+        nb_col[q] = co;
+        nb_nc[q] = ncols[b];
+        nb_off[q] = boff[b];
+      }
+    }
   }
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int R = nb_row0[nnb];
-  for (int job = wave; job < nj * nrhs; job += (blockDim.x >> 6)) {
-    const int jj = job % nj, rh = job / nj, j = e0 + jj;
-    T sr = 0, si = 0;
-    const cplx<T> *x = xs + (size_t)rh * N;
+  if (wave == 0) {
+    int pre = lane < 32 ? nb_row0[lane + 1] : 0;
+    for (int o = 1; o < 32; o <<= 1) {
+      const int v = __shfl_up(pre, o, 64);
+      if (lane >= o) pre += v;
+    }
+    if (lane < 32) nb_row0[lane + 1] = pre;
+    if (lane == 0) nb_row0[0] = 0;
+  }
+  __syncthreads();
+  const int R = nb_row0[nnb], ng = (nrhs + RC - 1) / RC;
+  for (int job = wave; job < nj * ng; job += (blockDim.x >> 6)) {
+    const int jj = job % nj, h0 = job / nj * RC, j = e0 + jj, to = perm[j];
+    T sr[RC], si[RC];
+    const cplx<T> *x[RC], *l[RC];
+#pragma unroll
+    for (int h = 0; h < RC; h++) {
+      const int rh = min(h0 + h, nrhs - 1);
+      sr[h] = si[h] = 0;
+      x[h] = xs + (size_t)rh * N;
+      l[h] = Mc + ((size_t)c * nrhs + rh) * ps;
+    }
     for (int u = (parts & 1) ? lane : R; u < R; u += 64) {
       int q = 0;
       while (q + 1 < nnb && nb_row0[q + 1] <= u) q++;
       const int r = u - nb_row0[q];
-      cplx<T> a = A[nb_off[q] + (size_t)r * nb_nc[q] + nb_col[q] + jj];
-      cplx<T> v = x[nb_first[q] + r];
-      sr += a.re * v.re - a.im * v.im;
-      si += a.re * v.im + a.im * v.re;
+      const cplx<T> a = A[nb_off[q] + (size_t)r * nb_nc[q] + nb_col[q] + jj];
+      const int i = nb_first[q] + r;
+#pragma unroll
+      for (int h = 0; h < RC; h++) {
+        const cplx<T> v = x[h][i];
+        sr[h] += a.re * v.re - a.im * v.im;
+        si[h] += a.re * v.im + a.im * v.re;
+      }
     }
     const cplx<T> *e = B + (size_t)j * ps;
-    const cplx<T> *l = Mc + ((size_t)c * nrhs + rh) * ps;
+#pragma unroll 4
     for (int f = (parts & 2) ? lane : ps; f < ps; f += 64) {
-      cplx<T> a = e[f], v = l[f];
-      T g = (isqrt_fix(f) & 1) ? T(-1) : T(1);
-      sr += g * (a.re * v.re - a.im * v.im);
-      si += g * (a.re * v.im + a.im * v.re);
+      cplx<T> a = e[f];
+      if (isqrt_fix(f) & 1) a = cmk<T>(-a.re, -a.im);
+#pragma unroll
+      for (int h = 0; h < RC; h++) {
+        const cplx<T> v = l[h][f];
+        sr[h] += a.re * v.re - a.im * v.im;
+        si[h] += a.re * v.im + a.im * v.re;
+      }
     }
-    sr = wave_sum(sr);
-    si = wave_sum(si);
-    if (lane == 0) ys[(size_t)rh * N + j] = cmk<T>(sr, si);
+#pragma unroll
+    for (int h = 0; h < RC; h++) {
+      if (h0 + h >= nrhs) break;
+      const T vr = wave_sum(sr[h]), vi = wave_sum(si[h]);
+      if (lane == 0)
+        y[(size_t)(h0 + h) * N + to] = make_double2((double)vr, (double)vi);
+    }
   }
 }
 
@@ -347,7 +435,7 @@ extern "C" int fmbh_near_dsigma(fmb_plan *pl, int op, void *out, void *stream) {
   return launch_near(pl, op, NULL, out, 1, stream);
 }
 
-extern "C" int fmbh_l2p_near(const fmb_plan *pl, int op, int nrhs, int parts,
+extern "C" int fmbh_l2p_near(const fmb_plan *pl, int op, fmb_c64 *y, int nrhs, int parts,
                              void *stream) {
   const fmb_tree *t = pl->tree;
   hipStream_t st = (hipStream_t)stream;
@@ -356,27 +444,27 @@ extern "C" int fmbh_l2p_near(const fmb_plan *pl, int op, int nrhs, int parts,
   size_t lds = sizeof(int) * (size_t)(pl->near_max_ncol > 0 ? pl->near_max_ncol : 1);
   const unsigned long long *off = (const unsigned long long *)pl->d_near_off;
   if (o->prec == FMB_FP64)
-    hipLaunchKernelGGL(k_l2p_near<double>, dim3(nb), dim3(256), lds, st,
+    hipLaunchKernelGGL((nrhs == 1 ? k_l2p_near<double, 1> : nrhs == 2 ? k_l2p_near<double, 2> : k_l2p_near<double, 4>), dim3(nb), dim3(256), lds, st,
                        t->d_box_start, t->d_near_start, t->d_near_box,
                        pl->d_near_ncol, off, (const cplx<double> *)o->d_near,
                        (const cplx<double> *)o->d_L2P,
                        (const cplx<double> *)o->d_L[L],
-                       (const cplx<double> *)o->d_xs, (cplx<double> *)o->d_ys,
+                       (const cplx<double> *)o->d_xs, t->d_perm, (double2 *)y,
                        t->nelem, pL * pL, nrhs, parts);
   else
-    hipLaunchKernelGGL(k_l2p_near<float>, dim3(nb), dim3(256), lds, st,
+    hipLaunchKernelGGL((nrhs == 1 ? k_l2p_near<float, 1> : nrhs == 2 ? k_l2p_near<float, 2> : k_l2p_near<float, 4>), dim3(nb), dim3(256), lds, st,
                        t->d_box_start, t->d_near_start, t->d_near_box,
                        pl->d_near_ncol, off, (const cplx<float> *)o->d_near,
                        (const cplx<float> *)o->d_L2P,
                        (const cplx<float> *)o->d_L[L],
-                       (const cplx<float> *)o->d_xs, (cplx<float> *)o->d_ys,
+                       (const cplx<float> *)o->d_xs, t->d_perm, (double2 *)y,
                        t->nelem, pL * pL, nrhs, parts);
   FMB_LAUNCH_CHECK();
   return FMB_OK;
 }
 
-extern "C" int fmbh_near_t(const fmb_plan *pl, int op, const void *near,
-                           const void *basis, int nrhs, int parts, void *stream) {
+extern "C" int fmbh_near_t(const fmb_plan *pl, int op, const void *near, const void *basis,
+                           fmb_c64 *y, int nrhs, int parts, void *stream) {
   const fmb_tree *t = pl->tree;
   hipStream_t st = (hipStream_t)stream;
   int L = t->lmax, nb = t->nbox[L], pL = pl->p[L];
@@ -385,18 +473,18 @@ extern "C" int fmbh_near_t(const fmb_plan *pl, int op, const void *near,
   const void *B = basis ? basis : o->d_P2M;
   const unsigned long long *off = (const unsigned long long *)pl->d_near_off;
   if (o->prec == FMB_FP64)
-    hipLaunchKernelGGL(k_near_t<double>, dim3(nb), dim3(256), 0, st,
+    hipLaunchKernelGGL((nrhs == 1 ? k_near_t<double, 1> : nrhs == 2 ? k_near_t<double, 2> : k_near_t<double, 4>), dim3(nb), dim3(256), 0, st,
                        t->d_box_start, t->d_near_start, t->d_near_box,
                        pl->d_near_ncol, off, (const cplx<double> *)A,
                        (const cplx<double> *)B, (const cplx<double> *)o->d_M[L],
-                       (const cplx<double> *)o->d_xs, (cplx<double> *)o->d_ys,
+                       (const cplx<double> *)o->d_xs, t->d_perm, (double2 *)y,
                        t->nelem, pL * pL, nrhs, parts);
   else
-    hipLaunchKernelGGL(k_near_t<float>, dim3(nb), dim3(256), 0, st,
+    hipLaunchKernelGGL((nrhs == 1 ? k_near_t<float, 1> : nrhs == 2 ? k_near_t<float, 2> : k_near_t<float, 4>), dim3(nb), dim3(256), 0, st,
                        t->d_box_start, t->d_near_start, t->d_near_box,
                        pl->d_near_ncol, off, (const cplx<float> *)A,
                        (const cplx<float> *)B, (const cplx<float> *)o->d_M[L],
-                       (const cplx<float> *)o->d_xs, (cplx<float> *)o->d_ys,
+                       (const cplx<float> *)o->d_xs, t->d_perm, (double2 *)y,
                        t->nelem, pL * pL, nrhs, parts);
   FMB_LAUNCH_CHECK();
   return FMB_OK;

@@ -113,8 +113,7 @@ static int opset_alloc(fmb_plan *pl, fmb_opset *o) {
   pl->bytes += nz;
   size_t vz = (size_t)N * nr * o->csz;
   if ((rc = fmbh_malloc(&o->d_xs, vz))) return rc;
-  if ((rc = fmbh_malloc(&o->d_ys, vz))) return rc;
-  pl->bytes += 2 * vz;
+  pl->bytes += vz;
   return FMB_OK;
 }
 
@@ -131,9 +130,8 @@ static void opset_free_freq(fmb_opset *o) {
   fmbh_free(o->d_L2P);
   fmbh_free(o->d_near);
   fmbh_free(o->d_xs);
-  fmbh_free(o->d_ys);
   fmbh_free(o->d_gws);
-  o->d_P2M = o->d_L2P = o->d_near = o->d_xs = o->d_ys = o->d_gws = NULL;
+  o->d_P2M = o->d_L2P = o->d_near = o->d_xs = o->d_gws = NULL;
   o->gws_grid = 0;
   o->gws_bytes = 0;
   o->gws_slot = 0;
@@ -345,8 +343,11 @@ static int plan_geometry(fmb_plan *pl, void *stream) {
   free(e);
   if (rc) return rc;
   /* the matrix-core L2L adds with atomics (the VALU one does not, so it
-   * cannot share L_l with that level's M2L) */
-  if (!prm->serial_levels && L >= 5 && prm->rcr_path != FMB_RCR_VALU) {
+   * cannot share L_l with that level's M2L).  At depth 3 the waits between
+   * the streams cost more than they hide (1,280 triangles: 136 us, 110 on one
+   * stream); at depth 4 they break even (an adjoint gradient at 5,120
+   * triangles 34.0 ms, 34.2 on one) */
+  if (!prm->serial_levels && L >= 4 && prm->rcr_path != FMB_RCR_VALU) {
     if ((rc = fmbh_stream_create(&pl->aux))) return rc;
     if ((rc = fmbh_event_create_sync(&pl->ev_up))) return rc;
     if ((rc = fmbh_event_create_sync(&pl->ev_aux))) return rc;
@@ -603,6 +604,71 @@ int fmb_last_timing(const fmb_plan *pl, double *phase7, double *m2l16) {
   return FMB_OK;
 }
 
+/* The translations of a pass between its first coefficients at the finest
+ * level L and its last: up the tree (M2M; transposed L2L^T), across each level
+ * (M2L; M2L^T) and down (L2L; M2M^T).  ev: phase events of a timed forward
+ * pass, or NULL.
+ *
+ * With a second stream the translations across L, the longest launch, start at
+ * once, since they need nothing of the other levels; the levels L-2 and L-1
+ * follow on the same stream.  The other stream carries the chains of small
+ * launches up and down and the coarser levels: translations down into l read
+ * level l - 1 complete, and add into l with atomics beside those across l.
+ * Against the finest level last and alone: 81,920 triangles FP32 3.31 -> 3.11
+ * ms, 20,480 FP64 1.95 -> 1.85; transposed, which had one stream, 20,480 FP32
+ * with three right-hand sides 3.68 -> 3.42.
+ * Inside a graph capture the levels stay on the capturing stream (a second
+ * fork there is not used, see fmb_gmres_batch). */
+static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev, void *stream) {
+  const int L = pl->tree->lmax, up = trans ? 2 : 1, down = trans ? 1 : 2;
+  int (*run)(const fmb_plan *, int, int, int, int, void *) = trans ? fmbx_rcr_run_t : fmbx_rcr_run;
+  int rc = FMB_OK;
+#define ACROSS(l, st)                                                                    \
+  do {                                                                                   \
+    if (ev) fmbh_event_record(ev[4 + 2 * (l)], st);                                      \
+    if ((rc = run(pl, op, 0, l, nrhs, st))) return rc;                                   \
+    if (ev) fmbh_event_record(ev[5 + 2 * (l)], st);                                      \
+  } while (0)
+  const int split = pl->aux && !pl->capturing;
+  void *aux = pl->aux;
+  if (split) {
+    if ((rc = fmbh_event_record(pl->ev_up, stream))) return rc;
+    if ((rc = fmbh_stream_wait(aux, pl->ev_up))) return rc;
+  }
+  /* (a timed pass keeps the chain up, a phase of its own, on the caller's
+   * stream) */
+  void *su = split && !ev ? aux : stream;
+  for (int l = L; l > 2; l--)
+    if ((rc = run(pl, op, up, l, nrhs, su))) return rc;
+  if (ev) fmbh_event_record(ev[2], stream);
+  if (!split) {
+    for (int l = 2; l <= L; l++) {
+      ACROSS(l, stream);
+      if (l > 2 && (rc = run(pl, op, down, l, nrhs, stream))) return rc;
+    }
+    return FMB_OK;
+  }
+  const int ls = L - 2 > 2 ? L - 2 : 2;
+  if ((rc = fmbh_event_record(pl->ev_m2l[L], su))) return rc;
+  ACROSS(L, stream);
+  if ((rc = fmbh_stream_wait(su == aux ? stream : aux, pl->ev_m2l[L]))) return rc;
+  for (int l = ls; l < L; l++) {
+    ACROSS(l, stream);
+    if ((rc = fmbh_event_record(pl->ev_m2l[l], stream))) return rc;
+  }
+  for (int l = 2; l < L; l++) {
+    if (l < ls) ACROSS(l, aux);
+    if (l > 2) {
+      if (l - 1 >= ls && (rc = fmbh_stream_wait(aux, pl->ev_m2l[l - 1]))) return rc;
+      if ((rc = run(pl, op, down, l, nrhs, aux))) return rc;
+    }
+  }
+#undef ACROSS
+  if ((rc = fmbh_event_record(pl->ev_aux, aux))) return rc;
+  if ((rc = fmbh_stream_wait(stream, pl->ev_aux))) return rc;
+  return L > 2 ? run(pl, op, down, L, nrhs, stream) : FMB_OK;
+}
+
 /* phase events: 0 start, 1 after gather+P2M, 2 after M2M, 3 after M2L/L2L,
  * 4 after L2P+near */
 int fmb_matvec(fmb_plan *pl, int prec, const fmb_c64 *x, fmb_c64 *y, int nrhs,
@@ -618,7 +684,6 @@ int fmb_matvec_parts(fmb_plan *pl, int prec, int parts, const fmb_c64 *x,
   if (!pl->ready) return fmb_set_error(FMB_ERR_ARG, "fmb_matvec: plan holds no operator");
   int op = (prec == FMB_MIXED && pl->nops == 2) ? 1 : 0;
   const fmb_tree *t = pl->tree;
-  fmb_opset *o = &pl->ops[op];
   int rc, L = t->lmax;
   void *ev[4 + 2 * FMB_MAXLEV] = {0};
   int tm = pl->timing;
@@ -626,66 +691,11 @@ int fmb_matvec_parts(fmb_plan *pl, int prec, int parts, const fmb_c64 *x,
     for (int i = 0; i < 4 + 2 * FMB_MAXLEV; i++)
       if ((rc = fmbh_event_create(&ev[i]))) return rc;
   if (tm) fmbh_event_record(ev[0], stream);
-  if ((rc = fmbh_gather(pl, op, x, nrhs, stream))) goto out;
-  for (int l = 2; l <= L; l++) {
-    size_t bytes = (size_t)t->nbox[l] * nrhs * pl->p[l] * pl->p[l] * o->csz;
-    if ((rc = fmbh_memset(o->d_L[l], 0, bytes, stream))) goto out;
-    /* parents receive the M2M translations of their children as sums */
-    if (l < L && (rc = fmbh_memset(o->d_M[l], 0, bytes, stream))) goto out;
-  }
-  if ((rc = fmbh_p2m(pl, op, nrhs, stream))) goto out;
+  if ((rc = fmbh_begin(pl, op, FMBH_BEGIN_FWD, x, nrhs, stream))) goto out;
   if (tm) fmbh_event_record(ev[1], stream);
-  for (int l = L; l > 2; l--)
-    if ((rc = fmbx_rcr_run(pl, op, 1, l, nrhs, stream))) goto out;
-  if (tm) fmbh_event_record(ev[2], stream);
-  /* inside a graph capture the levels stay on the capturing stream (see
-   * fmb_gmres_batch: a second fork there is not used) */
-  if (!pl->aux || pl->capturing) {
-    for (int l = 2; l <= L; l++) {
-      if (tm) fmbh_event_record(ev[4 + 2 * l], stream);
-      if ((rc = fmbx_rcr_run(pl, op, 0, l, nrhs, stream))) goto out;
-      if (tm) fmbh_event_record(ev[5 + 2 * l], stream);
-      if (l > 2 && (rc = fmbx_rcr_run(pl, op, 2, l, nrhs, stream))) goto out;
-    }
-  } else {
-    /* M2L levels need only the upward pass; L2L into level l reads L_{l-1}
-     * complete (its M2L and L2L), and adds into L_l with atomics beside
-     * that level's M2L.  The caller's stream runs the M2L levels L-2 and
-     * L-1; the second stream runs the coarser M2L levels and the L2L chain
-     * up to level L-1, waiting for a fine level's M2L before the L2L that
-     * reads it.  The finest M2L (the longest launch) then runs alone on the
-     * caller's stream, followed by the last L2L. */
-    const int ls = L - 2;
-    void *aux = pl->aux;
-    if ((rc = fmbh_event_record(pl->ev_up, stream))) goto out;
-    if ((rc = fmbh_stream_wait(aux, pl->ev_up))) goto out;
-    for (int l = ls; l < L; l++) {
-      if (tm) fmbh_event_record(ev[4 + 2 * l], stream);
-      if ((rc = fmbx_rcr_run(pl, op, 0, l, nrhs, stream))) goto out;
-      if (tm) fmbh_event_record(ev[5 + 2 * l], stream);
-      if ((rc = fmbh_event_record(pl->ev_m2l[l], stream))) goto out;
-    }
-    for (int l = 2; l < L; l++) {
-      if (l < ls) {
-        if (tm) fmbh_event_record(ev[4 + 2 * l], aux);
-        if ((rc = fmbx_rcr_run(pl, op, 0, l, nrhs, aux))) goto out;
-        if (tm) fmbh_event_record(ev[5 + 2 * l], aux);
-      }
-      if (l > 2) {
-        if (l - 1 >= ls && (rc = fmbh_stream_wait(aux, pl->ev_m2l[l - 1]))) goto out;
-        if ((rc = fmbx_rcr_run(pl, op, 2, l, nrhs, aux))) goto out;
-      }
-    }
-    if ((rc = fmbh_event_record(pl->ev_aux, aux))) goto out;
-    if ((rc = fmbh_stream_wait(stream, pl->ev_aux))) goto out;
-    if (tm) fmbh_event_record(ev[4 + 2 * L], stream);
-    if ((rc = fmbx_rcr_run(pl, op, 0, L, nrhs, stream))) goto out;
-    if (tm) fmbh_event_record(ev[5 + 2 * L], stream);
-    if ((rc = fmbx_rcr_run(pl, op, 2, L, nrhs, stream))) goto out;
-  }
+  if ((rc = translate_levels(pl, op, 0, nrhs, tm ? ev : NULL, stream))) goto out;
   if (tm) fmbh_event_record(ev[3], stream);
-  if ((rc = fmbh_l2p_near(pl, op, nrhs, parts, stream))) goto out;
-  if ((rc = fmbh_scatter(pl, op, y, nrhs, stream))) goto out;
+  if ((rc = fmbh_l2p_near(pl, op, y, nrhs, parts, stream))) goto out;
   if (tm) {
     void *e4;
     fmbh_event_create(&e4);
@@ -720,26 +730,13 @@ out:
 int fmbx_matvec_t(fmb_plan *pl, int op, int parts, const void *near,
                   const void *basis, const fmb_c64 *x, fmb_c64 *y, int nrhs,
                   void *stream) {
-  const fmb_tree *t = pl->tree;
-  fmb_opset *o = &pl->ops[op];
-  int rc, L = t->lmax;
-  if ((rc = fmbh_gather(pl, op, x, nrhs, stream))) return rc;
+  int rc;
+  if ((rc = fmbh_begin(pl, op, (parts & 2) ? FMBH_BEGIN_T : FMBH_BEGIN_NEAR, x, nrhs, stream)))
+    return rc;
   if (parts & 2) {
-    for (int l = 2; l <= L; l++) {
-      size_t bytes = (size_t)t->nbox[l] * nrhs * pl->p[l] * pl->p[l] * o->csz;
-      if (l < L && (rc = fmbh_memset(o->d_L[l], 0, bytes, stream))) return rc;
-      if ((rc = fmbh_memset(o->d_M[l], 0, bytes, stream))) return rc;
-    }
-    if ((rc = fmbh_l2p_t(pl, op, nrhs, stream))) return rc;
-    for (int l = L; l > 2; l--)
-      if ((rc = fmbx_rcr_run_t(pl, op, 2, l, nrhs, stream))) return rc;
-    for (int l = 2; l <= L; l++) {
-      if (l > 2 && (rc = fmbx_rcr_run_t(pl, op, 1, l, nrhs, stream))) return rc;
-      if ((rc = fmbx_rcr_run_t(pl, op, 0, l, nrhs, stream))) return rc;
-    }
+    if ((rc = translate_levels(pl, op, 1, nrhs, NULL, stream))) return rc;
   }
-  if ((rc = fmbh_near_t(pl, op, near, basis, nrhs, parts, stream))) return rc;
-  return fmbh_scatter(pl, op, y, nrhs, stream);
+  return fmbh_near_t(pl, op, near, basis, y, nrhs, parts, stream);
 }
 
 int fmb_matvec_transpose(fmb_plan *pl, int prec, int parts, const fmb_c64 *x,
@@ -799,7 +796,6 @@ int fmb_field_eval_fmm(fmb_plan *pl, const fmb_c64 *x, int nrhs,
       return fmb_set_error(FMB_ERR_ARG, "fmb_field_eval_fmm: point %zu is not finite", i / 3);
   const fmb_tree *t = pl->tree;
   const int L = t->lmax, N = t->nelem;
-  fmb_opset *o = &pl->ops[0];
   /* points in Morton order on a grid of 1/1024 of the cube over three cube
    * widths (points beyond clamp to its faces), so that the workgroups of
    * the box-major levels take compact groups of points */
@@ -841,11 +837,7 @@ int fmb_field_eval_fmm(fmb_plan *pl, const fmb_c64 *x, int nrhs,
   for (int c0 = 0; c0 < nrhs && !rc; c0 += pl->nrhs_max) {
     const int nc = nrhs - c0 < pl->nrhs_max ? nrhs - c0 : pl->nrhs_max;
     const fmb_c64 *xc = x + (size_t)c0 * N;
-    if ((rc = fmbh_gather(pl, 0, xc, nc, stream))) break;
-    for (int l = 2; l < L && !rc; l++)
-      rc = fmbh_memset(o->d_M[l], 0, (size_t)t->nbox[l] * nc * pl->p[l] * pl->p[l] * o->csz,
-                       stream);
-    if (!rc) rc = fmbh_p2m(pl, 0, nc, stream);
+    rc = fmbh_begin(pl, 0, FMBH_BEGIN_UP, xc, nc, stream);
     for (int l = L; l > 2 && !rc; l--) rc = fmbx_rcr_run(pl, 0, 1, l, nc, stream);
     if (!rc)
       rc = fmbh_field_tree(pl, 0, xc, nc, d_pts, d_qperm, npts,

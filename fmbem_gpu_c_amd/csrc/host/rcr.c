@@ -1286,7 +1286,7 @@ int fmbx_rcr_run_t(const fmb_plan *pl, int op, int kind, int l, int nrhs,
   j.pout = tb->pout;
   j.hlen = tb->hlen;
   j.xcd = kind == 0 && tb->tiled && j.mode == FMBH_RCR_LDS;
-  j.gws = o->d_gws;
+  j.gws = (pl->aux && stream == pl->aux) ? (char *)o->d_gws + o->gws_slot : o->d_gws;
   j.gws_grid = o->gws_grid;
   j.phase = o->d_phase_c[kind];
   j.pstride = pl->Pmax;

@@ -187,13 +187,14 @@ typedef struct fmb_plan_params {
                                 matrix-core translation at plan creation
                                 and keep the fastest (fmb_plan_tile_shape)  */
   int serial_levels;         /* 1: M2L levels one after another on the
-                                caller's stream; 0: the coarse levels and
-                                the L2L chain on a second stream, beside
-                                the M2L of levels L-2 and L-1 (the finest
-                                M2L then runs alone)                        */
+                                caller's stream; 0: trees of depth 4 and
+                                more run the M2M and L2L chains and the
+                                coarse levels on a second stream, beside
+                                the M2L of the finest levels                */
   int waves;                 /* waves per workgroup of the matrix-core
                                 translations in the fixed tile-shape rule:
-                                4 or 8 (0: 4); autotune overrides it        */
+                                4 or 8 (0: by the order and the launch's
+                                workgroups); autotune overrides it          */
   int split_bf16;            /* FMB_MIXED plans: 1 runs the rotations of the
                                 FP32 pass's LDS-mode translations in
                                 split-BF16 (hi + lo bf16 operands, three
