@@ -19,6 +19,8 @@
 // panels next to the point are summed directly with the rule above.  The
 // coarse levels, whose orders are high, run box-major over chunks of points
 // in Morton order; the finer levels per point.
+#include <hipcub/hipcub.hpp>
+
 #include "fmb_device.h"
 
 namespace {
@@ -176,7 +178,6 @@ constexpr int kCand = 256; // candidates of one level: <= 64 at level 2, <= 27*8
 constexpr int kFieldChunk = 32768; // points per pass of the box-major sums
 constexpr int kBoxMinP = 24;        // box-major from level 2 down while orders reach this
 constexpr int kBoxMaxBoxes = 32768; // and the level has at most this many boxes
-constexpr int kBoxWG = 64;          // points per box-major workgroup
 
 struct TreeLevels {
   int L;
@@ -437,31 +438,37 @@ __global__ void __launch_bounds__(kT)
   }
 }
 
-// The expansions of level l box-major: workgroup w evaluates box
-// w / nchunk of level l at the WG points of chunk w % nchunk (the points
-// come sorted in Morton order, so a chunk is compact), one point per lane,
-// for the points the traversal of k_field_tree meets the box at: the box is
-// well separated from the point at level l (indices 2 or more apart) and
-// its parent is next to the point at level l - 1 (no condition at level 2;
-// the parent's ancestors then lie next to the point too).  Column m of the
-// box's coefficients (n = m .. p-1, orders +m and -m, every right-hand side)
-// is staged in LDS by the whole workgroup and read by every lane at one
-// address; per lane the recurrences of k_field_tree run up that column,
-// h_n restarted from n = 0.  boxsum[r * npts + q] += -sum w_n Mt_n^m
-// S_n^m(y_q - c) for right-hand side r0 + r, by FP64 atomic adds (the order
-// of the boxes' contributions is not fixed).  Dynamic LDS: 2 p complex
-// values per right-hand side of the launch.
-template <int WG>
-__global__ void __launch_bounds__(WG)
-    k_field_box(TreeLevels tl, int l, const double2 *__restrict__ leg,
-                const double *__restrict__ dg, const double *__restrict__ pts, int npts,
-                int nchunk, double k, int nrhs, int r0, double2 *__restrict__ boxsum) {
-  extern __shared__ double2 col[];  // [rr][sign][n - m]
-  const int b = blockIdx.x / nchunk, tid = threadIdx.x;
-  const int q = (blockIdx.x % nchunk) * WG + tid;
+// The expansions of level l box-major: wavefront w evaluates box w / nchunk of
+// level l at the 64 points of chunk w % nchunk (the points come sorted in
+// Morton order, so a chunk is compact), one point per lane, for the points the
+// traversal of k_field_tree meets the box at: the box is well separated from
+// the point at level l (indices 2 or more apart) and its parent is next to the
+// point at level l - 1 (no condition at level 2; the parent's ancestors then
+// lie next to the point too).  boxsum[r * npts + q] += -sum w_n Mt_n^m
+// S_n^m(y_q - c) for right-hand sides r0 + r, r < nr <= NR, by FP64 atomic adds
+// (the order of the boxes' contributions is not fixed).
+//
+// Bound by FP64 issue.  A lane runs CB columns m0 .. of S_n^m up in n beside
+// each other, which share h_n and its weight and hide each other's chains: 13
+// operations a coefficient pair and 5 a step; the azimuth factors, the same
+// down a column, enter at its end.  The coefficients and the recurrence's
+// factors are the same for all lanes and come through scalar loads: from LDS
+// they would take as long as the arithmetic.  The state of h_n where the next
+// columns start is kept on the way.  Levels 2 to 4 of 81,920 triangles (orders
+// 47, 33, 25) at 16,384 points take 1.36 ms; 3.76 by single columns from LDS
+// with h_n run up from n = 0 for each.
+template <int CB, int NR>
+__global__ void __launch_bounds__(64)
+    k_field_box(const int *__restrict__ keys, int l, int p, double D, double p0, double p1,
+                double p2, const double *__restrict__ wsc, const double2 *__restrict__ M,
+                const double2 *__restrict__ leg, const double *__restrict__ dg,
+                const double *__restrict__ pts, int npts, int nchunk, double k, int nrhs, int r0,
+                int nr, double2 *__restrict__ boxsum) {
+  const int b = blockIdx.x / nchunk, q = (blockIdx.x % nchunk) * 64 + threadIdx.x;
   int tx, tyy, tz;
-  deinterleave3(tl.keys[l][b], l, tx, tyy, tz);
+  deinterleave3(keys[b], l, tx, tyy, tz);
   const double sc = ldexp(1.0, l);
+  const double pmin[3] = {p0, p1, p2};
   double y[3] = {0.0, 0.0, 0.0};
   bool active = false;
   if (q < npts) {
@@ -469,103 +476,177 @@ __global__ void __launch_bounds__(WG)
     const int t3[3] = {tx, tyy, tz};
     double sep = 0.0, psep = 0.0;
     for (int a = 0; a < 3; a++) {
-      const double u = (y[a] - tl.pmin[a]) / tl.D;
+      const double u = (y[a] - pmin[a]) / D;
       sep = fmax(sep, fabs(t3[a] - floor(u * sc)));
       psep = fmax(psep, fabs((t3[a] >> 1) - floor(u * (0.5 * sc))));
     }
     active = sep >= 2.0 && (l == 2 || psep <= 1.0);
   }
-  if (!__syncthreads_or(active)) return;
-  const double h = tl.D / sc;
-  const double v0 = y[0] - (tl.pmin[0] + (tx + 0.5) * h);
-  const double v1 = y[1] - (tl.pmin[1] + (tyy + 0.5) * h);
-  const double v2 = y[2] - (tl.pmin[2] + (tz + 0.5) * h);
+  if (!__any(active)) return;
+  const double h = D / sc;
+  const double v0 = y[0] - (p0 + (tx + 0.5) * h);
+  const double v1 = y[1] - (p1 + (tyy + 0.5) * h);
+  const double v2 = y[2] - (p2 + (tz + 0.5) * h);
   const double rho = sqrt(v0 * v0 + v1 * v1), r = sqrt(rho * rho + v2 * v2);
   // inactive lanes run the same steps on a harmless point and add nothing
   const double ct = active ? v2 / r : 1.0, st = active ? rho / r : 0.0;
   const double phi = active ? atan2(v1, v0) : 0.0;
   const double kr = active ? k * r : 1.0, ikr = 1.0 / kr;
-  double sx, cx;
+  double sx, cx, s1, c1;
   sincos(kr, &sx, &cx);
-  const double2 h0 = make_double2(sx * ikr, -cx * ikr);
-  const double2 h1 = make_double2((sx - cx * kr) * ikr * ikr, -(sx * kr + cx) * ikr * ikr);
-  const int p = tl.p[l], ps = p * p;
-  const int nr = min(kR, nrhs - r0);
-  const double *wsc = tl.scale[l];
-  const double2 *Mb = tl.M[l] + ((size_t)b * nrhs + r0) * ps;
-  double2 acc[kR];
+  sincos(phi, &s1, &c1);
+  const double2 e1 = make_double2(c1, s1);
+  // h_m and h_{m-1} of the first column: h_0 = -i e^{ix}/x, h_{-1} = e^{ix}/x
+  double2 hc0 = make_double2(sx * ikr, -cx * ikr), hp0 = make_double2(cx * ikr, sx * ikr);
+  const double2 *Mb[NR];
+  double2 acc[NR];
 #pragma unroll
-  for (int rr = 0; rr < kR; rr++) acc[rr] = make_double2(0.0, 0.0);
+  for (int i = 0; i < NR; i++) {
+    Mb[i] = M + ((size_t)b * nrhs + r0 + min(i, nr - 1)) * (size_t)(p * p);
+    acc[i] = make_double2(0.0, 0.0);
+  }
   double stm = 1.0;
-  for (int m = 0; m < p; m++) {
-    const int len = p - m;
-    __syncthreads();  // the previous column is read
-    for (int i = tid; i < 2 * nr * len; i += WG) {
-      const int j = i % len, sg = (i / len) & 1, rr = i / (2 * len);
-      const int n = m + j;
-      col[(rr * 2 + sg) * p + j] = Mb[(size_t)rr * ps + n * n + n + (sg ? -m : m)];
-    }
-    __syncthreads();
-    double P = dg[m] * stm, Pp = 0.0;
-    stm *= st;
-    double sm, cm;
-    sincos(m * phi, &sm, &cm);
-    const double2 ep = make_double2(cm, sm), em = make_double2(cm, -sm);
-    double2 hc = h0, hp = make_double2(0.0, 0.0);
-    for (int n = 0; n < m; n++) {
-      if (n == 0) {
-        hp = hc;
-        hc = h1;
-      } else {
-        const double c = (2.0 * n + 1.0) * ikr;
-        const double2 hn = make_double2(c * hc.x - hp.x, c * hc.y - hp.y);
-        hp = hc;
-        hc = hn;
-      }
-    }
-    for (int n = m; n < p; n++) {
-      if (n > m) {
-        const double2 ab = leg[n * (n + 1) / 2 + m];
-        const double Pn = ab.x * (ct * P - ab.y * Pp);
-        Pp = P;
-        P = Pn;
-      }
-      const double f = wsc[n] * P;
-      const double2 t = make_double2(f * hc.x, f * hc.y);
+  for (int m0 = 0; m0 < p; m0 += CB) {
+    double P[CB], Pp[CB], first[CB];
+    double2 ap[CB][NR], am[CB][NR];
 #pragma unroll
-      for (int rr = 0; rr < kR; rr++) {
-        if (rr < nr) {
-          double2 z = cmul2(col[(rr * 2) * p + n - m], ep);
-          if (m > 0) {
-            const double2 zm = cmul2(col[(rr * 2 + 1) * p + n - m], em);
-            z.x += zm.x;
-            z.y += zm.y;
-          }
-          const double2 tz = cmul2(t, z);
-          acc[rr].x -= tz.x;
-          acc[rr].y -= tz.y;
+    for (int c = 0; c < CB; c++) {
+      first[c] = m0 + c < p ? dg[m0 + c] * stm : 0.0;
+      stm *= st;
+      P[c] = Pp[c] = 0.0;
+#pragma unroll
+      for (int i = 0; i < NR; i++) ap[c][i] = am[c][i] = make_double2(0.0, 0.0);
+    }
+    double2 hc = hc0, hp = hp0;
+    // column c at degree n; j: n - m0 within the first CB degrees, else CB
+    auto step = [&](int n, int j) {
+      const double w = wsc[n];
+      const double2 t = make_double2(w * hc.x, w * hc.y);
+      const int f0 = n * n + n;
+#pragma unroll
+      for (int c = 0; c < CB; c++) {
+        if (c > j) break;
+        const int m = m0 + c;
+        if (c == j) {
+          P[c] = first[c];
+        } else {
+          const double2 ab = leg[n * (n + 1) / 2 + m];
+          const double Pn = ab.x * (ct * P[c] - ab.y * Pp[c]);
+          Pp[c] = P[c];
+          P[c] = Pn;
+        }
+        const double2 u = make_double2(t.x * P[c], t.y * P[c]);
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+          const double2 a = Mb[i][f0 + m], d = Mb[i][f0 - m];
+          ap[c][i].x = fma(u.x, a.x, ap[c][i].x);
+          ap[c][i].x = fma(-u.y, a.y, ap[c][i].x);
+          ap[c][i].y = fma(u.x, a.y, ap[c][i].y);
+          ap[c][i].y = fma(u.y, a.x, ap[c][i].y);
+          am[c][i].x = fma(u.x, d.x, am[c][i].x);
+          am[c][i].x = fma(-u.y, d.y, am[c][i].x);
+          am[c][i].y = fma(u.x, d.y, am[c][i].y);
+          am[c][i].y = fma(u.y, d.x, am[c][i].y);
         }
       }
-      if (n == 0) {
-        hp = hc;
-        hc = h1;
-      } else {
-        const double c = (2.0 * n + 1.0) * ikr;
-        const double2 hn = make_double2(c * hc.x - hp.x, c * hc.y - hp.y);
-        hp = hc;
-        hc = hn;
+      const double g = (2.0 * n + 1.0) * ikr;
+      const double2 hn = make_double2(g * hc.x - hp.x, g * hc.y - hp.y);
+      hp = hc;
+      hc = hn;
+    };
+#pragma unroll
+    for (int j = 0; j < CB; j++)
+      if (m0 + j < p) step(m0 + j, j);
+    hc0 = hc;
+    hp0 = hp;
+    for (int n = m0 + CB; n < p; n++) step(n, CB);
+    double sm, cm;
+    sincos(m0 * phi, &sm, &cm);
+    double2 ep = make_double2(cm, sm);
+#pragma unroll
+    for (int c = 0; c < CB; c++) {
+      if (m0 + c >= p) break;
+      const double2 em = make_double2(ep.x, -ep.y);
+#pragma unroll
+      for (int i = 0; i < NR; i++) {
+        double2 z = cmul2(ap[c][i], ep);
+        if (m0 + c > 0) {
+          const double2 zm = cmul2(am[c][i], em);
+          z.x += zm.x;
+          z.y += zm.y;
+        }
+        acc[i].x -= z.x;
+        acc[i].y -= z.y;
       }
+      ep = cmul2(ep, e1);
     }
   }
   if (active) {
 #pragma unroll
-    for (int rr = 0; rr < kR; rr++) {
-      if (rr < nr) {
-        atomicAdd(&boxsum[(size_t)rr * npts + q].x, acc[rr].x);
-        atomicAdd(&boxsum[(size_t)rr * npts + q].y, acc[rr].y);
+    for (int i = 0; i < NR; i++) {
+      if (i < nr) {
+        atomicAdd(&boxsum[(size_t)i * npts + q].x, acc[i].x);
+        atomicAdd(&boxsum[(size_t)i * npts + q].y, acc[i].y);
       }
     }
   }
+}
+
+// Order of the field points: Morton keys on a grid of 1/1024 of the cube over
+// three cube widths (points beyond clamp to its faces), so that the wavefronts
+// of the box-major levels take compact groups of points.
+__global__ void k_field_keys(const double *__restrict__ pts, int npts, double D, double p0,
+                             double p1, double p2, unsigned long long *__restrict__ key,
+                             int *__restrict__ idx) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= npts) return;
+  const double pmin[3] = {p0, p1, p2};
+  unsigned g[3];
+  for (int c = 0; c < 3; c++) {
+    const double v = floor((pts[3 * (size_t)i + c] - pmin[c]) / D * 1024.0) + 1024.0;
+    g[c] = v < 0.0 ? 0u : (v > 3071.0 ? 3071u : (unsigned)v);
+  }
+  unsigned long long z = 0;
+  for (int b = 11; b >= 0; b--)
+    z = z * 8 + 4 * ((g[0] >> b) & 1) + 2 * ((g[1] >> b) & 1) + ((g[2] >> b) & 1);
+  key[i] = z;
+  idx[i] = i;
+}
+
+__global__ void k_field_points(const double *__restrict__ pts, const int *__restrict__ idx,
+                               int npts, double *__restrict__ out) {
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < 3 * (size_t)npts) out[t] = pts[3 * (size_t)idx[t / 3] + t % 3];
+}
+
+// normalised Legendre recurrence: (a, b) per (n, m < n), then P_m^m / sin^m
+__global__ void k_field_leg(int pmax, double2 *__restrict__ leg, double *__restrict__ dg) {
+  const int f = blockIdx.x * blockDim.x + threadIdx.x;
+  if (f >= tri_idx(pmax, 0)) return;
+  int n, m;
+  tri_nm(f, n, m);
+  if (n == m) {
+    double a = 1.0 / (4.0 * M_PI);
+    for (int i = 1; i <= m; i++) a *= (2.0 * i + 1.0) / (2.0 * i);
+    dg[m] = sqrt(a);
+    return;
+  }
+  double b = 0.0;
+  if (n > m + 1)
+    b = sqrt(((double)(n - 1) * (n - 1) - (double)m * m) / (4.0 * (n - 1) * (n - 1) - 1.0));
+  leg[f] = make_double2(sqrt((4.0 * n * n - 1.0) / ((double)n * n - (double)m * m)), b);
+}
+
+template <int CB, int NR>
+void launch_box(const fmb_plan *pl, const fmb_opset *o, int l, const double2 *leg,
+                const double *dg, const double *pts, int npts, int nrhs, int r0, int nr,
+                double2 *boxsum, hipStream_t st) {
+  const fmb_tree *t = pl->tree;
+  const int nchunk = (npts + 63) / 64;
+  hipLaunchKernelGGL((k_field_box<CB, NR>), dim3(nchunk * t->nbox[l]), dim3(64), 0, st,
+                     t->d_keys[l], l, pl->p[l], t->D, t->pmin[0], t->pmin[1], t->pmin[2],
+                     pl->d_scale[l], (const double2 *)o->d_M[l], leg, dg, pts, npts, nchunk,
+                     pl->k, nrhs, r0, nr, boxsum);
 }
 
 }  // namespace
@@ -636,7 +717,7 @@ extern "C" int fmbh_field_tree(const fmb_plan *pl, int op, const fmb_c64 *x, int
   if (t->lmax < 2 || t->nbox[2] > 64)
     return fmb_set_error(FMB_ERR_ARG, "field through the tree: no level-2 boxes");
   for (int l = 2; l <= t->lmax; l++)
-    if (sizeof(double2) * 2 * kR * pl->p[l] > 64 * 1024)
+    if (pl->p[l] > 256)
       return fmb_set_error(FMB_ERR_RANGE, "field through the tree: order %d", pl->p[l]);
   TreeLevels tl = {};
   tl.L = t->lmax;
@@ -652,60 +733,35 @@ extern "C" int fmbh_field_tree(const fmb_plan *pl, int op, const fmb_c64 *x, int
     tl.M[l] = (const double2 *)o->d_M[l];
     pmax = pl->p[l] > pmax ? pl->p[l] : pmax;
   }
-  // normalised Legendre recurrence: (a, b) per (n, m), P_m^m / sin^m theta
   const int ntri = pmax * (pmax + 1) / 2;
-  double *h = (double *)malloc(sizeof(double) * (2 * (size_t)ntri + pmax));
-  if (!h) return fmb_set_error(FMB_ERR_NOMEM, "field through the tree: tables");
-  for (int n = 0; n < pmax; n++)
-    for (int m = 0; m <= n; m++) {
-      double a = 0.0, b = 0.0;
-      if (n == m + 1) {
-        a = sqrt(2.0 * m + 3.0);
-      } else if (n > m + 1) {
-        a = sqrt((4.0 * n * n - 1.0) / ((double)n * n - (double)m * m));
-        b = sqrt(((double)(n - 1) * (n - 1) - (double)m * m) /
-                 (4.0 * (n - 1) * (n - 1) - 1.0));
-      }
-      h[2 * (n * (n + 1) / 2 + m)] = a;
-      h[2 * (n * (n + 1) / 2 + m) + 1] = b;
-    }
-  double d = 1.0 / sqrt(4.0 * M_PI);
-  for (int m = 0; m < pmax; m++) {
-    if (m > 0) d *= sqrt((2.0 * m + 1.0) / (2.0 * m));
-    h[2 * ntri + m] = d;
-  }
   double *d_tab = NULL;
   int rc = fmbh_malloc((void **)&d_tab, sizeof(double) * (2 * (size_t)ntri + pmax));
-  if (!rc && hipMemcpy(d_tab, h, sizeof(double) * (2 * (size_t)ntri + pmax),
-                       hipMemcpyHostToDevice) != hipSuccess)
-    rc = fmb_set_error(FMB_ERR_HIP, "field through the tree: table copy");
-  free(h);
   if (rc) return rc;
+  double2 *leg = (double2 *)d_tab;
+  double *dg = d_tab + 2 * ntri;
+  hipLaunchKernelGGL(k_field_leg, dim3((ntri + 63) / 64), dim3(64), 0, st, pmax, leg, dg);
   // levels 2 .. lb box-major (orders of kBoxMinP and above), the rest per
   // point; the box-major sums of one chunk of points: [kR][chunk]
   int lb = 2;
   while (lb < t->lmax && pl->p[lb + 1] >= kBoxMinP && t->nbox[lb + 1] <= kBoxMaxBoxes) lb++;
-  int pb = 0;
-  for (int l = 2; l <= lb; l++) pb = pl->p[l] > pb ? pl->p[l] : pb;
   const int chunk = npts < kFieldChunk ? npts : kFieldChunk;
   double2 *d_box = NULL;
   if (!rc) rc = fmbh_malloc((void **)&d_box, sizeof(double2) * (size_t)kR * chunk);
   for (int q0 = 0; q0 < npts && !rc; q0 += chunk) {
     const int nq0 = npts - q0 < chunk ? npts - q0 : chunk;
-    const int nchunk = (nq0 + kBoxWG - 1) / kBoxWG;
     for (int r0 = 0; r0 < nrhs && !rc; r0 += kR) {
       const int nr = nrhs - r0 < kR ? nrhs - r0 : kR;
-      if (hipMemsetAsync(d_box, 0, sizeof(double2) * (size_t)kR * nq0, st) != hipSuccess) {
-        rc = fmb_set_error(FMB_ERR_HIP, "field through the tree: clear");
-        break;
-      }
+      if ((rc = fmbh_memset(d_box, 0, sizeof(double2) * (size_t)kR * nq0, stream))) break;
+      // one column group and several right-hand sides share the registers
       for (int l = 2; l <= lb; l++)
-        hipLaunchKernelGGL(k_field_box<kBoxWG>, dim3(nchunk * t->nbox[l]), dim3(kBoxWG),
-                           sizeof(double2) * 2 * nr * pb, st, tl, l, (const double2 *)d_tab,
-                           d_tab + 2 * ntri, d_pts + 3 * (size_t)q0, nq0, nchunk, pl->k,
-                           nrhs, r0, d_box);
+        for (int q = 0; q < nr; q += 4) {
+          const int nb = nr - q < 4 ? nr - q : 4;
+          auto launch = nb == 1 ? launch_box<4, 1> : nb == 2 ? launch_box<2, 2> : launch_box<1, 4>;
+          launch(pl, o, l, leg, dg, d_pts + 3 * (size_t)q0, nq0, nrhs, r0 + q, nb,
+                 d_box + (size_t)q * nq0, st);
+        }
       hipLaunchKernelGGL(k_field_tree, dim3(nq0), dim3(kT), 0, st, tl,
-                         (const double2 *)d_tab, d_tab + 2 * ntri, d_pts + 3 * (size_t)q0,
+                         (const double2 *)leg, dg, d_pts + 3 * (size_t)q0,
                          t->d_tri, t->d_geo, t->d_perm, t->d_box_start, t->nelem, pl->k,
                          (const double2 *)pl->d_robin, pl->d_quad, pl->nq, pl->d_quadn,
                          pl->nqn, pl->prm.near_ratio, (const double2 *)x, nrhs, r0,
@@ -720,4 +776,35 @@ extern "C" int fmbh_field_tree(const fmb_plan *pl, int op, const fmb_c64 *x, int
   fmbh_free(d_tab);
   fmbh_free(d_box);
   return rc;
+}
+
+// Morton order of npts points (device, caller order): sorted points and the
+// caller's index of each, in memory of the caller (fmbh_field_order_bytes).
+extern "C" size_t fmbh_field_order_bytes(int npts) {
+  size_t tb = 0;
+  if (hipcub::DeviceRadixSort::SortPairs(nullptr, tb, (unsigned long long *)nullptr,
+                                         (unsigned long long *)nullptr, (int *)nullptr,
+                                         (int *)nullptr, npts, 0, 36) != hipSuccess)
+    return 0;
+  const size_t n = ((size_t)npts + 1) & ~(size_t)1;
+  return 16 * n + 4 * n + tb + 256;
+}
+
+extern "C" int fmbh_field_order(const fmb_tree *t, const double *d_pts, int npts, double *d_spts,
+                                int *d_qperm, void *work, size_t bytes, void *stream) {
+  hipStream_t st = (hipStream_t)stream;
+  const size_t n = ((size_t)npts + 1) & ~(size_t)1;
+  unsigned long long *key = (unsigned long long *)work, *key2 = key + n;
+  int *idx = (int *)(key2 + n);
+  void *tmp = (void *)(((size_t)(idx + n) + 255) & ~(size_t)255);
+  size_t tb = (char *)work + bytes - (char *)tmp;
+  hipLaunchKernelGGL(k_field_keys, dim3((npts + 255) / 256), dim3(256), 0, st, d_pts, npts, t->D,
+                     t->pmin[0], t->pmin[1], t->pmin[2], key, idx);
+  FMB_LAUNCH_CHECK();
+  FMB_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, key, key2, idx, d_qperm, npts, 0, 36,
+                                                   st));
+  hipLaunchKernelGGL(k_field_points, dim3((unsigned)((3 * (size_t)npts + 255) / 256)), dim3(256), 0, st, d_pts,
+                     d_qperm, npts, d_spts);
+  FMB_LAUNCH_CHECK();
+  return FMB_OK;
 }

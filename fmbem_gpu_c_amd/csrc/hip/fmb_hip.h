@@ -194,6 +194,11 @@ int fmbh_field(const fmb_plan *pl, const fmb_c64 *x, int nrhs, const double *d_p
 /* the same through the tree, from the multipole expansions that opset op
  * (FP64) holds for the nrhs vectors of x (field.hip); d_pts in Morton
  * order, d_qperm[i] the caller's index of point i */
+/* Morton order of field points: sorted copies and the caller's indices; work:
+ * fmbh_field_order_bytes (0: an error) */
+size_t fmbh_field_order_bytes(int npts);
+int fmbh_field_order(const fmb_tree *t, const double *d_pts, int npts, double *d_spts,
+                     int *d_qperm, void *work, size_t bytes, void *stream);
 int fmbh_field_tree(const fmb_plan *pl, int op, const fmb_c64 *x, int nrhs,
                     const double *d_pts, const int *d_qperm, int npts,
                     const double *d_dirs, fmb_c64 *out, void *stream);
