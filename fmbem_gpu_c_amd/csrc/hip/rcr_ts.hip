@@ -842,18 +842,27 @@ template <typename T, int W> int launch_ts(const fmbh_ts_job *j, int nrhs, hipSt
   a.sched = j->sched;
   a.in = j->in;
   a.out = j->out;
-  // Workgroups of a group: about 2,048 in all (8 a CU, for an even finish) as long as each keeps
-  // 4 batches or more to set up and flush for, and 256 if there are batches for them.  Level 6 of
-  // the 20,480-triangle sphere (FP64, order 14): 1.00 / 0.91 / 0.88 ms at 512 / 1,024 / 2,048;
-  // level 3 of the 1,280-triangle one: 0.071 / 0.044 ms at 1,024 / 256.
+  // Workgroups of a group: setting up and flushing costs one about two batches, and the last
+  // round of workgroups may be nearly empty, so J has the least (rounds) x (2 + batches), the
+  // largest J within 2% of it (an even finish).  A group's classes leave half a batch each.
+  // Against about 2,048 workgroups for every launch (FP64): level 4 of the 5,120-triangle sphere
+  // 131 -> 90 us (560 -> 248 workgroups), levels 6 and 5 of 20,480 with the levels beside them
+  // 1.85 -> 1.73 ms a product.
   const long long wg = (long long)a.ngroups * a.nrb;
-  const long long per = (long long)j->npairs * nrhs / kV / wg;  // batches of a group at least
-  long long J = (2048 + wg - 1) / wg;
-  if (J > per / 4) J = per / 4;
-  const long long fill = 256 / wg;
-  if (J < fill) J = fill < per ? fill : per;
-  a.J = J < 1 ? 1 : (int)J;
+  const double per = (double)j->npairs * nrhs / kV / wg + (a.R < kV ? 0.5 * kNC : 0.0);
   const size_t lds = fmbh_ts_lds_bytes(j->p, sizeof(T) == 8 ? FMB_FP64 : FMB_MIXED, j->slots);
+  const int cu = 160 * 1024 / (int)lds, fit = cu < 1 ? 1 : (cu < 16 / W ? cu : 16 / W);
+  auto cost = [&](long long J) {
+    const long long rounds = ((wg * J + 7) / 8 + 32 * fit - 1) / (32 * fit);
+    return rounds * (2.0 + per / J);
+  };
+  double least = 1e300;
+  long long most = (long long)j->npairs * nrhs / kV / wg;
+  if (most > 8192 / wg + 1) most = 8192 / wg + 1;
+  for (long long J = 1; J <= most; J++) least = cost(J) < least ? cost(J) : least;
+  a.J = 1;
+  for (long long J = most; J > 1 && a.J == 1; J--)
+    if (cost(J) <= 1.02 * least) a.J = (int)J;
   auto kern = k_m2l_ts<T, W>;
   if (lds > 160 * 1024)
     return fmb_set_error(FMB_ERR_RANGE, "M2L sums need %zu B of LDS", lds);

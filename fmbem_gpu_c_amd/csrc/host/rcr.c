@@ -316,8 +316,9 @@ static int octant_pairs(const fmb_tree *t, int l, fmb_rcr_tab *tb, void *stream)
  * long).  In the global workspace, FP64 alone, with 8 vectors a batch and
  * blocks in one piece: order 94 3.7 -> 2.7 ms, 62 3.1 -> 2.9, 42 4.8 -> 3.9
  * (FP32 order 62 13.2 -> 13.4).  Second (job_shape), launches that leave half
- * of the 256 CUs empty: FP64 M2M of 16 workgroups, order 16, 21 -> 17 us, of
- * 64, order 23, 36 -> 33, but of 204 41 -> 42. */
+ * of the 256 CUs empty, with 8 vectors a batch: FP64 M2M of 16 workgroups,
+ * order 16, 21 us with 4 waves and 16 vectors, 17 with 8 waves, 13 with 8
+ * vectors as well; of 64, order 23, 36 -> 33, but of 204 41 -> 42. */
 static int wide_form(fmb_plan *pl, fmb_rcr_tab *tb, int op, const int *hoff, const int *coff,
                      void *stream) {
   const int prec = pl->ops[op].prec, P = tb->P, mode = tb->mode[op];
@@ -333,6 +334,7 @@ static int wide_form(fmb_plan *pl, fmb_rcr_tab *tb, int op, const int *hoff, con
   } else {
     const size_t b = fmbh_rcr_lds_bytes(P, prec, nt, tb->sched_len[op]);
     wide = 160 * 1024 / b <= (prec == FMB_FP64 ? 1 : 2);
+    if (!wide) nt = 1;
   }
   int *sched = NULL, slen = 0;
   if ((rc = build_sched(tb->pin, tb->pout, P, mode, mt, 8, hoff, 0, coff, &sched, &slen, stream)))
