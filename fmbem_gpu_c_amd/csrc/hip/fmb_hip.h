@@ -148,6 +148,7 @@ int fmbh_pad_coax(int prec, const void *d_C, int ncoax, int P, int pin,
                   int pout, const int *d_coff, size_t pstride, void *d_Cp,
                   void *stream);
 /* ---- target-stationary M2L of low orders (rcr_ts.hip) */
+#define FMBH_TS_LEVELS 4
 #define FMBH_TS_PMAX 16    /* largest order                                 */
 #define FMBH_TS_WAVES64 16 /* waves of a workgroup in the FP64 pass         */
 #define FMBH_TS_WAVES32 8  /* in the FP32 pass                              */
@@ -171,7 +172,8 @@ typedef struct fmbh_ts_job {
 } fmbh_ts_job;
 /* LDS of a workgroup */
 size_t fmbh_ts_lds_bytes(int p, int prec, int slots);
-int fmbh_ts_run(const fmbh_ts_job *j, int prec, int nrhs, void *stream);
+/* n levels (at most FMBH_TS_LEVELS) in one launch */
+int fmbh_ts_run(const fmbh_ts_job *jobs, int n, int prec, int nrhs, void *stream);
 /* level l's pairs by (group of tgrp targets, class), allocated here; h_cls:
  * class of each offset code */
 int fmbh_ts_lists(const fmb_tree *t, int l, int tgrp, const int *h_cls, void **d_pairs,

@@ -551,11 +551,30 @@ struct TsArgs {
   void *out;
 };
 
+// Levels of one launch: level i takes workgroups end[i - 1] .. end[i] - 1.
+struct TsLevels {
+  int n;
+  unsigned end[FMBH_TS_LEVELS];
+  TsArgs a[FMBH_TS_LEVELS];
+};
+
 // LDS: the batch rows, then the sums' real and imaginary planes [coefficient][slot].  Slot: place
 // of the target in the group x R + right-hand side.
-template <typename T, int W>
+// The arguments of a workgroup's level and its place among the level's workgroups.  (One level has
+// its arguments to itself: choosing among levels costs the kernel 1%.)
+__device__ __forceinline__ const TsArgs &level_of(const TsArgs &a, unsigned &) { return a; }
+__device__ __forceinline__ const TsArgs &level_of(const TsLevels &lv, unsigned &block) {
+  int i = 0;
+  while (i + 1 < lv.n && block >= lv.end[i]) i++;
+  if (i) block -= lv.end[i - 1];
+  return lv.a[i];
+}
+
+template <typename T, int W, typename A>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4)))
-    k_m2l_ts(TsArgs a) {
+    k_m2l_ts(A args) {
+  unsigned block = blockIdx.x;
+  const TsArgs &a = level_of(args, block);
   constexpr int TS = (int)sizeof(T), CS = 2 * TS;
   extern __shared__ __align__(16) unsigned char smem[];
   const int p = a.p, p2 = p * p, SA = a.SA;
@@ -567,8 +586,8 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
   int g, jj, rb;
   {
     const unsigned items = (unsigned)a.ngroups * a.J * a.nrb, per = (items + 7) / 8;
-    const unsigned it = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (it >= items || (blockIdx.x >> 3) >= per) return;
+    const unsigned it = (block & 7) * per + (block >> 3);
+    if (it >= items || (block >> 3) >= per) return;
     rb = it % a.nrb;
     const unsigned q = it / a.nrb;
     jj = q % a.J;
@@ -814,63 +833,97 @@ __global__ void k_ts_coax(const cplx<T> *__restrict__ C, size_t cs, int p,
   }
 }
 
-template <typename T, int W> int launch_ts(const fmbh_ts_job *j, int nrhs, hipStream_t st) {
-  TsArgs a;
-  a.pairs = (const int2 *)j->pairs;
-  a.seg = j->seg;
-  a.ngroups = j->ngroups;
-  a.tgrp = j->tgrp;
-  a.nbox = j->nbox;
-  a.SA = j->slots | 1;  // odd: neighbouring coefficients fall into different LDS banks
-  // right-hand sides of a block: what the slots hold, in even blocks, which from 16 on are
-  // multiples of a batch
-  a.R = j->slots / j->tgrp;
-  a.nrb = (nrhs + a.R - 1) / a.R;
-  int even = (nrhs + a.nrb - 1) / a.nrb;
-  if (even >= kV) even = (even + kV - 1) / kV * kV;
-  if (even < a.R) a.R = even;
-  a.nrb = (nrhs + a.R - 1) / a.R;
-  a.p = j->p;
-  a.nrhs = nrhs;
-  a.phase = j->phase;
-  a.pstride = j->pstride;
-  a.H = j->H;
-  a.hstride = j->hstride;
-  a.C = j->C;
-  a.cstride = j->cstride;
-  for (int c = 0; c < kNC; c++) a.cdist[c] = j->cdist[c];
-  a.sched = j->sched;
-  a.in = j->in;
-  a.out = j->out;
-  // Workgroups of a group: setting up and flushing costs one about two batches, and the last
-  // round of workgroups may be nearly empty, so J has the least (rounds) x (2 + batches), the
-  // largest J within 2% of it (an even finish).  A group's classes leave half a batch each.
-  // Against about 2,048 workgroups for every launch (FP64): level 4 of the 5,120-triangle sphere
-  // 131 -> 90 us (560 -> 248 workgroups), levels 6 and 5 of 20,480 with the levels beside them
-  // 1.85 -> 1.73 ms a product.
-  const long long wg = (long long)a.ngroups * a.nrb;
-  const double per = (double)j->npairs * nrhs / kV / wg + (a.R < kV ? 0.5 * kNC : 0.0);
-  const size_t lds = fmbh_ts_lds_bytes(j->p, sizeof(T) == 8 ? FMB_FP64 : FMB_MIXED, j->slots);
-  const int cu = 160 * 1024 / (int)lds, fit = cu < 1 ? 1 : (cu < 16 / W ? cu : 16 / W);
-  auto cost = [&](long long J) {
-    const long long rounds = ((wg * J + 7) / 8 + 32 * fit - 1) / (32 * fit);
-    return rounds * (2.0 + per / J);
-  };
-  double least = 1e300;
-  long long most = (long long)j->npairs * nrhs / kV / wg;
-  if (most > 8192 / wg + 1) most = 8192 / wg + 1;
-  for (long long J = 1; J <= most; J++) least = cost(J) < least ? cost(J) : least;
-  a.J = 1;
-  for (long long J = most; J > 1 && a.J == 1; J--)
-    if (cost(J) <= 1.02 * least) a.J = (int)J;
-  auto kern = k_m2l_ts<T, W>;
+template <typename T, int W> int launch_ts(const fmbh_ts_job *jobs, int n, int nrhs, hipStream_t st) {
+  TsLevels lv;
+  lv.n = n;
+  double per[FMBH_TS_LEVELS];
+  long long wg[FMBH_TS_LEVELS], most[FMBH_TS_LEVELS], total = 0;
+  size_t lds = 0;
+  for (int i = 0; i < n; i++) {
+    const fmbh_ts_job *j = jobs + i;
+    TsArgs &a = lv.a[i];
+    a.pairs = (const int2 *)j->pairs;
+    a.seg = j->seg;
+    a.ngroups = j->ngroups;
+    a.tgrp = j->tgrp;
+    a.nbox = j->nbox;
+    a.SA = j->slots | 1;  // odd: neighbouring coefficients fall into different LDS banks
+    // right-hand sides of a block: what the slots hold, in even blocks, which from 16 on are
+    // multiples of a batch
+    a.R = j->slots / j->tgrp;
+    a.nrb = (nrhs + a.R - 1) / a.R;
+    int even = (nrhs + a.nrb - 1) / a.nrb;
+    if (even >= kV) even = (even + kV - 1) / kV * kV;
+    if (even < a.R) a.R = even;
+    a.nrb = (nrhs + a.R - 1) / a.R;
+    a.p = j->p;
+    a.nrhs = nrhs;
+    a.phase = j->phase;
+    a.pstride = j->pstride;
+    a.H = j->H;
+    a.hstride = j->hstride;
+    a.C = j->C;
+    a.cstride = j->cstride;
+    for (int c = 0; c < kNC; c++) a.cdist[c] = j->cdist[c];
+    a.sched = j->sched;
+    a.in = j->in;
+    a.out = j->out;
+    wg[i] = (long long)a.ngroups * a.nrb;
+    // batches of a group: its classes leave half a batch each
+    per[i] = (double)j->npairs * nrhs / kV / wg[i] + (a.R < kV ? 0.5 * kNC : 0.0);
+    most[i] = (long long)j->npairs * nrhs / kV / wg[i];
+    if (most[i] > 8192 / wg[i] + 1) most[i] = 8192 / wg[i] + 1;
+    if (most[i] < 1) most[i] = 1;
+    const size_t b = fmbh_ts_lds_bytes(j->p, sizeof(T) == 8 ? FMB_FP64 : FMB_MIXED, j->slots);
+    lds = b > lds ? b : lds;
+  }
   if (lds > 160 * 1024)
     return fmb_set_error(FMB_ERR_RANGE, "M2L sums need %zu B of LDS", lds);
-  FMB_HIP_CHECK(hipFuncSetAttribute((const void *)kern,
+  // Workgroups of a group (J): setting up and flushing costs one about two batches, and the last
+  // round of workgroups may be nearly empty, so the batches of a workgroup, the same at each level,
+  // have the least (rounds) x (2 + batches), and the most workgroups within 2% of it (an even
+  // finish).  (The host loop is at most 8,192 short steps.)  Against about 2,048 workgroups for every launch (FP64): level 4 of the 5,120-triangle
+  // sphere 131 -> 90 us (560 -> 248 workgroups), levels 6 and 5 of 20,480 with the levels beside
+  // them 1.85 -> 1.73 ms a product.
+  const int cu = 160 * 1024 / (int)lds, fit = cu < 1 ? 1 : (cu < 16 / W ? cu : 16 / W);
+  auto split = [&](int i, double b) {
+    const long long J = (long long)(per[i] / b + 0.999);
+    return J < 1 ? 1 : (J > most[i] ? most[i] : J);
+  };
+  auto cost = [&](double b) {
+    long long x = 0;
+    double longest = 0.0;
+    for (int i = 0; i < n; i++) {
+      const long long J = split(i, b);
+      x += (wg[i] * J + 7) / 8;
+      longest = per[i] / J > longest ? per[i] / J : longest;
+    }
+    return ((x + 32 * fit - 1) / (32 * fit)) * (2.0 + longest);
+  };
+  double least = 1e300, batches = per[0];
+  for (long long J = 1; J <= most[0]; J++) {
+    const double c = cost(per[0] / J);
+    least = c < least ? c : least;
+  }
+  for (long long J = most[0]; J >= 1; J--)
+    if (cost(per[0] / J) <= 1.02 * least) {
+      batches = per[0] / J;
+      break;
+    }
+  for (int i = 0; i < n; i++) {
+    lv.a[i].J = (int)split(i, batches);
+    total += 8 * ((wg[i] * lv.a[i].J + 7) / 8);
+    if (total > 0x7fffffffLL) return fmb_set_error(FMB_ERR_RANGE, "M2L grid too large");
+    lv.end[i] = (unsigned)total;
+  }
+  auto one = k_m2l_ts<T, W, TsArgs>;
+  auto more = k_m2l_ts<T, W, TsLevels>;
+  FMB_HIP_CHECK(hipFuncSetAttribute(n == 1 ? (const void *)one : (const void *)more,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-  const long long grid = 8 * ((wg * a.J + 7) / 8);
-  if (grid > 0x7fffffffLL) return fmb_set_error(FMB_ERR_RANGE, "M2L grid too large");
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * W), lds, st, a);
+  if (n == 1)
+    hipLaunchKernelGGL(one, dim3((unsigned)total), dim3(64 * W), lds, st, lv.a[0]);
+  else
+    hipLaunchKernelGGL(more, dim3((unsigned)total), dim3(64 * W), lds, st, lv);
   FMB_LAUNCH_CHECK();
   return FMB_OK;
 }
@@ -882,12 +935,21 @@ extern "C" size_t fmbh_ts_lds_bytes(int p, int prec, int slots) {
   return (p2 + p) / 2 * kL * tsz + 2 * p2 * (slots | 1) * tsz;
 }
 
-extern "C" int fmbh_ts_run(const fmbh_ts_job *j, int prec, int nrhs, void *stream) {
-  if (!j->npairs) return FMB_OK;
-  if (j->p > FMBH_TS_PMAX || j->tgrp < 1 || j->tgrp > j->slots || j->slots > 255)
-    return fmb_set_error(FMB_ERR_RANGE, "no target-stationary M2L for order %d", j->p);
-  if (prec == FMB_FP64) return launch_ts<double, FMBH_TS_WAVES64>(j, nrhs, (hipStream_t)stream);
-  return launch_ts<float, FMBH_TS_WAVES32>(j, nrhs, (hipStream_t)stream);
+extern "C" int fmbh_ts_run(const fmbh_ts_job *jobs, int n, int prec, int nrhs, void *stream) {
+  fmbh_ts_job j[FMBH_TS_LEVELS];
+  int m = 0;
+  if (n < 0 || n > FMBH_TS_LEVELS)
+    return fmb_set_error(FMB_ERR_RANGE, "target-stationary M2L of %d levels", n);
+  for (int i = 0; i < n; i++) {
+    if (!jobs[i].npairs) continue;
+    if (jobs[i].p > FMBH_TS_PMAX || jobs[i].tgrp < 1 || jobs[i].tgrp > jobs[i].slots ||
+        jobs[i].slots > 255)
+      return fmb_set_error(FMB_ERR_RANGE, "no target-stationary M2L for order %d", jobs[i].p);
+    j[m++] = jobs[i];
+  }
+  if (!m) return FMB_OK;
+  if (prec == FMB_FP64) return launch_ts<double, FMBH_TS_WAVES64>(j, m, nrhs, (hipStream_t)stream);
+  return launch_ts<float, FMBH_TS_WAVES32>(j, m, nrhs, (hipStream_t)stream);
 }
 
 extern "C" int fmbh_ts_lists(const fmb_tree *t, int l, int tgrp, const int *h_cls, void **d_pairs,

@@ -16,6 +16,7 @@ int fmbx_rcr_setup(fmb_plan *pl, void *stream);
 void fmbx_rcr_free(fmb_plan *pl);
 int fmbx_rcr_run(const fmb_plan *pl, int op, int kind, int l, int nrhs,
                  void *stream);
+int fmbx_m2l_levels(const fmb_plan *pl, int op, int trans, int nrhs, int *from, void *stream);
 /* transposed translations, coefficients kept multiplied by (-1)^n */
 int fmbx_rcr_run_t(const fmb_plan *pl, int op, int kind, int l, int nrhs,
                    void *stream);

@@ -642,8 +642,12 @@ static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev
     if ((rc = run(pl, op, up, l, nrhs, su))) return rc;
   if (ev) fmbh_event_record(ev[2], stream);
   if (!split) {
+    int from = L + 1;
+    if (!ev && pl->prm.rcr_path != FMB_RCR_VALU &&
+        (rc = fmbx_m2l_levels(pl, op, trans, nrhs, &from, stream)))
+      return rc;
     for (int l = 2; l <= L; l++) {
-      ACROSS(l, stream);
+      if (l < from) ACROSS(l, stream);
       if (l > 2 && (rc = run(pl, op, down, l, nrhs, stream))) return rc;
     }
     return FMB_OK;

@@ -622,7 +622,7 @@ static int ts_setup(fmb_plan *pl, int l, fmb_rcr_tab *tb, int op, void *stream) 
   return rc;
 }
 
-static int ts_run(const fmb_plan *pl, int op, int l, int trans, int nrhs, void *stream) {
+static void ts_job(const fmb_plan *pl, int op, int l, int trans, int nrhs, fmbh_ts_job *job) {
   const fmb_rcr_tab *tb = &pl->rcr[0][l];
   const fmb_opset *o = &pl->ops[op];
   const int S = tb->ts_slots[op];
@@ -652,13 +652,33 @@ static int ts_run(const fmb_plan *pl, int op, int l, int trans, int nrhs, void *
   j.sched = tb->d_ts_sched[op];
   j.in = trans ? o->d_L[l] : o->d_M[l];
   j.out = trans ? o->d_M[l] : o->d_L[l];
-  return fmbh_ts_run(&j, o->prec, nrhs, stream);
+  *job = j;
+}
+
+static int ts_run(const fmb_plan *pl, int op, int l, int trans, int nrhs, void *stream) {
+  fmbh_ts_job j;
+  ts_job(pl, op, l, trans, nrhs, &j);
+  return fmbh_ts_run(&j, 1, pl->ops[op].prec, nrhs, stream);
 }
 
 /* the target-stationary M2L was set up for this pass */
 static int ts_ready(const fmb_plan *pl, int op, int l, int nrhs) {
   return pl->rcr[0][l].ts_slots[op] &&
          ts_use(pl->ops[op].prec, pl->p[l], pl->tree->npairs[l], nrhs);
+}
+
+/* M2L (M2L^T) of the finest levels that run target-stationary, in one launch;
+ * *from: the coarsest level done, lmax + 1 if none.  A level of a few hundred
+ * workgroups ends in a round that leaves CUs idle, and each launch sets up its
+ * tables again: levels 2 and 3 of 1,280 triangles (FP64) 27 + 41 us apart, 55
+ * together. */
+int fmbx_m2l_levels(const fmb_plan *pl, int op, int trans, int nrhs, int *from, void *stream) {
+  fmbh_ts_job j[FMBH_TS_LEVELS];
+  int n = 0, l = pl->tree->lmax;
+  for (; l >= 2 && n < FMBH_TS_LEVELS && pl->rcr[0][l].mode[op] && ts_ready(pl, op, l, nrhs); l--)
+    ts_job(pl, op, l, trans, nrhs, &j[n++]);
+  *from = l + 1;
+  return fmbh_ts_run(j, n, pl->ops[op].prec, nrhs, stream);
 }
 
 int fmbx_rcr_rot_setup(fmb_plan *pl, void *stream) {

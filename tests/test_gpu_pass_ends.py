@@ -54,3 +54,19 @@ def test_two_streams_match_one(depth):
             ref = getattr(one, fn)(x, prec=prec)
             for _ in range(3):   # the streams' order of one pass must not matter to the next
                 assert _err(getattr(two, fn)(x, prec=prec), ref) < tol, (prec, fn)
+
+
+@pytest.mark.parametrize("orders", [[16, 14, 11, 9, 6], [20, 16, 15, 12, 14], [5, 5, 17, 5, 4]])
+def test_levels_of_one_launch(orders):
+    """A pass on one stream runs the finest target-stationary levels, four at
+    most, in one launch: five such levels, and levels that end or interrupt
+    their run, against a launch a level on two streams."""
+    t = F.Tree(F.Mesh.ellipsoid(23, 0.08, 0.07, 0.10, seed=3), depth=6)
+    k = wavenumber(3000.0)
+    kw = dict(precision=F.FMB_MIXED, nrhs_max=2, p_rule=F.PRULE_EXPLICIT, p_levels=[0, 0] + orders)
+    two, one = F.Plan(t, k, **kw), F.Plan(t, k, serial_levels=1, **kw)
+    for nrhs in (1, 2):
+        x = _vec(nrhs, t.n, nrhs)
+        for prec, tol in ((F.FMB_FP64, 1e-13), (F.FMB_MIXED, 1e-5)):
+            for fn in ("matvec", "matvec_t"):
+                assert _err(getattr(one, fn)(x, prec=prec), getattr(two, fn)(x, prec=prec)) < tol
