@@ -26,8 +26,13 @@
 namespace {
 
 constexpr int kT = 256, kR = 8;
-constexpr int kFieldSlicePts = 1024; // below this many points k_field slices the panels
+constexpr int kFieldSlicePts = 1024; // below this many point groups k_field slices the panels
 
+// R right-hand sides at P field points a workgroup: a thread takes a panel for
+// all P, so that its 136 bytes, strided over the lanes, are read once for them
+// and the points' chains run beside each other.  81,920 panels at 32 points
+// with one right-hand side: 120 us at P = 1, 87 at 4.
+template <int P, int R>
 __global__ void __launch_bounds__(kT)
     k_field(const double *__restrict__ pts, int npts, const double *__restrict__ tri,
             const double *__restrict__ geo, const int *__restrict__ perm, int N,
@@ -36,63 +41,103 @@ __global__ void __launch_bounds__(kT)
             int nqn, double ratio, const double2 *__restrict__ x, int nrhs, int r0,
             const double *__restrict__ dirs, double2 *__restrict__ out,
             double2 *__restrict__ part) {
-  __shared__ double2 red[kT / 64][kR];
-  const int q = blockIdx.x, nsl = gridDim.y;
-  const double y[3] = {pts[3 * q], pts[3 * q + 1], pts[3 * q + 2]};
+  __shared__ double2 red[kT / 64][P * R];
+  const int q0 = blockIdx.x * P, nsl = gridDim.y;
   const double nz[3] = {0.0, 0.0, 0.0};
-  const int nr = min(kR, nrhs - r0);
-  double2 acc[kR];
+  const int nr = min(R, nrhs - r0);
+  double y[P][3];
+  double2 acc[P][R];
 #pragma unroll
-  for (int r = 0; r < kR; r++) acc[r] = make_double2(0.0, 0.0);
+  for (int i = 0; i < P; i++) {
+    const int q = min(q0 + i, npts - 1);  // (points beyond the last repeat it)
+    for (int a = 0; a < 3; a++) y[i][a] = pts[3 * (size_t)q + a];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[i][r] = make_double2(0.0, 0.0);
+  }
   for (int j = blockIdx.y * kT + threadIdx.x; j < N; j += nsl * kT) {
-    const double *gj = geo + 8 * (size_t)j;
-    const double dx = y[0] - gj[0], dy = y[1] - gj[1], dz = y[2] - gj[2];
-    const bool close = dx * dx + dy * dy + dz * dz < ratio * ratio * gj[7] * gj[7];
-    double2 o[4];
-    panel_sum(k, y, nz, tri + 9 * (size_t)j, gj + 3, gj[6], close ? quadn : quad,
-              close ? nqn : nq, o);
-    double2 g = o[1];
-    if (robin) {
-      const double2 s = robin[j];
-      g.x -= s.x * o[0].x - s.y * o[0].y;
-      g.y -= s.x * o[0].y + s.y * o[0].x;
+    const double *gj = geo + 8 * (size_t)j, *tr = tri + 9 * (size_t)j;
+    double t[9], g8[8];
+    for (int a = 0; a < 9; a++) t[a] = tr[a];
+    for (int a = 0; a < 8; a++) g8[a] = gj[a];
+    const double lim = ratio * ratio * g8[7] * g8[7];
+    bool close[P];
+    double2 S[P], K[P];  // int G, int dG/dn_y
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+      const double dx = y[i][0] - g8[0], dy = y[i][1] - g8[1], dz = y[i][2] - g8[2];
+      close[i] = dx * dx + dy * dy + dz * dz < lim;
+      S[i] = K[i] = make_double2(0.0, 0.0);
     }
+    for (int q = 0; q < nq; q++) {  // (panel_sum's S and K)
+      const double *qq = quad + 4 * q;
+      const double w = qq[3] * g8[6];
+      double z[3];
+      for (int a = 0; a < 3; a++) z[a] = qq[0] * t[a] + qq[1] * t[3 + a] + qq[2] * t[6 + a];
+#pragma unroll
+      for (int i = 0; i < P; i++) {
+        const double d0 = y[i][0] - z[0], d1 = y[i][1] - z[1], d2 = y[i][2] - z[2];
+        const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2), ir = 1.0 / r;
+        double sn, cs;
+        sincos(k * r, &sn, &cs);
+        const double g0 = (1.0 / (4.0 * M_PI)) * ir, gr = cs * g0, gi = sn * g0;
+        const double wn = -w * ((d0 * g8[3] + d1 * g8[4] + d2 * g8[5]) * ir);
+        const double gpr = -gr * ir - k * gi, gpi = -gi * ir + k * gr;
+        S[i].x += w * gr;
+        S[i].y += w * gi;
+        K[i].x += wn * gpr;
+        K[i].y += wn * gpi;
+      }
+    }
+    const double2 sg = robin ? robin[j] : make_double2(0.0, 0.0);
     const int c = perm[j];
 #pragma unroll
-    for (int r = 0; r < kR; r++) {
-      if (r < nr) {
-        const double2 v = x[(size_t)(r0 + r) * N + c];
-        acc[r].x += g.x * v.x - g.y * v.y;
-        acc[r].y += g.x * v.y + g.y * v.x;
+    for (int i = 0; i < P; i++) {
+      if (close[i]) {
+        double2 o[4];
+        panel_sum(k, y[i], nz, t, g8 + 3, g8[6], quadn, nqn, o);
+        S[i] = o[0];
+        K[i] = o[1];
+      }
+      double2 g = K[i];
+      if (robin) {
+        g.x -= sg.x * S[i].x - sg.y * S[i].y;
+        g.y -= sg.x * S[i].y + sg.y * S[i].x;
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        if (r < nr) {
+          const double2 v = x[(size_t)(r0 + r) * N + c];
+          acc[i][r].x += g.x * v.x - g.y * v.y;
+          acc[i][r].y += g.x * v.y + g.y * v.x;
+        }
       }
     }
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
-  for (int r = 0; r < kR; r++) {
-    double re = acc[r].x, im = acc[r].y;
-    for (int o = 32; o > 0; o >>= 1) {
-      re += __shfl_down(re, o, 64);
-      im += __shfl_down(im, o, 64);
+  for (int i = 0; i < P; i++)
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const double re = wave_all_sum(acc[i][r].x), im = wave_all_sum(acc[i][r].y);
+      if (lane == 0) red[w][i * R + r] = make_double2(re, im);
     }
-    if (lane == 0) red[w][r] = make_double2(re, im);
-  }
   __syncthreads();
-  if (threadIdx.x < nr) {
-    const int r = threadIdx.x;
+  if (threadIdx.x < P * R) {
+    const int r = threadIdx.x % R, q = q0 + threadIdx.x / R;
+    if (r >= nr || q >= npts) return;
     double2 s = make_double2(0.0, 0.0);
     for (int i = 0; i < kT / 64; i++) {
-      s.x += red[i][r].x;
-      s.y += red[i][r].y;
+      s.x += red[i][threadIdx.x].x;
+      s.y += red[i][threadIdx.x].y;
     }
     if (part) {
       part[((size_t)blockIdx.y * kR + r) * npts + q] = s;
       return;
     }
     if (dirs) {
-      const double *d = dirs + 3 * (r0 + r);
+      const double *d = dirs + 3 * (r0 + r), *yq = pts + 3 * (size_t)q;
       double sn, cs;
-      sincos(k * (d[0] * y[0] + d[1] * y[1] + d[2] * y[2]), &sn, &cs);
+      sincos(k * (d[0] * yq[0] + d[1] * yq[1] + d[2] * yq[2]), &sn, &cs);
       s.x += cs;
       s.y += sn;
     }
@@ -100,22 +145,25 @@ __global__ void __launch_bounds__(kT)
   }
 }
 
-// The panel slices of k_field summed in slice order, plus the incident
-// waves: one thread per (point, right-hand side).
+// The panel slices of k_field summed in a fixed order, plus the incident
+// waves: one wavefront per (point, right-hand side).
 __global__ void __launch_bounds__(kT)
     k_field_sum(const double2 *__restrict__ part, int nsl, const double *__restrict__ pts,
                 int npts, double k, int nrhs, int r0, const double *__restrict__ dirs,
                 double2 *__restrict__ out) {
-  const int i = blockIdx.x * kT + threadIdx.x;
+  const int i = (blockIdx.x * kT + threadIdx.x) >> 6, lane = threadIdx.x & 63;
   const int nr = min(kR, nrhs - r0);
   if (i >= npts * nr) return;
   const int r = i / npts, q = i % npts;
   double2 s = make_double2(0.0, 0.0);
-  for (int sl = 0; sl < nsl; sl++) {
+  for (int sl = lane; sl < nsl; sl += 64) {
     const double2 v = part[((size_t)sl * kR + r) * npts + q];
     s.x += v.x;
     s.y += v.y;
   }
+  s.x = wave_all_sum(s.x);
+  s.y = wave_all_sum(s.y);
+  if (lane != 0) return;
   if (dirs) {
     const double *d = dirs + 3 * (r0 + r);
     double sn, cs;
@@ -673,23 +721,27 @@ extern "C" int fmbh_field(const fmb_plan *pl, const fmb_c64 *x, int nrhs,
                           fmb_c64 *out, void *stream) {
   const fmb_tree *t = pl->tree;
   hipStream_t st = (hipStream_t)stream;
-  // few points: each point's panels in slices over several workgroups, so
-  // that the launch fills the device; the slices are summed in order
-  const int nsl = npts >= kFieldSlicePts ? 1 : min(32, (2 * kFieldSlicePts + npts - 1) / npts);
+  // one right-hand side: four points a workgroup; few points: their panels in
+  // slices over several workgroups, so that the launch fills the device; the
+  // slices are summed in order
+  const int P = nrhs == 1 && npts >= 4 ? 4 : 1, ng = (npts + P - 1) / P;
+  const int nsl = ng >= kFieldSlicePts
+                      ? 1
+                      : min(P == 4 ? 128 : 32, (2 * kFieldSlicePts + ng - 1) / ng);
   double2 *d_part = NULL;
   int rc = FMB_OK;
   if (nsl > 1 && (rc = fmbh_malloc((void **)&d_part, sizeof(double2) * (size_t)nsl * kR * npts)))
     return rc;
   for (int r0 = 0; r0 < nrhs && !rc; r0 += kR) {
-    hipLaunchKernelGGL(k_field, dim3(npts, nsl), dim3(kT), 0, st, d_pts, npts, t->d_tri,
-                       t->d_geo, t->d_perm, t->nelem, pl->k,
-                       (const double2 *)pl->d_robin, pl->d_quad, pl->nq, pl->d_quadn,
-                       pl->nqn, pl->prm.near_ratio, (const double2 *)x, nrhs, r0,
+    hipLaunchKernelGGL((P == 4 ? k_field<4, 1> : nrhs == 1 ? k_field<1, 1> : k_field<1, kR>),
+                       dim3(ng, nsl), dim3(kT), 0, st, d_pts, npts, t->d_tri, t->d_geo, t->d_perm,
+                       t->nelem, pl->k, (const double2 *)pl->d_robin, pl->d_quad, pl->nq,
+                       pl->d_quadn, pl->nqn, pl->prm.near_ratio, (const double2 *)x, nrhs, r0,
                        d_dirs, (double2 *)out, d_part);
     if (nsl > 1) {
       const int nr = nrhs - r0 < kR ? nrhs - r0 : kR;
-      hipLaunchKernelGGL(k_field_sum, dim3((npts * nr + kT - 1) / kT), dim3(kT), 0, st, d_part,
-                         nsl, d_pts, npts, pl->k, nrhs, r0, d_dirs, (double2 *)out);
+      hipLaunchKernelGGL(k_field_sum, dim3((npts * nr + 3) / 4), dim3(kT), 0, st, d_part, nsl,
+                         d_pts, npts, pl->k, nrhs, r0, d_dirs, (double2 *)out);
     }
     if (hipGetLastError() != hipSuccess) rc = fmb_set_error(FMB_ERR_HIP, "k_field launch");
   }

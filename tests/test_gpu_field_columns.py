@@ -35,3 +35,26 @@ def test_vs_oracle(p2, p3, nrhs, npts):
     e = np.linalg.norm(got - want) / np.linalg.norm(want)
     print(p2, p3, nrhs, npts, "%.1e" % e, flush=True)
     assert e < 1e-10
+
+
+@pytest.mark.parametrize("npts", [1, 3, 4, 5, 63, 257, 4096, 4099])
+def test_direct_points_of_a_workgroup(npts):
+    """The direct sum takes four points a workgroup with one right-hand side
+    and one with more: the same panel sums of 1,280 terms in another order,
+    1e-13, off the surface and within the refined rule's distance of it."""
+    m = F.Mesh.icosphere(3, 0.1)
+    t = F.Tree(m, depth=3)
+    k = wavenumber(2000.0)
+    rng = np.random.default_rng(npts)
+    sig = torch.tensor(rng.standard_normal(t.n) + 1j * rng.standard_normal(t.n), device="cuda")
+    pl = F.Plan(t, k, robin=sig, nrhs_max=2)
+    x = torch.tensor(rng.standard_normal((2, t.n)) + 1j * rng.standard_normal((2, t.n)),
+                     device="cuda")
+    d = rng.standard_normal((npts, 3))
+    pts = d / np.linalg.norm(d, axis=1)[:, None] * rng.choice([0.101, 0.105, 0.3], npts)[:, None]
+    dirs = np.array([[0.0, 0.0, 1.0], [0.6, 0.8, 0.0]])
+    both = pl.field(x, pts, dirs)
+    for r in range(2):
+        one = pl.field(x[r:r + 1].contiguous(), pts, dirs[r:r + 1])
+        e = float(torch.linalg.norm(one[0] - both[r]) / torch.linalg.norm(both[r]))
+        assert e < 1e-13, (npts, r, e)
