@@ -636,7 +636,8 @@ static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev
     if ((rc = fmbh_stream_wait(aux, pl->ev_up))) return rc;
   }
   /* (a timed pass keeps the chain up, a phase of its own, on the caller's
-   * stream) */
+   * stream, and runs the finest level last and alone, so that its events time
+   * that launch and not what ran beside it) */
   void *su = split && !ev ? aux : stream;
   for (int l = L; l > 2; l--)
     if ((rc = run(pl, op, up, l, nrhs, su))) return rc;
@@ -654,7 +655,7 @@ static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev
   }
   const int ls = L - 2 > 2 ? L - 2 : 2;
   if ((rc = fmbh_event_record(pl->ev_m2l[L], su))) return rc;
-  ACROSS(L, stream);
+  if (!ev) ACROSS(L, stream);
   if ((rc = fmbh_stream_wait(su == aux ? stream : aux, pl->ev_m2l[L]))) return rc;
   for (int l = ls; l < L; l++) {
     ACROSS(l, stream);
@@ -667,9 +668,10 @@ static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev
       if ((rc = run(pl, op, down, l, nrhs, aux))) return rc;
     }
   }
-#undef ACROSS
   if ((rc = fmbh_event_record(pl->ev_aux, aux))) return rc;
   if ((rc = fmbh_stream_wait(stream, pl->ev_aux))) return rc;
+  if (ev) ACROSS(L, stream);
+#undef ACROSS
   return L > 2 ? run(pl, op, down, L, nrhs, stream) : FMB_OK;
 }
 
