@@ -39,11 +39,11 @@
 #include <type_traits>
 
 #include "fmb_device.h"
+#include "rcr_ts_rows.h"
 
 namespace {
 
-constexpr int kV = 16;  // vectors of a batch
-constexpr int kL = 64;  // reals of a batch row
+using namespace fmb_ts;
 constexpr int kNC = FMB_NCLASS;
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -320,22 +320,14 @@ template <int RG> struct Coax<double, RG> {
   }
 };
 
-// what a wave needs of the batch: lanes li, li + 16, .. stand for vector li
-struct Vec {
-  int soff, phr, slot;  // byte offsets of its source and phase row; its target's slot, or -1
-  int rank;             // FP32: its place among the batch's vectors of that slot, or -1
-};
-
 template <typename T> struct Ctx {
+  typedef T real;
   __amdgpu_buffer_rsrc_t rin, rph;
   T *X, *accr, *acci;
   int p, SA, par, lane;  // par: bytes of a phase row
 };
 
-// rows m = 4 j + lane / 16 (clamped to n) of degree n: coefficients +-m of the sources, phases
-template <int RG> __device__ __forceinline__ int row_of(int j, int lk, int n) {
-  return j < RG - 1 ? 4 * j + lk : min(4 * j + lk, n);
-}
+// rows row_of of degree n: coefficients +-m of the sources, phases
 template <typename T, int RG> struct Src {
   cplx<T> zp[RG], zm[RG];
   __device__ __forceinline__ void load(const Ctx<T> &x, const Vec &v, int n) {
@@ -357,93 +349,6 @@ template <typename T, int RG> struct Pha {
           (n & 1) * x.par);
   }
 };
-
-// sources to e and o with their phases, then the first rotation: rows of degree n
-template <typename T, int RG>
-__device__ __forceinline__ void first_rot(const Ctx<T> &x, const Src<T, RG> &z,
-                                          const Pha<T, RG> &f, Rot<T, RG> &B, int n) {
-  T *xn = x.X + ((n * (n + 1)) >> 1) * kL;
-  const int li = x.lane & 15, lk = x.lane >> 4;
-#pragma unroll
-  for (int j = 0; j < RG; j++) {
-    const T sr = z.zp[j].re + z.zm[j].re, dr = z.zp[j].re - z.zm[j].re;
-    const T si = z.zp[j].im + z.zm[j].im, di = z.zp[j].im - z.zm[j].im;
-    const cplx<T> w = f.w[j];
-    T *y = xn + row_of<RG>(j, lk, n) * kL + li;
-    y[0] = sr * w.re - di * w.im;
-    y[16] = si * w.re + dr * w.im;
-    y[32] = dr * w.re - si * w.im;
-    y[48] = di * w.re + sr * w.im;
-  }
-  B.run(xn + x.lane, n);
-#pragma unroll
-  for (int i = 0; i < 4 * RG; i++)
-    if (i <= 4 * RG - 4 || i <= n) xn[i * kL + x.lane] = B.row(i);
-}
-
-// back rotation of degree n, output phases, sums into the targets' slots; most: the largest rank
-// of the batch (FP32)
-template <typename T, int RG>
-__device__ __forceinline__ void back_rot(const Ctx<T> &x, const Vec &v, int most,
-                                         const Pha<T, RG> &f, Rot<T, RG> &B, int n) {
-  T *xn = x.X + ((n * (n + 1)) >> 1) * kL;
-  const int li = x.lane & 15, lk = x.lane >> 4;
-  B.run(xn + x.lane, n);
-#pragma unroll
-  for (int i = 0; i < 4 * RG; i++)
-    if (i <= 4 * RG - 4 || i <= n) xn[i * kL + x.lane] = B.row(i);
-  T y0[RG], y1[RG], y2[RG], y3[RG];
-#pragma unroll
-  for (int j = 0; j < RG; j++) {
-    const T *y = xn + row_of<RG>(j, lk, n) * kL + li;
-    const T er = y[0], ei = y[16], orr = y[32], oi = y[48];
-    const T pr = er + orr, pi = ei + oi, qr = er - orr, qi = ei - oi;
-    const cplx<T> w = f.w[j];
-    y0[j] = pr * w.re + pi * w.im;
-    y1[j] = pi * w.re - pr * w.im;
-    y2[j] = qr * w.re - qi * w.im;
-    y3[j] = qi * w.re + qr * w.im;
-  }
-  const int c0 = n * n + n;
-  const int fp0 = (c0 + lk) * x.SA + v.slot, fm0 = (c0 - lk) * x.SA + v.slot;
-  const bool tail = 4 * RG - 4 + lk <= n;  // the last rows may lie past the block
-  if constexpr (sizeof(T) == 8) {
-    if (v.slot >= 0) {
-#pragma unroll
-      for (int j = 0; j < RG; j++) {
-        if (j == RG - 1 && !tail) break;
-        unsafeAtomicAdd(x.accr + fp0 + 4 * j * x.SA, y0[j]);
-        unsafeAtomicAdd(x.acci + fp0 + 4 * j * x.SA, y1[j]);
-        if (j > 0 || lk) {
-          unsafeAtomicAdd(x.accr + fm0 - 4 * j * x.SA, y2[j]);
-          unsafeAtomicAdd(x.acci + fm0 - 4 * j * x.SA, y3[j]);
-        }
-      }
-    }
-  } else {
-    for (int q = 0; q <= most; q++)
-      if (v.rank == q) {
-        T s0[RG], s1[RG], s2[RG], s3[RG];
-#pragma unroll
-        for (int j = 0; j < RG; j++) {
-          const int d = 4 * (j == RG - 1 && !tail ? 0 : j) * x.SA;
-          s0[j] = x.accr[fp0 + d];
-          s1[j] = x.acci[fp0 + d];
-          s2[j] = x.accr[fm0 - d];
-          s3[j] = x.acci[fm0 - d];
-        }
-#pragma unroll
-        for (int j = 0; j < RG; j++) {
-          if (j == RG - 1 && !tail) break;
-          const int d = 4 * j * x.SA;
-          x.accr[fm0 - d] = s2[j] + y2[j];
-          x.acci[fm0 - d] = s3[j] + y3[j];
-          x.accr[fp0 + d] = s0[j] + y0[j];  // (m = 0: the same element, written last)
-          x.acci[fp0 + d] = s1[j] + y1[j];
-        }
-      }
-  }
-}
 
 // One unit of the phase between two batches: the back rotation of the current batch (vc) and the
 // first rotation of the next one (vn), both of degree n.  FIRST: the wave's first unit, with the
@@ -469,8 +374,8 @@ __device__ __forceinline__ void rot_unit(const Ctx<T> &x, bool cur, bool nxt, co
       g.load(x, vn, n);
     }
     if constexpr (FIRST) __syncthreads();
-    if (cur) back_rot<T, RG>(x, vc, most, f, B, n);
-    if (nxt) first_rot<T, RG>(x, z, g, N, n);
+    if (cur) back_rot<RG>(x, vc, most, f, B, n);
+    if (nxt) first_rot<RG>(x, z, g, N, n);
   } else {
     if (cur) {
       Rot<T, RG> B;
@@ -478,7 +383,7 @@ __device__ __forceinline__ void rot_unit(const Ctx<T> &x, bool cur, bool nxt, co
       B.load(rhc, aoff, x.lane);
       f.load(x, vc, n);
       if constexpr (FIRST) __syncthreads();
-      back_rot<T, RG>(x, vc, most, f, B, n);
+      back_rot<RG>(x, vc, most, f, B, n);
     }
     if (nxt) {
       Src<T, RG> z;
@@ -487,7 +392,7 @@ __device__ __forceinline__ void rot_unit(const Ctx<T> &x, bool cur, bool nxt, co
       z.load(x, vn, n);
       f.load(x, vn, n);
       B.load(rhn, aoff, x.lane);
-      first_rot<T, RG>(x, z, f, B, n);
+      first_rot<RG>(x, z, f, B, n);
     }
   }
 }
@@ -500,12 +405,7 @@ __device__ __forceinline__ void coax_unit(const Ctx<T> &x, __amdgpu_buffer_rsrc_
   B.load(rc, aoff, x.lane);
   if constexpr (FIRST) __syncthreads();
   B.run(x.X, rc, aoff, m, x.p, x.lane);
-#pragma unroll
-  for (int i = 0; i < 4 * RG; i++)
-    if (i <= 4 * RG - 4 || m + i < x.p) {
-      const int r = m + i;
-      x.X[(((r * (r + 1)) >> 1) + m) * kL + x.lane] = B.row(i);
-    }
+  coax_put<RG>(x, B, m);
 }
 
 // unit<RG> for a wave-uniform rg in [1, 4]
