@@ -23,7 +23,16 @@ struct Vec {
 };
 
 #ifdef __HIPCC__
+// What the lanes of this wave wrote to LDS before is seen by all of them after, and nothing that
+// they read before changes: the hardware keeps a wave's LDS accesses in order, so this is for the
+// compiler, which may reorder or fold what it sees as the accesses of one lane.  No instruction.
+FMB_TS_FN void order_lanes() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 FMB_TS_FN void add_sum(double *p, double v) { unsafeAtomicAdd(p, v); }
+#else
+void order_lanes();
 #endif
 
 // row m = 4 j + lane / 16 of degree n, clamped to n
@@ -48,6 +57,7 @@ FMB_TS_FN void first_rot(const C &x, const Z &z, const F &f, B &rot, int n) {
     y[32] = dr * w.re - si * w.im;
     y[48] = di * w.re + sr * w.im;
   }
+  order_lanes();
   rot.run(xn + x.lane, n);
 #pragma unroll
   for (int i = 0; i < 4 * RG; i++)
@@ -57,6 +67,7 @@ FMB_TS_FN void first_rot(const C &x, const Z &z, const F &f, B &rot, int n) {
 // rows of coaxial block |m|, which a lane's product has read for itself and for the lane of the
 // other part (re, im)
 template <int RG, typename C, typename B> FMB_TS_FN void coax_put(const C &x, const B &cx, int m) {
+  order_lanes();
 #pragma unroll
   for (int i = 0; i < 4 * RG; i++)
     if (i <= 4 * RG - 4 || m + i < x.p) {
@@ -76,6 +87,7 @@ FMB_TS_FN void back_rot(const C &x, const Vec &v, int most, const F &f, B &rot, 
 #pragma unroll
   for (int i = 0; i < 4 * RG; i++)
     if (i <= 4 * RG - 4 || i <= n) xn[i * kL + x.lane] = rot.row(i);
+  order_lanes();
   T y0[RG], y1[RG], y2[RG], y3[RG];
 #pragma unroll
   for (int j = 0; j < RG; j++) {
@@ -104,8 +116,9 @@ FMB_TS_FN void back_rot(const C &x, const Vec &v, int most, const F &f, B &rot, 
         }
       }
     }
+    order_lanes();  // (the next batch writes these rows)
   } else {
-    for (int q = 0; q <= most; q++)
+    for (int q = 0; q <= most; q++) {
       if (v.rank == q) {
         T s0[RG], s1[RG], s2[RG], s3[RG];
 #pragma unroll
@@ -127,6 +140,8 @@ FMB_TS_FN void back_rot(const C &x, const Vec &v, int most, const F &f, B &rot, 
           x.acci[fp0 + d] = s1[j] + y1[j];
         }
       }
+      order_lanes();  // (the next rank adds to the same sums, the next batch writes these rows)
+    }
   }
 }
 

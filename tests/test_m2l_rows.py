@@ -10,7 +10,7 @@ import pytest
 from conftest import ROOT
 
 
-@pytest.mark.parametrize("what", ["range"])
+@pytest.mark.parametrize("what", ["range", "order"])
 def test_accesses(what, tmp_path):
     exe = str(tmp_path / "check")
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wno-unknown-pragmas",
