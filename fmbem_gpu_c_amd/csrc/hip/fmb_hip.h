@@ -35,6 +35,7 @@ int fmbh_event_create_sync(void **ev);
 int fmbh_stream_create(void **s);
 int fmbh_stream_destroy(void *s);
 int fmbh_stream_wait(void *stream, void *ev);
+int fmbh_stream_capturing(void *stream); /* 1: its work is being captured, else 0 */
 int fmbh_capture_begin(void *stream);
 int fmbh_capture_end(void *stream, void **exec);
 int fmbh_graph_launch(void *exec, void *stream);

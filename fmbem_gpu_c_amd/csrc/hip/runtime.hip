@@ -156,6 +156,15 @@ extern "C" int fmbh_stream_wait(void *stream, void *ev) {
   return FMB_OK;
 }
 
+extern "C" int fmbh_stream_capturing(void *stream) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &s) != hipSuccess) {
+    (void)hipGetLastError(); /* (the null stream while another is captured) */
+    return 0;
+  }
+  return s != hipStreamCaptureStatusNone;
+}
+
 extern "C" int fmbh_capture_begin(void *stream) {
   FMB_HIP_CHECK(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeRelaxed));
   return FMB_OK;

@@ -617,8 +617,8 @@ int fmb_last_timing(const fmb_plan *pl, double *phase7, double *m2l16) {
  * Against the finest level last and alone: 81,920 triangles FP32 3.31 -> 3.11
  * ms, 20,480 FP64 1.95 -> 1.85; transposed, which had one stream, 20,480 FP32
  * with three right-hand sides 3.68 -> 3.42.
- * Inside a graph capture the levels stay on the capturing stream (a second
- * fork there is not used, see fmb_gmres_batch). */
+ * Inside a graph capture, a batch's or the caller's own, the levels stay on
+ * the capturing stream (a fork there is not used, see graph_capture). */
 static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev, void *stream) {
   const int L = pl->tree->lmax, up = trans ? 2 : 1, down = trans ? 1 : 2;
   int (*run)(const fmb_plan *, int, int, int, int, void *) = trans ? fmbx_rcr_run_t : fmbx_rcr_run;
@@ -629,7 +629,7 @@ static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev
     if ((rc = run(pl, op, 0, l, nrhs, st))) return rc;                                   \
     if (ev) fmbh_event_record(ev[5 + 2 * (l)], st);                                      \
   } while (0)
-  const int split = pl->aux && !pl->capturing;
+  const int split = pl->aux && !pl->capturing && !fmbh_stream_capturing(stream);
   void *aux = pl->aux;
   if (split) {
     if ((rc = fmbh_event_record(pl->ev_up, stream))) return rc;
