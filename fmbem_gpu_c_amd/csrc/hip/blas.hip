@@ -10,6 +10,13 @@ constexpr int BS = 256;
 // blocks per inner product and per vector update at most: an inner product has nv nrhs rows of
 // blocks beside each other, an update only nrhs
 constexpr int DOT_CHUNKS = 128, UPD_CHUNKS = 2048;
+// Blocks up to which a reduction completes in its own launch.  Each block of such a launch releases
+// its partial sum, which writes its XCD's L2 back: 16 ns a block, one after the other, against 3 us
+// for a launch.  A step over 30 vectors, two right-hand sides of 10,580 elements (2,520 blocks an
+// inner product): 36 us with a launch of its own for the sums, 187 without (with an acquire in
+// every block too); over 29, nine of 327,680 (33,408): 1.31 ms, its bytes at the rate of a copy,
+// against 8.4.
+constexpr size_t kOneLaunch = 64;
 
 // sum of v over the block in a fixed order, in every thread
 __device__ __forceinline__ double block_sum(double v, double *sh) {
@@ -24,14 +31,17 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
 
 // Whether this block is the last of the n of reduction q to arrive: it then reads the others'
 // partial sums and completes the reduction, so a reduction takes one launch and its order does
-// not depend on which block is last.  Leaves the counter at 0.
+// not depend on which block is last.  Leaves the counter at 0.  A release writes the XCD's L2
+// back, so this is for launches of few blocks (kOneLaunch).
 __device__ __forceinline__ bool last_block(unsigned *cnt, int q, unsigned n) {
   __shared__ unsigned seen;
   if (threadIdx.x == 0) {
-    __threadfence();
-    seen = atomicAdd(cnt + q, 1u);
-    if (seen == n - 1) cnt[q] = 0u;
-    __threadfence();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    seen = __hip_atomic_fetch_add(cnt + q, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (seen == n - 1) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      cnt[q] = 0u;
+    }
   }
   __syncthreads();
   return seen == n - 1;
@@ -44,8 +54,24 @@ __device__ __forceinline__ void chunk_range(int N, int c, int C, int &i0, int &i
   i1 = min(i0 + per, N);
 }
 
+// partial sums of row q -> its inner product, in every thread
+__device__ __forceinline__ double2 sum_dots(const double2 *part, int q, int C, double *sh) {
+  double2 t = make_double2(0.0, 0.0);
+  if (threadIdx.x < C) t = part[(size_t)q * C + threadIdx.x];
+  t.x = block_sum(t.x, sh);
+  t.y = block_sum(t.y, sh);
+  return t;
+}
+static_assert(DOT_CHUNKS <= BS, "a thread per partial sum");
+// the same of a sum of squares -> its root
+__device__ __forceinline__ double sum_norm(const double *part, int r, int C, double *sh) {
+  double s = 0.0;
+  for (int i = threadIdx.x; i < C; i += BS) s += part[(size_t)r * C + i];
+  return sqrt(block_sum(s, sh));
+}
+
 // h[j nrhs + r] = <V_j^r, w^r>, also to hp (host memory): grid (chunks, vectors x right-hand
-// sides)
+// sides).  cnt NULL: only the partial sums, which k_sum_dots completes.
 __global__ void __launch_bounds__(BS)
     k_dots(const double2 *__restrict__ V, int nrhs, int N, const double2 *__restrict__ w,
            double2 *__restrict__ part, unsigned *__restrict__ cnt, double2 *__restrict__ h,
@@ -65,28 +91,45 @@ __global__ void __launch_bounds__(BS)
   si = block_sum(si, sh);
   if (C > 1) {
     if (threadIdx.x == 0) part[(size_t)jr * C + c] = make_double2(sr, si);
-    if (!last_block(cnt, jr, C)) return;
-    double2 t = make_double2(0.0, 0.0);
-    if (threadIdx.x < C) t = part[(size_t)jr * C + threadIdx.x];
-    sr = block_sum(t.x, sh);
-    si = block_sum(t.y, sh);
+    if (!cnt || !last_block(cnt, jr, C)) return;
+    const double2 t = sum_dots(part, jr, C, sh);
+    sr = t.x;
+    si = t.y;
   }
   if (threadIdx.x == 0) h[jr] = hp[jr] = make_double2(sr, si);
 }
 
-// |w|^2 of the block's chunk -> norm of right-hand side r
+// a block a row
+__global__ void __launch_bounds__(BS)
+    k_sum_dots(const double2 *__restrict__ part, int C, double2 *__restrict__ h,
+               double2 *__restrict__ hp) {
+  __shared__ double sh[BS / 64];
+  const int q = blockIdx.x;
+  const double2 t = sum_dots(part, q, C, sh);
+  if (threadIdx.x == 0) h[q] = hp[q] = t;
+}
+__global__ void __launch_bounds__(BS)
+    k_sum_norms(const double *__restrict__ part, int C, double *__restrict__ nrm,
+                double *__restrict__ hp) {
+  __shared__ double sh[BS / 64];
+  const int r = blockIdx.x;
+  const double n = sum_norm(part, r, C, sh);
+  if (threadIdx.x == 0) nrm[r] = hp[r] = n;
+}
+
+// |w|^2 of the block's chunk -> norm of right-hand side r (cnt NULL: k_sum_norms completes it)
 __device__ __forceinline__ void norm_end(double s, double *sh, double *part, unsigned *cnt, int r,
                                          double *nrm, double *hp) {
   const int C = gridDim.x, c = blockIdx.x;
   s = block_sum(s, sh);
   if (C > 1) {
     if (threadIdx.x == 0) part[(size_t)r * C + c] = s;
-    if (!last_block(cnt, r, C)) return;
-    s = 0.0;
-    for (int i = threadIdx.x; i < C; i += BS) s += part[(size_t)r * C + i];
-    s = block_sum(s, sh);
+    if (!cnt || !last_block(cnt, r, C)) return;
+    s = sum_norm(part, r, C, sh);
+  } else {
+    s = sqrt(s);
   }
-  if (threadIdx.x == 0) nrm[r] = hp[r] = sqrt(s);
+  if (threadIdx.x == 0) nrm[r] = hp[r] = s;
 }
 
 // w^r += sign sum_j h[j nrhs + r] V_j^r, and with NORM |w^r|: grid (chunks, right-hand sides)
@@ -221,6 +264,32 @@ static int chunks_for(int N, int limit) {
   return c < 1 ? 1 : (c > limit ? limit : c);
 }
 
+// counters of a reduction of grid g, NULL where a launch of its own completes it
+static unsigned *counters(const fmbh_vecws *ws, dim3 g) {
+  return (size_t)g.x * g.y <= kOneLaunch ? ws->cnt : NULL;
+}
+static int sum_norms(dim3 g, const fmbh_vecws *ws, hipStream_t st) {
+  if (g.x == 1 || counters(ws, g)) return FMB_OK;
+  hipLaunchKernelGGL(k_sum_norms, dim3(g.y), dim3(BS), 0, st, (const double *)ws->part, (int)g.x,
+                     ws->nrm, ws->hpn);
+  FMB_LAUNCH_CHECK();
+  return FMB_OK;
+}
+static int dots(const double2 *V, int nv, const double2 *w, int nrhs, int N, const fmbh_vecws *ws,
+                fmb_c64 *h, fmb_c64 *hp, hipStream_t st) {
+  const dim3 g(chunks_for(N, DOT_CHUNKS), nv * nrhs);
+  double2 *part = (double2 *)ws->part;
+  unsigned *cnt = counters(ws, g);
+  hipLaunchKernelGGL(k_dots, g, dim3(BS), 0, st, V, nrhs, N, w, part, cnt, (double2 *)h,
+                     (double2 *)hp);
+  FMB_LAUNCH_CHECK();
+  if (g.x == 1 || cnt) return FMB_OK;
+  hipLaunchKernelGGL(k_sum_dots, dim3(g.y), dim3(BS), 0, st, (const double2 *)part, (int)g.x,
+                     (double2 *)h, (double2 *)hp);
+  FMB_LAUNCH_CHECK();
+  return FMB_OK;
+}
+
 // Layout of the vector workspace: partial sums, counters, h1, h2, norms; the host mirror holds
 // h1, h2, norms
 static size_t ws_part(int nv, int nrhs, int N) {
@@ -255,37 +324,35 @@ extern "C" int fmbh_vecws_init(fmbh_vecws *ws, void *dev, void *host, int nv, in
 
 // One Arnoldi step: w -= V (V^H w) twice (classical Gram-Schmidt with one reorthogonalisation),
 // |w|, V_nv = w / |w|.  The inner products of both passes and the norms reach the host mirror; the
-// caller waits for the stream once.  A small solve is bound by launches and waits: five launches and
-// no transfers take 0.06 ms a step beside the product at 1,280 triangles, ten launches, six
-// transfers, three allocations and eleven waits took 0.19 ms (its whole solve 7.5 ms then, 4.2
-// now; 0.5 ms of the difference are M2L's).
+// caller waits for the stream once.  A small solve is bound by launches and waits: five to eight
+// launches and no transfers, 21 us over ten vectors of 1,280 elements, where ten launches, six
+// transfers, three allocations and eleven waits took 0.19 ms.
 extern "C" int fmbh_arnoldi(fmb_c64 *d_V, int nv, fmb_c64 *d_w, int nrhs, int N,
                             const fmbh_vecws *ws, void *stream) {
   hipStream_t st = (hipStream_t)stream;
-  double2 *V = (double2 *)d_V, *w = (double2 *)d_w, *part = (double2 *)ws->part;
-  const dim3 gd(chunks_for(N, DOT_CHUNKS), nv * nrhs), gv(chunks_for(N, UPD_CHUNKS), nrhs), blk(BS);
-  hipLaunchKernelGGL(k_dots, gd, blk, 0, st, V, nrhs, N, w, part, ws->cnt, (double2 *)ws->h1,
-                     (double2 *)ws->hp1);
-  FMB_LAUNCH_CHECK();
+  double2 *V = (double2 *)d_V, *w = (double2 *)d_w;
+  const dim3 gv(chunks_for(N, UPD_CHUNKS), nrhs), blk(BS);
+  int rc;
+  if ((rc = dots(V, nv, w, nrhs, N, ws, ws->h1, ws->hp1, st))) return rc;
   hipLaunchKernelGGL(k_gemv<false>, gv, blk, 0, st, V, nv, (const double2 *)ws->h1, w, nrhs, N,
                      -1.0, nullptr, nullptr, nullptr, nullptr);
   FMB_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_dots, gd, blk, 0, st, V, nrhs, N, w, part, ws->cnt, (double2 *)ws->h2,
-                     (double2 *)ws->hp2);
-  FMB_LAUNCH_CHECK();
+  if ((rc = dots(V, nv, w, nrhs, N, ws, ws->h2, ws->hp2, st))) return rc;
   hipLaunchKernelGGL(k_gemv<true>, gv, blk, 0, st, V, nv, (const double2 *)ws->h2, w, nrhs, N,
-                     -1.0, (double *)ws->part, ws->cnt, ws->nrm, ws->hpn);
+                     -1.0, (double *)ws->part, counters(ws, gv), ws->nrm, ws->hpn);
   FMB_LAUNCH_CHECK();
+  if ((rc = sum_norms(gv, ws, st))) return rc;
   return fmbh_unit(d_w, ws->nrm, d_V + (size_t)nv * nrhs * N, nrhs, N, stream);
 }
 
 extern "C" int fmbh_resid(const fmb_c64 *d_b, const fmb_c64 *d_w, fmb_c64 *d_r, int nrhs, int N,
                           const fmbh_vecws *ws, void *stream) {
-  hipLaunchKernelGGL(k_resid, dim3(chunks_for(N, UPD_CHUNKS), nrhs), dim3(BS), 0, (hipStream_t)stream,
-                     (const double2 *)d_b, (const double2 *)d_w, (double2 *)d_r, N,
-                     (double *)ws->part, ws->cnt, ws->nrm, ws->hpn);
+  const dim3 g(chunks_for(N, UPD_CHUNKS), nrhs);
+  hipLaunchKernelGGL(k_resid, g, dim3(BS), 0, (hipStream_t)stream, (const double2 *)d_b,
+                     (const double2 *)d_w, (double2 *)d_r, N, (double *)ws->part, counters(ws, g),
+                     ws->nrm, ws->hpn);
   FMB_LAUNCH_CHECK();
-  return FMB_OK;
+  return sum_norms(g, ws, (hipStream_t)stream);
 }
 
 extern "C" int fmbh_unit(const fmb_c64 *d_x, const double *d_nrm, fmb_c64 *d_y, int nrhs, int N,
