@@ -481,15 +481,20 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))
   T *X = (T *)smem;
   T *accr = X + (size_t)((p * (p + 1)) >> 1) * kL, *acci = accr + (size_t)p2 * SA;
   const int tid = threadIdx.x, wave = uni(tid >> 6), lane = tid & 63, li = lane & 15;
-  // workgroups are dealt to the 8 XCDs in turn; XCD x takes a contiguous range of the items, so
-  // that the groups whose sources overlap share its L2
+  // workgroups are dealt to the 8 XCDs in turn; XCD x takes a contiguous range of the groups, so
+  // that those whose sources overlap share its L2.  The blocks of right-hand sides of a group lie
+  // beside each other (FP64, 64 right-hand sides: 2% faster than one after the other) unless the
+  // last is short: an XCD deals its workgroups to four shader engines in turn, and the short ones
+  // would meet the same engines every time (33 right-hand sides took as long as 64).
   int g, jj, rb;
   {
-    const unsigned items = (unsigned)a.ngroups * a.J * a.nrb, per = (items + 7) / 8;
-    const unsigned it = (block & 7) * per + (block >> 3);
-    if (it >= items || (block >> 3) >= per) return;
-    rb = it % a.nrb;
-    const unsigned q = it / a.nrb;
+    const unsigned items = (unsigned)a.ngroups * a.J, per = (items + 7) / 8;
+    const unsigned i = block >> 3;
+    if (i >= per * a.nrb) return;
+    const bool even = a.nrhs % a.R == 0;
+    rb = even ? i % a.nrb : i / per;
+    const unsigned q = (block & 7) * per + (even ? i / a.nrb : i % per);
+    if (q >= items) return;
     jj = q % a.J;
     g = q / a.J;
   }
@@ -795,7 +800,7 @@ template <typename T, int W> int launch_ts(const fmbh_ts_job *jobs, int n, int n
     double longest = 0.0;
     for (int i = 0; i < n; i++) {
       const long long J = split(i, b);
-      x += (wg[i] * J + 7) / 8;
+      x += (lv.a[i].ngroups * J + 7) / 8 * lv.a[i].nrb;
       longest = per[i] / J > longest ? per[i] / J : longest;
     }
     return ((x + 32 * fit - 1) / (32 * fit)) * (2.0 + longest);
@@ -812,7 +817,7 @@ template <typename T, int W> int launch_ts(const fmbh_ts_job *jobs, int n, int n
     }
   for (int i = 0; i < n; i++) {
     lv.a[i].J = (int)split(i, batches);
-    total += 8 * ((wg[i] * lv.a[i].J + 7) / 8);
+    total += 8 * (((long long)lv.a[i].ngroups * lv.a[i].J + 7) / 8) * lv.a[i].nrb;
     if (total > 0x7fffffffLL) return fmb_set_error(FMB_ERR_RANGE, "M2L grid too large");
     lv.end[i] = (unsigned)total;
   }

@@ -1,0 +1,39 @@
+"""Blocks of right-hand sides of the target-stationary M2L (csrc/hip/rcr_ts.hip):
+a short last block, whose workgroups end early, beside full ones."""
+import pytest
+import torch
+
+import fmbem_gpu_c_amd as F
+from conftest import wavenumber
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def tree():
+    return F.Tree(F.Mesh.ellipsoid(23, 0.1, 0.0875, 0.125, seed=3), depth=5)
+
+
+def _fine_m2l(plan, nrhs, prec):
+    """Milliseconds of levels 4 and 5, the best of five."""
+    x = torch.randn((nrhs, plan.n), dtype=torch.complex128, device="cuda")
+    plan.set_timing(True)
+    best = []
+    for _ in range(5):
+        plan.matvec(x, prec=prec)
+        best.append(plan.timing()[1][4:6])
+    plan.set_timing(False)
+    return sum(min(t) for t in zip(*best))
+
+
+@pytest.mark.parametrize("prec", [F.FMB_FP64, F.FMB_MIXED])
+def test_short_block_costs_less_than_a_full_one(tree, prec):
+    """Orders 14: 33 right-hand sides are a block of 32 and one of 1, three
+    batches of 16 vectors a pair where 64 take four.  Under 0.85 of the time
+    of 64: where the short blocks' workgroups all met the same shader engines,
+    the others took as long as for 64 (measured 0.98 to 1.06; 0.63 now)."""
+    pl = F.Plan(tree, wavenumber(1500.0), precision=F.FMB_MIXED, nrhs_max=64, serial_levels=1,
+                p_rule=F.PRULE_EXPLICIT, p_levels=[0, 0, 16, 14, 14, 14])
+    few, full = _fine_m2l(pl, 33, prec), _fine_m2l(pl, 64, prec)
+    print("33: %.3f ms, 64: %.3f ms" % (few, full), flush=True)
+    assert few < 0.85 * full
