@@ -22,6 +22,7 @@ RULE_COLLAPSED, RULE_GAUSS7 = 0, 1
 COAX_RR, COAX_SR = 0, 1
 RCR_AUTO, RCR_VALU = 0, 1
 RCR_MODE_RULE, RCR_MODE_LDS, RCR_MODE_GWS, RCR_MODE_LDSP, RCR_MODE_LDSO = 0, 1, 2, 3, 4
+RCR_MODE_TS = 5
 
 
 class FmbError(RuntimeError):
@@ -134,6 +135,8 @@ _SIGS = {
                                        ctypes.c_int, ctypes.c_double, ctypes.c_int, _vp, _vp]),
     "fmb_plan_tile_shape": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                            _vp, _vp, _vp, _vp, _vp, _vp]),
+    "fmb_plan_launch_shape": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                             ctypes.c_int, _vp, _vp, _vp, _vp, _vp]),
     "fmb_plan_wavenumber": (ctypes.c_int, [_vp, _vp]),
     "fmb_sweep_guess": (ctypes.c_int, [_vp, ctypes.c_double, _vp, _vp, ctypes.c_int, _vp, _vp]),
     "fmb_gmres": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_double,
@@ -405,6 +408,15 @@ class Plan:
                                          ctypes.byref(v[3]), ctypes.byref(v[4]),
                                          ctypes.byref(ms)))
         return tuple(x.value for x in v) + (ms.value,)
+
+    def launch_shape(self, kind, level, nrhs, prec=FMB_FP64):
+        """(mode, nt, mt, waves per workgroup, split-BF16 rotations) of the form
+        that the translation takes in a pass of nrhs right-hand sides
+        (fmb_plan_launch_shape)."""
+        v = [ctypes.c_int() for _ in range(5)]
+        _check(lib().fmb_plan_launch_shape(self.h, kind, level, prec, nrhs,
+                                           *[ctypes.byref(x) for x in v]))
+        return tuple(x.value for x in v)
 
     def _nrhs(self, t, name, like=None):
         """Vectors in t (checked against the plan's element count and

@@ -1352,3 +1352,29 @@ int fmb_plan_tile_shape(const fmb_plan *pl, int kind, int level, int prec, int *
   if (ms) *ms = tb->tuned_ms[op];
   return FMB_OK;
 }
+
+int fmb_plan_launch_shape(const fmb_plan *pl, int kind, int level, int prec, int nrhs,
+                          int *mode, int *nt, int *mt, int *nw, int *bf) {
+  if (!pl || !pl->ready || kind < 0 || kind > 2 || level < 2 || level > pl->tree->lmax ||
+      (kind && level < 3) || nrhs < 1 || nrhs > pl->nrhs_max)
+    return fmb_set_error(FMB_ERR_ARG, "fmb_plan_launch_shape: invalid arguments");
+  const int op = (prec == FMB_MIXED && pl->nops == 2) ? 1 : 0;
+  const fmb_rcr_tab *tb = &pl->rcr[kind][level];
+  fmbh_rcr_job j;
+  memset(&j, 0, sizeof(j));
+  if (kind == 0 && tb->mode[op] && ts_ready(pl, op, level, nrhs)) {
+    j.mode = FMB_RCR_MODE_TS;
+    j.nt = 2;
+    j.nw = pl->ops[op].prec == FMB_FP64 ? FMBH_TS_WAVES64 : FMBH_TS_WAVES32;
+  } else if (tb->mode[op]) {
+    j.nchunks = (kind == 0 ? tb : &pl->rcr[1][level])->nchunks;
+    j.chunk_pairs = RCR_CHUNK;
+    job_shape(tb, op, nrhs, &j);
+  }
+  if (mode) *mode = j.mode;
+  if (nt) *nt = j.nt;
+  if (mt) *mt = j.mt;
+  if (nw) *nw = j.nw;
+  if (bf) *bf = j.bf;
+  return FMB_OK;
+}

@@ -164,6 +164,9 @@ typedef struct fmb_plan fmb_plan;
 #define FMB_RCR_MODE_GWS 2  /* batch in a global workspace, persistent grid */
 #define FMB_RCR_MODE_LDSP 3 /* batch in LDS, persistent grid               */
 #define FMB_RCR_MODE_LDSO 4 /* as LDSP, with the bucket's operators in LDS  */
+#define FMB_RCR_MODE_TS 5   /* M2L by target groups, their sums in LDS
+                               (reported by fmb_plan_launch_shape; cannot be
+                               requested)                                  */
 
 typedef struct fmb_plan_params {
   double k;                  /* wavenumber (rad/m)                          */
@@ -256,15 +259,18 @@ int fmb_plan_retune(fmb_plan *pl, double k, const fmb_c64 *robin, void *stream);
  * tiles per batch nt (8 nt vectors), row tiles per unit mt, waves per
  * workgroup nw (4 or 8), bf = 1 where the rotations run in split-BF16, and
  * with autotune the timed milliseconds of one launch (else 0).  Any output
- * pointer may be NULL.  For M2L this is the shape of the offset-batched
- * kernel; levels of order 16 and less whose shape is left to the rule or the
- * autotuner (rcr_mode, waves, ldso and m2l_tile at their defaults) run
- * target-stationary instead where that is faster (csrc/hip/rcr_ts.hip).  A
- * shape of the fixed rule (autotune and waves 0) names the 4-wave form: high
- * orders and launches of few workgroups run its 8-wave form
- * (csrc/host/rcr.c). */
+ * pointer may be NULL.  This is the shape of the fixed rule or the autotuner;
+ * fmb_plan_launch_shape names the form that a pass takes. */
 int fmb_plan_tile_shape(const fmb_plan *pl, int kind, int level, int prec, int *mode,
                         int *nt, int *mt, int *nw, int *bf, double *ms);
+/* Form of that translation in a pass of nrhs (1 .. nrhs_max) right-hand sides,
+ * forward or transposed, as above: with waves and autotune 0, high orders and
+ * launches of few workgroups take 8 waves (csrc/host/rcr.c), and M2L levels of
+ * order 16 and less whose shape is not requested (rcr_mode, waves, ldso and
+ * m2l_tile at their defaults) run target-stationary where that is faster
+ * (csrc/hip/rcr_ts.hip): mode FMB_RCR_MODE_TS, nt 2, mt 0. */
+int fmb_plan_launch_shape(const fmb_plan *pl, int kind, int level, int prec, int nrhs,
+                          int *mode, int *nt, int *mt, int *nw, int *bf);
 /* Wavenumber of the operator the plan holds (0 after a failed retune). */
 int fmb_plan_wavenumber(const fmb_plan *pl, double *k);
 /* Device bytes held by the plan. */
