@@ -870,6 +870,7 @@ typedef struct {
 } tuned_t;
 #define TUNE_CACHE 4096
 #define TUNE_MAGIC "fmbem-rcr-tile-v2"
+#define TUNE_TS 3 /* kind of the target-stationary M2L's entries */
 static tuned_t tune_cache[TUNE_CACHE];
 static int tune_cached, tune_loaded;
 static char tune_dev[64];
@@ -941,6 +942,10 @@ static void tune_load(void) {
                &v.shape.nt, &v.shape.mt, &v.shape.nw, &v.shape.bf, &v.ms) != 15)
       continue;
     if (strcmp(magic, TUNE_MAGIC) || strcmp(dev, tune_dev)) continue;
+    if (v.kind == TUNE_TS) { /* a time only */
+      if (v.shape.mode == FMB_RCR_MODE_TS && v.ms > 0) cache_store(&v);
+      continue;
+    }
     /* only shapes this build can launch; split-BF16 only where allowed */
     if (v.shape.mode < FMBH_RCR_LDS || v.shape.mode > FMBH_RCR_LDSO || v.shape.nt < 1 ||
         v.shape.nt > 2 || (v.shape.nw != 4 && v.shape.nw != 8) || v.kind < 0 || v.kind > 2 ||
@@ -1103,6 +1108,25 @@ static int autotune(fmb_plan *pl, int op, void *stream) {
   return rc;
 }
 
+/* A tuned plan's M2L runs target-stationary where that is faster than the
+ * tuned shape too, by its own time at nrhs_max right-hand sides (timed, or
+ * from the cache). */
+static int ts_tuned(fmb_plan *pl, int op, int l, void *stream) {
+  fmb_rcr_tab *tb = &pl->rcr[0][l];
+  if (!(tb->tuned_ms[op] > 0) || !ts_ready(pl, op, l, pl->nrhs_max)) return FMB_OK;
+  tuned_t key = {pl->ops[op].prec, TUNE_TS, tb->pin, tb->pout, tb->nchunks, pl->nrhs_max, 0,
+                 {FMB_RCR_MODE_TS, 2, 0, 0, 0}, 0.0f}, hit;
+  if (cache_find(&key, &hit)) {
+    key.ms = hit.ms;
+  } else {
+    int rc = time_run(pl, op, 0, l, stream, &key.ms);
+    if (rc) return rc;
+    cache_put(&key);
+  }
+  if (key.ms >= tb->tuned_ms[op]) tb->ts_slots[op] = 0;
+  return FMB_OK;
+}
+
 /* The tile-major M2L order keeps a tile's sources in its XCD's L2.  It pays
  * where the level's FP64 source coefficients (boxes x right-hand sides x
  * p^2 x 16 bytes) outgrow the GPU's 256 MB last-level (Infinity) cache, the
@@ -1169,11 +1193,13 @@ int fmbx_rcr_setup(fmb_plan *pl, void *stream) {
   if (pl->prm.autotune && pl->prm.rcr_path != FMB_RCR_VALU)
     for (int op = 0; op < pl->nops; op++)
       if ((rc = autotune(pl, op, stream))) return rc;
-  /* (last: the autotuner times the offset-batched shapes) */
+  /* (last: the autotuner's shapes are those of the offset-batched kernels) */
   if (pl->prm.rcr_path != FMB_RCR_VALU)
     for (int op = 0; op < pl->nops; op++)
-      for (int l = 2; l <= L; l++)
+      for (int l = 2; l <= L; l++) {
         if ((rc = ts_setup(pl, l, &pl->rcr[0][l], op, stream))) return rc;
+        if (pl->prm.autotune && (rc = ts_tuned(pl, op, l, stream))) return rc;
+      }
   return FMB_OK;
 }
 
