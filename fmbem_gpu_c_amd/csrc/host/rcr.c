@@ -556,19 +556,23 @@ static int ts_sched(int prec, int p, int **d_out, void *stream) {
 }
 
 /* Whether an M2L of order p over npairs pairs and nrhs right-hand sides runs
- * target-stationary.  Measured against the offset-batched kernels on the
- * 20,480-triangle sphere, speedup at 1 / 3 / 16 right-hand sides:
- *   FP64, 170,400 and 400,056 pairs: order 14 1.32 / 1.45 / 1.9, order 16
- *     1.1-1.2 / 1.29 / 1.46, orders 2 to 12 1.2-1.7; 9,744 pairs: 1.2-1.5;
- *     2,504 pairs 0.9-1.2.  Order 18 (327,680 triangles) 0.78.
- *   FP32: order 14 1.15-1.2 / 1.25 / 1.6-1.8, order 16 0.92 / 1.0 / 1.3,
- *     orders 2 to 12 1.15-1.6; at or under 36,192 vectors 0.85-1.1.
+ * target-stationary.  Measured against the offset-batched kernels on trees of
+ * 3 to 6 levels (926 to 400,056 pairs a level), as speedups:
+ *   FP64, up to 16 right-hand sides: orders 2 to 15 1.1-2.0 (the least on level
+ *     2, whose 2,504 pairs had 0.9-1.2 before the launch's split fitted them),
+ *     order 16 1.02-1.7.  17 to 100: 1.0-2.0; the worst levels 0.96 (order 16,
+ *     17 right-hand sides) and 0.93 (level 2, 33).  Order 18 0.78.
+ *   FP32: orders 2 to 14 1.1-2.3, at or under 36,192 vectors 0.85-1.1; order 15
+ *     from 16 right-hand sides on 1.0-1.5, order 16 1.1-1.3 where the batches of
+ *     a pair fill up, but 0.85-0.98 at 17 to 29 right-hand sides, two batches a
+ *     pair, 0.92-1.0 with fewer than 16, and 0.78-0.92 on a level of 926 pairs.
  * (Above order 16 the batch and the sums no longer fit the LDS at a useful
  * size.) */
 static int ts_use(int prec, int p, int npairs, int nrhs) {
   if (p > FMBH_TS_PMAX) return 0;
   if (prec == FMB_FP64) return 1;
-  return (p <= 14 || nrhs >= 16) && (double)npairs * nrhs >= 40000;
+  if ((double)npairs * nrhs < 40000 || (p > 14 && nrhs < 16)) return 0;
+  return p < 16 || (npairs >= 4000 && (nrhs == 16 || nrhs >= 30));
 }
 
 /* sums of a workgroup: at most 32 target vectors in 160 KB of LDS, or in the
@@ -582,8 +586,8 @@ static int ts_slots(int prec, int p) {
 
 /* schedule, pair lists and coaxial tables of the target-stationary M2L at
  * level l, where its shape was not requested otherwise.  Two lists: groups of
- * as many targets as fill the slots at nrhs_max right-hand sides, and at one
- * (passes with fewer right-hand sides than the plan holds). */
+ * as many targets as fill the slots at the most right-hand sides that run so,
+ * and at one (passes with fewer right-hand sides than the plan holds). */
 static int ts_setup(fmb_plan *pl, int l, fmb_rcr_tab *tb, int op, void *stream) {
   const fmb_tree *t = pl->tree;
   const fmb_plan_params *prm = &pl->prm;
@@ -595,11 +599,13 @@ static int ts_setup(fmb_plan *pl, int l, fmb_rcr_tab *tb, int op, void *stream) 
   if (prm->rcr_mode || prm->waves || prm->ldso || (prm->split_bf16 && op == 1) ||
       prm->m2l_tile != RCR_TILE || prm->m2l_tile_min_mb != RCR_TILE_MIN_MB)
     return FMB_OK;
-  if (!t->npairs[l] || !ts_use(o->prec, p, t->npairs[l], pl->nrhs_max)) return FMB_OK;
+  int most = pl->nrhs_max; /* the most right-hand sides that a pass may run so */
+  while (most && !(t->npairs[l] && ts_use(o->prec, p, t->npairs[l], most))) most--;
+  if (!most) return FMB_OK;
   const int S = ts_slots(o->prec, p);
   tb->ts_slots[op] = S;
   for (int i = 0; i < (pl->nrhs_max > 1 ? 2 : 1); i++) {
-    const int R = i || pl->nrhs_max == 1 ? 1 : (pl->nrhs_max < S ? pl->nrhs_max : S);
+    const int R = i || pl->nrhs_max == 1 ? 1 : (most < S ? most : S);
     tb->ts_tgrp[op][i] = S / R;
     const size_t bytes = sizeof(int) * (2 * (size_t)t->npairs[l] +
                                         (size_t)FMB_NCLASS * (t->nbox[l] / (S / R) + 1));

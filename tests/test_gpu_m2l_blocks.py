@@ -37,3 +37,24 @@ def test_short_block_costs_less_than_a_full_one(tree, prec):
     few, full = _fine_m2l(pl, 33, prec), _fine_m2l(pl, 64, prec)
     print("33: %.3f ms, 64: %.3f ms" % (few, full), flush=True)
     assert few < 0.85 * full
+
+
+def test_half_empty_batches_of_order_16(tree):
+    """FP32, order 16: 17 to 29 right-hand sides would leave the second batch of
+    a pair's vectors too empty, and level 2 has too few pairs; a plan that holds
+    such a count still takes 16 target-stationary.  Both forms are the same
+    operator: FP32 1e-6 as in the tests of the kernels (the order of the sums)."""
+    kw = dict(precision=F.FMB_MIXED, p_rule=F.PRULE_EXPLICIT, p_levels=[0, 0, 16, 16, 16, 16])
+    k = wavenumber(1500.0)
+    for nmax in (24, 33):
+        pl = F.Plan(tree, k, nrhs_max=nmax, **kw)
+        ref = F.Plan(tree, k, nrhs_max=nmax, m2l_tile=255, **kw)
+        for nrhs in (1, 15, 16, 17, 24, 29, 30, 33):
+            if nrhs > nmax:
+                continue
+            for l in (2, 3, 4, 5):
+                ts = l > 2 and nrhs in (16, 30, 33)
+                assert (pl.launch_shape(0, l, nrhs, F.FMB_MIXED)[0] == F.RCR_MODE_TS) == ts
+            x = torch.randn((nrhs, pl.n), dtype=torch.complex128, device="cuda")
+            a, b = pl.matvec_parts(x, 2, prec=F.FMB_MIXED), ref.matvec_parts(x, 2, prec=F.FMB_MIXED)
+            assert float(torch.linalg.norm(a - b) / torch.linalg.norm(b)) < 1e-6, (nmax, nrhs)
