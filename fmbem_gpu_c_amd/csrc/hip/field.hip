@@ -54,6 +54,31 @@ __global__ void __launch_bounds__(kT)
 #pragma unroll
     for (int r = 0; r < R; r++) acc[i][r] = make_double2(0.0, 0.0);
   }
+  if constexpr (P == 1) {
+    for (int j = blockIdx.y * kT + threadIdx.x; j < N; j += nsl * kT) {
+      const double *gj = geo + 8 * (size_t)j;
+      const double dx = y[0][0] - gj[0], dy = y[0][1] - gj[1], dz = y[0][2] - gj[2];
+      const bool close = dx * dx + dy * dy + dz * dz < ratio * ratio * gj[7] * gj[7];
+      double2 o[4];
+      panel_sum(k, y[0], nz, tri + 9 * (size_t)j, gj + 3, gj[6], close ? quadn : quad,
+                close ? nqn : nq, o);
+      double2 g = o[1];
+      if (robin) {
+        const double2 sg = robin[j];
+        g.x -= sg.x * o[0].x - sg.y * o[0].y;
+        g.y -= sg.x * o[0].y + sg.y * o[0].x;
+      }
+      const int c = perm[j];
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        if (r < nr) {
+          const double2 v = x[(size_t)(r0 + r) * N + c];
+          acc[0][r].x += g.x * v.x - g.y * v.y;
+          acc[0][r].y += g.x * v.y + g.y * v.x;
+        }
+      }
+    }
+  } else
   for (int j = blockIdx.y * kT + threadIdx.x; j < N; j += nsl * kT) {
     const double *gj = geo + 8 * (size_t)j, *tr = tri + 9 * (size_t)j;
     double t[9], g8[8];
