@@ -46,3 +46,12 @@ def test_second_right_hand_side_adds_little(plan):
     one, two = (_us(plan, r, _shell(1000, 0.2, 0.5)) for r in (1, 2))
     print("one %.0f us, two %.0f us" % (one, two), flush=True)
     assert two < 1.4 * one
+
+
+def test_two_groups_of_right_hand_sides_share_their_launches(plan):
+    """64 points through the tree: eight right-hand sides are two groups of four
+    in the box-major sums, whose launches are a round of workgroups each.  Under
+    1.65 times four (measured 1.43; 1.92 with a launch for each group)."""
+    four, eight = (_us(plan, r, _shell(64, 0.2, 0.5), "fmm") for r in (4, 8))
+    print("four %.0f us, eight %.0f us" % (four, eight), flush=True)
+    assert eight < 1.65 * four
