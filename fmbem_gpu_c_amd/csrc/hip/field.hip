@@ -54,91 +54,92 @@ __global__ void __launch_bounds__(kT)
 #pragma unroll
     for (int r = 0; r < R; r++) acc[i][r] = make_double2(0.0, 0.0);
   }
-  if constexpr (P == 1) {
-    for (int j = blockIdx.y * kT + threadIdx.x; j < N; j += nsl * kT) {
-      const double *gj = geo + 8 * (size_t)j;
-      const double dx = y[0][0] - gj[0], dy = y[0][1] - gj[1], dz = y[0][2] - gj[2];
-      const bool close = dx * dx + dy * dy + dz * dz < ratio * ratio * gj[7] * gj[7];
-      double2 o[4];
-      panel_sum(k, y[0], nz, tri + 9 * (size_t)j, gj + 3, gj[6], close ? quadn : quad,
-                close ? nqn : nq, o);
-      double2 g = o[1];
-      if (robin) {
-        const double2 sg = robin[j];
-        g.x -= sg.x * o[0].x - sg.y * o[0].y;
-        g.y -= sg.x * o[0].y + sg.y * o[0].x;
-      }
-      const int c = perm[j];
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        if (r < nr) {
-          const double2 v = x[(size_t)(r0 + r) * N + c];
-          acc[0][r].x += g.x * v.x - g.y * v.y;
-          acc[0][r].y += g.x * v.y + g.y * v.x;
-        }
-      }
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  auto add = [&](int i, const double2 &S, const double2 &K, int j) {
+    double2 g = K;
+    if (robin) {
+      const double2 sg = robin[j];
+      g.x -= sg.x * S.x - sg.y * S.y;
+      g.y -= sg.x * S.y + sg.y * S.x;
     }
-  } else
-  for (int j = blockIdx.y * kT + threadIdx.x; j < N; j += nsl * kT) {
-    const double *gj = geo + 8 * (size_t)j, *tr = tri + 9 * (size_t)j;
-    double t[9], g8[8];
-    for (int a = 0; a < 9; a++) t[a] = tr[a];
-    for (int a = 0; a < 8; a++) g8[a] = gj[a];
-    const double lim = ratio * ratio * g8[7] * g8[7];
-    bool close[P];
-    double2 S[P], K[P];  // int G, int dG/dn_y
-#pragma unroll
-    for (int i = 0; i < P; i++) {
-      const double dx = y[i][0] - g8[0], dy = y[i][1] - g8[1], dz = y[i][2] - g8[2];
-      close[i] = dx * dx + dy * dy + dz * dz < lim;
-      S[i] = K[i] = make_double2(0.0, 0.0);
-    }
-    for (int q = 0; q < nq; q++) {  // (panel_sum's S and K)
-      const double *qq = quad + 4 * q;
-      const double w = qq[3] * g8[6];
-      double z[3];
-      for (int a = 0; a < 3; a++) z[a] = qq[0] * t[a] + qq[1] * t[3 + a] + qq[2] * t[6 + a];
-#pragma unroll
-      for (int i = 0; i < P; i++) {
-        const double d0 = y[i][0] - z[0], d1 = y[i][1] - z[1], d2 = y[i][2] - z[2];
-        const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2), ir = 1.0 / r;
-        double sn, cs;
-        sincos(k * r, &sn, &cs);
-        const double g0 = (1.0 / (4.0 * M_PI)) * ir, gr = cs * g0, gi = sn * g0;
-        const double wn = -w * ((d0 * g8[3] + d1 * g8[4] + d2 * g8[5]) * ir);
-        const double gpr = -gr * ir - k * gi, gpi = -gi * ir + k * gr;
-        S[i].x += w * gr;
-        S[i].y += w * gi;
-        K[i].x += wn * gpr;
-        K[i].y += wn * gpi;
-      }
-    }
-    const double2 sg = robin ? robin[j] : make_double2(0.0, 0.0);
     const int c = perm[j];
 #pragma unroll
-    for (int i = 0; i < P; i++) {
-      if (close[i]) {
-        double2 o[4];
-        panel_sum(k, y[i], nz, t, g8 + 3, g8[6], quadn, nqn, o);
-        S[i] = o[0];
-        K[i] = o[1];
-      }
-      double2 g = K[i];
-      if (robin) {
-        g.x -= sg.x * S[i].x - sg.y * S[i].y;
-        g.y -= sg.x * S[i].y + sg.y * S[i].x;
-      }
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        if (r < nr) {
-          const double2 v = x[(size_t)(r0 + r) * N + c];
-          acc[i][r].x += g.x * v.x - g.y * v.y;
-          acc[i][r].y += g.x * v.y + g.y * v.x;
-        }
+    for (int r = 0; r < R; r++) {
+      if (r < nr) {
+        const double2 v = x[(size_t)(r0 + r) * N + c];
+        acc[i][r].x += g.x * v.x - g.y * v.y;
+        acc[i][r].y += g.x * v.y + g.y * v.x;
       }
     }
+  };
+  for (int j0 = blockIdx.y * kT + 64 * w; j0 < N; j0 += nsl * kT) {
+    const int j = j0 + lane;
+    unsigned long long near[P];  // lanes whose panel is close to point i
+    if constexpr (P == 1) {
+      const double *gj = geo + 8 * (size_t)min(j, N - 1);
+      const double dx = y[0][0] - gj[0], dy = y[0][1] - gj[1], dz = y[0][2] - gj[2];
+      const bool close = dx * dx + dy * dy + dz * dz < ratio * ratio * gj[7] * gj[7];
+      near[0] = __ballot(j < N && close);
+      if (j < N && !close) {
+        double2 o[4];
+        panel_sum(k, y[0], nz, tri + 9 * (size_t)j, gj + 3, gj[6], quad, nq, o);
+        add(0, o[0], o[1], j);
+      }
+    } else {
+      const double *gj = geo + 8 * (size_t)min(j, N - 1), *tr = tri + 9 * (size_t)min(j, N - 1);
+      double t[9], g8[8];
+      for (int a = 0; a < 9; a++) t[a] = tr[a];
+      for (int a = 0; a < 8; a++) g8[a] = gj[a];
+      const double lim = ratio * ratio * g8[7] * g8[7];
+      double2 S[P], K[P];  // int G, int dG/dn_y
+      bool far[P];
+#pragma unroll
+      for (int i = 0; i < P; i++) {
+        const double dx = y[i][0] - g8[0], dy = y[i][1] - g8[1], dz = y[i][2] - g8[2];
+        const bool close = dx * dx + dy * dy + dz * dz < lim;
+        near[i] = __ballot(j < N && close);
+        far[i] = j < N && !close;
+        S[i] = K[i] = make_double2(0.0, 0.0);
+      }
+      for (int q = 0; q < nq; q++) {  // (panel_sum's S and K)
+        const double *qq = quad + 4 * q;
+        const double wt = qq[3] * g8[6];
+        double z[3];
+        for (int a = 0; a < 3; a++) z[a] = qq[0] * t[a] + qq[1] * t[3 + a] + qq[2] * t[6 + a];
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+          const double d0 = y[i][0] - z[0], d1 = y[i][1] - z[1], d2 = y[i][2] - z[2];
+          const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2), ir = 1.0 / r;
+          double sn, cs;
+          sincos(k * r, &sn, &cs);
+          const double g0 = (1.0 / (4.0 * M_PI)) * ir, gr = cs * g0, gi = sn * g0;
+          const double wn = -wt * ((d0 * g8[3] + d1 * g8[4] + d2 * g8[5]) * ir);
+          const double gpr = -gr * ir - k * gi, gpi = -gi * ir + k * gr;
+          S[i].x += wt * gr;
+          S[i].y += wt * gi;
+          K[i].x += wn * gpr;
+          K[i].y += wn * gpi;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < P; i++)
+        if (far[i]) add(i, S[i], K[i], j);
+    }
+    // panels of the refined rule, a point of the rule a lane (128 points next to
+    // a surface of 1,280 panels: 90 us with the rule by the lane of the panel, one
+    // point a workgroup; 137 with four points, one after the other)
+#pragma unroll
+    for (int i = 0; i < P; i++)
+      for (; near[i]; near[i] &= near[i] - 1) {
+        const int jj = j0 + __ffsll(near[i]) - 1;
+        const double *gj = geo + 8 * (size_t)jj;
+        for (int q = lane; q < nqn; q += 64) {
+          double2 o[4];
+          panel_sum(k, y[i], nz, tri + 9 * (size_t)jj, gj + 3, gj[6], quadn + 4 * q, 1, o);
+          add(i, o[0], o[1], jj);
+        }
+      }
   }
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
   for (int i = 0; i < P; i++)
 #pragma unroll
