@@ -365,9 +365,9 @@ extern "C" int fmbh_unit(const fmb_c64 *d_x, const double *d_nrm, fmb_c64 *d_y, 
 
 extern "C" int fmbh_zgemv_add(const fmb_c64 *d_V, int nv, const fmb_c64 *d_y, fmb_c64 *d_x,
                               int nrhs, int N, void *stream) {
-  hipLaunchKernelGGL(k_gemv<false>, dim3(chunks_for(N, UPD_CHUNKS), nrhs), dim3(BS), 0, (hipStream_t)stream,
-                     (const double2 *)d_V, nv, (const double2 *)d_y, (double2 *)d_x, nrhs, N, 1.0,
-                     nullptr, nullptr, nullptr, nullptr);
+  hipLaunchKernelGGL(k_gemv<false>, dim3(chunks_for(N, UPD_CHUNKS), nrhs), dim3(BS), 0,
+                     (hipStream_t)stream, (const double2 *)d_V, nv, (const double2 *)d_y,
+                     (double2 *)d_x, nrhs, N, 1.0, nullptr, nullptr, nullptr, nullptr);
   FMB_LAUNCH_CHECK();
   return FMB_OK;
 }

@@ -754,7 +754,9 @@ extern "C" int fmbh_field(const fmb_plan *pl, const fmb_c64 *x, int nrhs,
   hipStream_t st = (hipStream_t)stream;
   // one right-hand side: four points a workgroup; few points: their panels in
   // slices over several workgroups, so that the launch fills the device; the
-  // slices are summed in order
+  // slices are summed in order.  (81,920 panels at 32 points, 32 / 64 / 128
+  // slices: 149 / 133 / 130 us a call; at 1,280 to 81,920 panels and 4 to 6,000
+  // points 0.60 to 0.96 of the time of one point a workgroup in 32 slices.)
   const int P = nrhs == 1 && npts >= 4 ? 4 : 1, ng = (npts + P - 1) / P;
   const int nsl = ng >= kFieldSlicePts
                       ? 1
@@ -889,8 +891,8 @@ extern "C" int fmbh_field_order(const fmb_tree *t, const double *d_pts, int npts
   FMB_LAUNCH_CHECK();
   FMB_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, key, key2, idx, d_qperm, npts, 0, 36,
                                                    st));
-  hipLaunchKernelGGL(k_field_points, dim3((unsigned)((3 * (size_t)npts + 255) / 256)), dim3(256), 0, st, d_pts,
-                     d_qperm, npts, d_spts);
+  hipLaunchKernelGGL(k_field_points, dim3((unsigned)((3 * (size_t)npts + 255) / 256)), dim3(256),
+                     0, st, d_pts, d_qperm, npts, d_spts);
   FMB_LAUNCH_CHECK();
   return FMB_OK;
 }

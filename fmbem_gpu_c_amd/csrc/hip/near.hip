@@ -444,7 +444,10 @@ extern "C" int fmbh_l2p_near(const fmb_plan *pl, int op, fmb_c64 *y, int nrhs, i
   size_t lds = sizeof(int) * (size_t)(pl->near_max_ncol > 0 ? pl->near_max_ncol : 1);
   const unsigned long long *off = (const unsigned long long *)pl->d_near_off;
   if (o->prec == FMB_FP64)
-    hipLaunchKernelGGL((nrhs == 1 ? k_l2p_near<double, 1> : nrhs == 2 ? k_l2p_near<double, 2> : k_l2p_near<double, 4>), dim3(nb), dim3(256), lds, st,
+    hipLaunchKernelGGL((nrhs == 1   ? k_l2p_near<double, 1>
+                        : nrhs == 2 ? k_l2p_near<double, 2>
+                                    : k_l2p_near<double, 4>),
+                       dim3(nb), dim3(256), lds, st,
                        t->d_box_start, t->d_near_start, t->d_near_box,
                        pl->d_near_ncol, off, (const cplx<double> *)o->d_near,
                        (const cplx<double> *)o->d_L2P,
@@ -452,7 +455,10 @@ extern "C" int fmbh_l2p_near(const fmb_plan *pl, int op, fmb_c64 *y, int nrhs, i
                        (const cplx<double> *)o->d_xs, t->d_perm, (double2 *)y,
                        t->nelem, pL * pL, nrhs, parts);
   else
-    hipLaunchKernelGGL((nrhs == 1 ? k_l2p_near<float, 1> : nrhs == 2 ? k_l2p_near<float, 2> : k_l2p_near<float, 4>), dim3(nb), dim3(256), lds, st,
+    hipLaunchKernelGGL((nrhs == 1   ? k_l2p_near<float, 1>
+                        : nrhs == 2 ? k_l2p_near<float, 2>
+                                    : k_l2p_near<float, 4>),
+                       dim3(nb), dim3(256), lds, st,
                        t->d_box_start, t->d_near_start, t->d_near_box,
                        pl->d_near_ncol, off, (const cplx<float> *)o->d_near,
                        (const cplx<float> *)o->d_L2P,
@@ -473,14 +479,20 @@ extern "C" int fmbh_near_t(const fmb_plan *pl, int op, const void *near, const v
   const void *B = basis ? basis : o->d_P2M;
   const unsigned long long *off = (const unsigned long long *)pl->d_near_off;
   if (o->prec == FMB_FP64)
-    hipLaunchKernelGGL((nrhs == 1 ? k_near_t<double, 1> : nrhs == 2 ? k_near_t<double, 2> : k_near_t<double, 4>), dim3(nb), dim3(256), 0, st,
+    hipLaunchKernelGGL((nrhs == 1   ? k_near_t<double, 1>
+                        : nrhs == 2 ? k_near_t<double, 2>
+                                    : k_near_t<double, 4>),
+                       dim3(nb), dim3(256), 0, st,
                        t->d_box_start, t->d_near_start, t->d_near_box,
                        pl->d_near_ncol, off, (const cplx<double> *)A,
                        (const cplx<double> *)B, (const cplx<double> *)o->d_M[L],
                        (const cplx<double> *)o->d_xs, t->d_perm, (double2 *)y,
                        t->nelem, pL * pL, nrhs, parts);
   else
-    hipLaunchKernelGGL((nrhs == 1 ? k_near_t<float, 1> : nrhs == 2 ? k_near_t<float, 2> : k_near_t<float, 4>), dim3(nb), dim3(256), 0, st,
+    hipLaunchKernelGGL((nrhs == 1   ? k_near_t<float, 1>
+                        : nrhs == 2 ? k_near_t<float, 2>
+                                    : k_near_t<float, 4>),
+                       dim3(nb), dim3(256), 0, st,
                        t->d_box_start, t->d_near_start, t->d_near_box,
                        pl->d_near_ncol, off, (const cplx<float> *)A,
                        (const cplx<float> *)B, (const cplx<float> *)o->d_M[L],

@@ -31,7 +31,7 @@
 //    Sources, phases and operators of the first unit are loaded before the barrier.
 //  * Sums.  FP64: LDS double atomics (6 cycles a wave).  LDS float atomics take 177 cycles a wave
 //    here, so FP32 adds by plain read and write, one vector of a target after the other; no two
-//    waves share a row.
+//    waves share a row.  (Rows and sums: rcr_ts_rows.h.)
 //
 // What bounds it: instruction latency and the stages' serial chain at 16 waves per CU (FP32: two
 // workgroups of 8; FP64: one of 16); the vector and matrix pipes are busy about half the time.
@@ -458,8 +458,6 @@ struct TsLevels {
   TsArgs a[FMBH_TS_LEVELS];
 };
 
-// LDS: the batch rows, then the sums' real and imaginary planes [coefficient][slot].  Slot: place
-// of the target in the group x R + right-hand side.
 // The arguments of a workgroup's level and its place among the level's workgroups.  (One level has
 // its arguments to itself: choosing among levels costs the kernel 1%.)
 __device__ __forceinline__ const TsArgs &level_of(const TsArgs &a, unsigned &) { return a; }
@@ -470,6 +468,8 @@ __device__ __forceinline__ const TsArgs &level_of(const TsLevels &lv, unsigned &
   return lv.a[i];
 }
 
+// LDS: the batch rows, then the sums' real and imaginary planes [coefficient][slot].  Slot: place
+// of the target in the group x R + right-hand side.
 template <typename T, int W, typename A>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4)))
     k_m2l_ts(A args) {
@@ -787,9 +787,10 @@ template <typename T, int W> int launch_ts(const fmbh_ts_job *jobs, int n, int n
   // Workgroups of a group (J): setting up and flushing costs one about two batches, and the last
   // round of workgroups may be nearly empty, so the batches of a workgroup, the same at each level,
   // have the least (rounds) x (2 + batches), and the most workgroups within 2% of it (an even
-  // finish).  (The host loop is at most 8,192 short steps.)  Against about 2,048 workgroups for every launch (FP64): level 4 of the 5,120-triangle
-  // sphere 131 -> 90 us (560 -> 248 workgroups), levels 6 and 5 of 20,480 with the levels beside
-  // them 1.85 -> 1.73 ms a product.
+  // finish).  The search takes two passes over J, at most the finest level's batches of a group:
+  // 32 vectors of 189 sources, 378.  Against about 2,048 workgroups for every launch (FP64): level 4
+  // of the 5,120-triangle sphere 131 -> 90 us (560 -> 248 workgroups), levels 6 and 5 of 20,480 with
+  // the levels beside them 1.85 -> 1.73 ms a product.
   const int cu = 160 * 1024 / (int)lds, fit = cu < 1 ? 1 : (cu < 16 / W ? cu : 16 / W);
   auto split = [&](int i, double b) {
     const long long J = (long long)(per[i] / b + 0.999);
