@@ -80,6 +80,7 @@ typedef struct fmb_opset {
    * and phases [343][2][ts_P] of the forward and the transposed pass        */
   void *d_ts_H, *d_ts_phase[2];
   int ts_hstride, ts_P;
+  double wide_share; /* share of M2L's work in levels of the 8-wave form      */
 } fmb_opset;
 
 /* one translation kind at one level on the matrix cores */
@@ -163,6 +164,7 @@ struct fmb_plan {
    * events ordering it against the fine M2L levels (NULL: one stream) */
   void *aux, *ev_up, *ev_aux, *ev_m2l[FMB_MAXLEV];
   int capturing;        /* set while a batch captures this plan's pass      */
+  int split;            /* set while the levels of a pass run on two streams */
   void *stream;
 };
 

@@ -619,7 +619,8 @@ int fmb_last_timing(const fmb_plan *pl, double *phase7, double *m2l16) {
  * with three right-hand sides 3.68 -> 3.42.
  * Inside a graph capture, a batch's or the caller's own, the levels stay on
  * the capturing stream (a fork there is not used, see graph_capture). */
-static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev, void *stream) {
+static int run_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev, int split,
+                      void *stream) {
   const int L = pl->tree->lmax, up = trans ? 2 : 1, down = trans ? 1 : 2;
   int (*run)(const fmb_plan *, int, int, int, int, void *) = trans ? fmbx_rcr_run_t : fmbx_rcr_run;
   int rc = FMB_OK;
@@ -629,7 +630,6 @@ static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev
     if ((rc = run(pl, op, 0, l, nrhs, st))) return rc;                                   \
     if (ev) fmbh_event_record(ev[5 + 2 * (l)], st);                                      \
   } while (0)
-  const int split = pl->aux && !pl->capturing && !fmbh_stream_capturing(stream);
   void *aux = pl->aux;
   if (split) {
     if ((rc = fmbh_event_record(pl->ev_up, stream))) return rc;
@@ -673,6 +673,13 @@ static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev
   if (ev) ACROSS(L, stream);
 #undef ACROSS
   return L > 2 ? run(pl, op, down, L, nrhs, stream) : FMB_OK;
+}
+
+static int translate_levels(fmb_plan *pl, int op, int trans, int nrhs, void **ev, void *stream) {
+  pl->split = pl->aux && !pl->capturing && !fmbh_stream_capturing(stream);
+  const int rc = run_levels(pl, op, trans, nrhs, ev, pl->split, stream);
+  pl->split = 0;
+  return rc;
 }
 
 /* phase events: 0 start, 1 after gather+P2M, 2 after M2M, 3 after M2L/L2L,

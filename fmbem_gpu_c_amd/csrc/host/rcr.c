@@ -351,27 +351,6 @@ static int wide_form(fmb_plan *pl, fmb_rcr_tab *tb, int op, const int *hoff, con
   return FMB_OK;
 }
 
-/* tile shape of one launch */
-static void job_shape(const fmb_rcr_tab *tb, int op, int nrhs, fmbh_rcr_job *j) {
-  j->mode = tb->mode[op];
-  j->bf = tb->bf[op];
-  const int v = 8 * tb->nt[op];
-  const long wgs = (long)j->nchunks * ((j->chunk_pairs * nrhs + v - 1) / v);
-  if (tb->d_sched8[op] && (tb->wide8[op] || wgs <= 128)) {
-    j->nt = tb->nt8[op];
-    j->mt = tb->mt8[op];
-    j->nw = 8;
-    j->sched = tb->d_sched8[op];
-    j->sched_len = tb->sched8_len[op];
-    return;
-  }
-  j->nt = tb->nt[op];
-  j->mt = tb->mt[op];
-  j->nw = tb->nw[op];
-  j->sched = tb->d_sched[op];
-  j->sched_len = tb->sched_len[op];
-}
-
 /* tile shapes, schedules and padded coaxial blocks of one translation;
  * C: the scaled coaxial matrices of each opset (ncoax of them, order P) */
 static int plan_tab(fmb_plan *pl, fmb_rcr_tab *tb, int pin, int pout,
@@ -671,6 +650,46 @@ static int ts_run(const fmb_plan *pl, int op, int l, int trans, int nrhs, void *
 static int ts_ready(const fmb_plan *pl, int op, int l, int nrhs) {
   return pl->rcr[0][l].ts_slots[op] &&
          ts_use(pl->ops[op].prec, pl->p[l], pl->tree->npairs[l], nrhs);
+}
+
+/* Whether an FP64 pass on two streams keeps to 4 waves in every launch.  The
+ * 8-wave forms fill a CU, so that little runs beside them: where the finest
+ * levels have no such form, what they win is less than what the streams then
+ * hide.  327,680 triangles, 8 to 16 kHz, nine right-hand sides, 4 against 8
+ * waves, with the share of M2L's work (pairs x order^3) in levels of the
+ * 8-wave form: 265.6 and 279.0 ms at 0.35, 326.2 and 341.0 at 0.38, 430.5 and
+ * 428.0 at 0.64, 700.1 and 683.7 at 0.67; 81,920 triangles 64.6 and 65.2 at
+ * 0.31, 153.2 and 144.4 at 0.60, 101.3 and 97.4 at 0.61.  One right-hand side:
+ * no difference at 0.35 and 0.38.  A target-stationary finest level fills the
+ * CUs itself (1.02 to 1.09 in favour of 8 waves); one stream has nothing to
+ * hide (351 ms with 8 waves, 368 with 4, at 0.38).  (FP32, whose batches take
+ * half the LDS, gains with 8 waves on either.) */
+static int narrow_pass(const fmb_plan *pl, int op, int nrhs, int split) {
+  const int L = pl->tree->lmax;
+  return split && pl->ops[op].prec == FMB_FP64 && nrhs > 1 && pl->ops[op].wide_share < 0.5 &&
+         !pl->rcr[0][L].wide8[op] && !ts_ready(pl, op, L, nrhs);
+}
+
+/* tile shape of one launch; split: of a pass on two streams */
+static void job_shape(const fmb_plan *pl, const fmb_rcr_tab *tb, int op, int nrhs, int split,
+                      fmbh_rcr_job *j) {
+  j->mode = tb->mode[op];
+  j->bf = tb->bf[op];
+  const int v = 8 * tb->nt[op];
+  const long wgs = (long)j->nchunks * ((j->chunk_pairs * nrhs + v - 1) / v);
+  if (tb->d_sched8[op] && (wgs <= 128 || (tb->wide8[op] && !narrow_pass(pl, op, nrhs, split)))) {
+    j->nt = tb->nt8[op];
+    j->mt = tb->mt8[op];
+    j->nw = 8;
+    j->sched = tb->d_sched8[op];
+    j->sched_len = tb->sched8_len[op];
+    return;
+  }
+  j->nt = tb->nt[op];
+  j->mt = tb->mt[op];
+  j->nw = tb->nw[op];
+  j->sched = tb->d_sched[op];
+  j->sched_len = tb->sched_len[op];
 }
 
 /* M2L (M2L^T) of the finest levels that run target-stationary, in one launch;
@@ -1206,6 +1225,15 @@ int fmbx_rcr_setup(fmb_plan *pl, void *stream) {
         if ((rc = ts_setup(pl, l, &pl->rcr[0][l], op, stream))) return rc;
         if (pl->prm.autotune && (rc = ts_tuned(pl, op, l, stream))) return rc;
       }
+  for (int op = 0; op < pl->nops; op++) {
+    double all = 0.0, wide = 0.0;
+    for (int l = 2; l <= L; l++) {
+      const double w = (double)t->npairs[l] * pl->p[l] * pl->p[l] * pl->p[l];
+      all += w;
+      if (pl->rcr[0][l].wide8[op]) wide += w;
+    }
+    pl->ops[op].wide_share = all > 0.0 ? wide / all : 0.0;
+  }
   return FMB_OK;
 }
 
@@ -1262,7 +1290,7 @@ int fmbx_rcr_run(const fmb_plan *pl, int op, int kind, int l, int nrhs,
   j.chunks = pairs->d_chunks;
   j.nchunks = pairs->nchunks;
   j.chunk_pairs = RCR_CHUNK;
-  job_shape(tb, op, nrhs, &j);
+  job_shape(pl, tb, op, nrhs, pl->split, &j);
   j.H = o->d_Hpad;
   j.hstride = o->hpad_stride;
   j.C = tb->d_Cpad[op];
@@ -1330,7 +1358,7 @@ int fmbx_rcr_run_t(const fmb_plan *pl, int op, int kind, int l, int nrhs,
   j.chunks = pairs->d_chunks;
   j.nchunks = pairs->nchunks;
   j.chunk_pairs = RCR_CHUNK;
-  job_shape(tb, op, nrhs, &j);
+  job_shape(pl, tb, op, nrhs, pl->split, &j);
   j.H = o->d_Hpad;
   j.hstride = o->hpad_stride;
   j.C = tb->d_Cpad[op];
@@ -1401,7 +1429,7 @@ int fmb_plan_launch_shape(const fmb_plan *pl, int kind, int level, int prec, int
   } else if (tb->mode[op]) {
     j.nchunks = (kind == 0 ? tb : &pl->rcr[1][level])->nchunks;
     j.chunk_pairs = RCR_CHUNK;
-    job_shape(tb, op, nrhs, &j);
+    job_shape(pl, tb, op, nrhs, pl->aux != NULL, &j);
   }
   if (mode) *mode = j.mode;
   if (nt) *nt = j.nt;

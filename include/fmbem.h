@@ -264,11 +264,12 @@ int fmb_plan_retune(fmb_plan *pl, double k, const fmb_c64 *robin, void *stream);
 int fmb_plan_tile_shape(const fmb_plan *pl, int kind, int level, int prec, int *mode,
                         int *nt, int *mt, int *nw, int *bf, double *ms);
 /* Form of that translation in a pass of nrhs (1 .. nrhs_max) right-hand sides,
- * forward or transposed, as above: with waves and autotune 0, high orders and
- * launches of few workgroups take 8 waves (csrc/host/rcr.c), and M2L levels of
- * order 16 and less whose shape is not requested (rcr_mode, waves, ldso and
- * m2l_tile at their defaults) run target-stationary where that is faster
- * (csrc/hip/rcr_ts.hip): mode FMB_RCR_MODE_TS, nt 2, mt 0. */
+ * forward or transposed and not under capture, as above: with waves and
+ * autotune 0, high orders and launches of few workgroups take 8 waves
+ * (csrc/host/rcr.c), and M2L levels of order 16 and less whose shape is not
+ * requested (rcr_mode, waves, ldso and m2l_tile at their defaults) run
+ * target-stationary where that is faster (csrc/hip/rcr_ts.hip): mode
+ * FMB_RCR_MODE_TS, nt 2, mt 0. */
 int fmb_plan_launch_shape(const fmb_plan *pl, int kind, int level, int prec, int nrhs,
                           int *mode, int *nt, int *mt, int *nw, int *bf);
 /* Wavenumber of the operator the plan holds (0 after a failed retune). */

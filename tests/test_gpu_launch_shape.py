@@ -1,6 +1,7 @@
 """Plan.launch_shape: the form that a pass of so many right-hand sides takes,
 which the rule's shape (Plan.tile_shape) alone does not name."""
 import pytest
+import torch
 
 import fmbem_gpu_c_amd as F
 from conftest import wavenumber
@@ -50,3 +51,31 @@ def test_refusals(tree):
         assert e.value.code == -1
     valu = F.Plan(tree, wavenumber(4000.0), rcr_path=F.RCR_VALU)
     assert valu.launch_shape(0, 5, 1) == (0, 0, 0, 0, 0)
+
+
+def test_passes_on_two_streams_keep_to_four_waves(tree):
+    """FP64, several right-hand sides, and most of M2L's work in levels without
+    an 8-wave form: the streams hide more with 4 waves in every launch (327,680
+    triangles at 10 kHz with nine right-hand sides 326 ms, 341 with 8 waves).
+    Not with one right-hand side, on one stream, or with most of the work in
+    levels of that form."""
+    pairs = [len(tree.pairs(l)[0]) for l in range(2, 6)]
+
+    def share(orders):
+        w = [n * p ** 3 for n, p in zip(pairs, orders)]
+        return sum(w[:2]) / sum(w)
+
+    few, most = [44, 30, 21, 20], [94, 62, 21, 20]
+    assert share(few) < 0.45 and share(most) > 0.55
+    pl = _plan(tree, few, nrhs_max=4)
+    waves = lambda p, n: [p.launch_shape(0, l, n)[3] for l in range(2, 6)]  # noqa: E731
+    assert waves(pl, 1)[:2] == [8, 8] and waves(pl, 4) == [4, 4, 4, 4]
+    assert waves(_plan(tree, few, nrhs_max=4, serial_levels=1), 4)[:2] == [8, 8]
+    assert waves(_plan(tree, most, nrhs_max=4), 4)[:2] == [8, 8]
+    # FP32, whose batches take half the LDS, on either stream count
+    assert pl.launch_shape(0, 2, 4, F.FMB_MIXED)[3] == 8
+    x = torch.randn((4, pl.n), dtype=torch.complex128, device="cuda")
+    ref = _plan(tree, few, nrhs_max=4, serial_levels=1)
+    for fn in ("matvec", "matvec_t"):
+        a, b = getattr(pl, fn)(x), getattr(ref, fn)(x)
+        assert float(torch.linalg.norm(a - b) / torch.linalg.norm(b)) < 1e-13   # order of the sums
