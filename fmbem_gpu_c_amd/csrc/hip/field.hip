@@ -31,9 +31,10 @@ constexpr int kFieldSlicePts = 1024; // below this many point groups k_field sli
 // R right-hand sides at P field points a workgroup: a thread takes a panel for
 // all P, so that its 136 bytes, strided over the lanes, are read once for them
 // and the points' chains run beside each other.  81,920 panels at 32 points
-// with one right-hand side: 120 us at P = 1, 87 at 4.
+// with one right-hand side: 120 us at P = 1, 87 at 4.  (Several right-hand sides
+// at 168 VGPRs, for a third workgroup a CU, spill: 3-9% slower than at 181.)
 template <int P, int R>
-__global__ void __launch_bounds__(kT)
+__global__ void __launch_bounds__(kT, P * R > 1 ? 2 : 4)
     k_field(const double *__restrict__ pts, int npts, const double *__restrict__ tri,
             const double *__restrict__ geo, const int *__restrict__ perm, int N,
             double k, const double2 *__restrict__ robin,
@@ -55,50 +56,79 @@ __global__ void __launch_bounds__(kT)
     for (int r = 0; r < R; r++) acc[i][r] = make_double2(0.0, 0.0);
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  auto add = [&](int i, const double2 &S, const double2 &K, int j) {
+  // panel j's integrals S, K at point i times its values (Robin coefficient, right-hand sides)
+  struct Val {
+    double2 sg, v[R];
+  };
+  auto values = [&](int j) {
+    Val u;
+    u.sg = robin ? robin[j] : make_double2(0.0, 0.0);
+    const int c = perm[j];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      u.v[r] = r < nr ? x[(size_t)(r0 + r) * N + c] : make_double2(0.0, 0.0);
+    return u;
+  };
+  auto add = [&](int i, const double2 &S, const double2 &K, const Val &u) {
     double2 g = K;
     if (robin) {
-      const double2 sg = robin[j];
-      g.x -= sg.x * S.x - sg.y * S.y;
-      g.y -= sg.x * S.y + sg.y * S.x;
+      g.x -= u.sg.x * S.x - u.sg.y * S.y;
+      g.y -= u.sg.x * S.y + u.sg.y * S.x;
     }
-    const int c = perm[j];
 #pragma unroll
     for (int r = 0; r < R; r++) {
       if (r < nr) {
-        const double2 v = x[(size_t)(r0 + r) * N + c];
-        acc[i][r].x += g.x * v.x - g.y * v.y;
-        acc[i][r].y += g.x * v.y + g.y * v.x;
+        acc[i][r].x += g.x * u.v[r].x - g.y * u.v[r].y;
+        acc[i][r].y += g.x * u.v[r].y + g.y * u.v[r].x;
       }
     }
   };
-  for (int j0 = blockIdx.y * kT + 64 * w; j0 < N; j0 += nsl * kT) {
-    const int j = j0 + lane;
-    unsigned long long near[P];  // lanes whose panel is close to point i
-    if constexpr (P == 1) {
+  const double lim2 = ratio * ratio;
+  auto is_close = [&](int i, const double *g) {
+    const double dx = y[i][0] - g[0], dy = y[i][1] - g[1], dz = y[i][2] - g[2];
+    return dx * dx + dy * dy + dz * dz < lim2 * g[7] * g[7];
+  };
+  // panels of the refined rule, a point of the rule a lane (128 points next to a
+  // surface of 1,280 panels: 90 us with the rule by the lane of the panel, one
+  // point a workgroup; 137 with four points, one after the other; 64 now)
+  auto refined = [&](int i, int j0, unsigned long long near) {
+    for (; near; near &= near - 1) {
+      const int j = j0 + __ffsll(near) - 1;
+      const double *gj = geo + 8 * (size_t)j;
+      const Val u = values(j);
+      for (int q = lane; q < nqn; q += 64) {
+        double2 o[4];
+        panel_sum(k, y[i], nz, tri + 9 * (size_t)j, gj + 3, gj[6], quadn + 4 * q, 1, o);
+        add(i, o[0], o[1], u);
+      }
+    }
+  };
+  const int first = blockIdx.y * kT + 64 * w;  // the wave's first panel
+  if constexpr (P == 1) {
+    for (int j0 = first; j0 < N; j0 += nsl * kT) {
+      const int j = j0 + lane;
       const double *gj = geo + 8 * (size_t)min(j, N - 1);
-      const double dx = y[0][0] - gj[0], dy = y[0][1] - gj[1], dz = y[0][2] - gj[2];
-      const bool close = dx * dx + dy * dy + dz * dz < ratio * ratio * gj[7] * gj[7];
-      near[0] = __ballot(j < N && close);
+      const bool close = is_close(0, gj);
       if (j < N && !close) {
         double2 o[4];
         panel_sum(k, y[0], nz, tri + 9 * (size_t)j, gj + 3, gj[6], quad, nq, o);
-        add(0, o[0], o[1], j);
+        add(0, o[0], o[1], values(j));
       }
-    } else {
-      const double *gj = geo + 8 * (size_t)min(j, N - 1), *tr = tri + 9 * (size_t)min(j, N - 1);
+      refined(0, j0, __ballot(j < N && close));
+    }
+  } else {
+    // (the refined rule in a loop of its own: most wavefronts have no use for it)
+    bool met = false;
+    for (int j = first + lane; j < N; j += nsl * kT) {
+      const double *gj = geo + 8 * (size_t)j, *tr = tri + 9 * (size_t)j;
       double t[9], g8[8];
       for (int a = 0; a < 9; a++) t[a] = tr[a];
       for (int a = 0; a < 8; a++) g8[a] = gj[a];
-      const double lim = ratio * ratio * g8[7] * g8[7];
+      bool close[P];
       double2 S[P], K[P];  // int G, int dG/dn_y
-      bool far[P];
 #pragma unroll
       for (int i = 0; i < P; i++) {
-        const double dx = y[i][0] - g8[0], dy = y[i][1] - g8[1], dz = y[i][2] - g8[2];
-        const bool close = dx * dx + dy * dy + dz * dz < lim;
-        near[i] = __ballot(j < N && close);
-        far[i] = j < N && !close;
+        close[i] = is_close(i, g8);
         S[i] = K[i] = make_double2(0.0, 0.0);
       }
       for (int q = 0; q < nq; q++) {  // (panel_sum's S and K)
@@ -121,23 +151,19 @@ __global__ void __launch_bounds__(kT)
           K[i].y += wn * gpi;
         }
       }
+      const Val u = values(j);
 #pragma unroll
-      for (int i = 0; i < P; i++)
-        if (far[i]) add(i, S[i], K[i], j);
+      for (int i = 0; i < P; i++) {
+        met |= close[i];
+        if (!close[i]) add(i, S[i], K[i], u);
+      }
     }
-    // panels of the refined rule, a point of the rule a lane (128 points next to
-    // a surface of 1,280 panels: 90 us with the rule by the lane of the panel, one
-    // point a workgroup; 137 with four points, one after the other)
+    if (__any(met))
+      for (int j0 = first; j0 < N; j0 += nsl * kT) {
+        const int j = j0 + lane;
 #pragma unroll
-    for (int i = 0; i < P; i++)
-      for (; near[i]; near[i] &= near[i] - 1) {
-        const int jj = j0 + __ffsll(near[i]) - 1;
-        const double *gj = geo + 8 * (size_t)jj;
-        for (int q = lane; q < nqn; q += 64) {
-          double2 o[4];
-          panel_sum(k, y[i], nz, tri + 9 * (size_t)jj, gj + 3, gj[6], quadn + 4 * q, 1, o);
-          add(i, o[0], o[1], jj);
-        }
+        for (int i = 0; i < P; i++)
+          refined(i, j0, __ballot(j < N && is_close(i, geo + 8 * (size_t)min(j, N - 1))));
       }
   }
 #pragma unroll
