@@ -196,8 +196,9 @@ typedef struct fmb_plan_params {
                                 the M2L of the finest levels                */
   int waves;                 /* waves per workgroup of the matrix-core
                                 translations in the fixed tile-shape rule:
-                                4 or 8 (0: by the order and the launch's
-                                workgroups); autotune overrides it          */
+                                4 or 8 (0: by the order, the launch's
+                                workgroups and, in FP64, the streams of the
+                                pass); autotune overrides it                */
   int split_bf16;            /* FMB_MIXED plans: 1 runs the rotations of the
                                 FP32 pass's LDS-mode translations in
                                 split-BF16 (hi + lo bf16 operands, three
