@@ -31,10 +31,12 @@ constexpr int kFieldSlicePts = 1024; // below this many point groups k_field sli
 // R right-hand sides at P field points a workgroup: a thread takes a panel for
 // all P, so that its 136 bytes, strided over the lanes, are read once for them
 // and the points' chains run beside each other.  81,920 panels at 32 points
-// with one right-hand side: 120 us at P = 1, 87 at 4.  (Several right-hand sides
-// at 168 VGPRs, for a third workgroup a CU, spill: 3-9% slower than at 181.)
+// with one right-hand side: 120 us at P = 1, 87 at 4.  The refined rule
+// has a loop of its own, so that its registers do not cost the plain one a
+// workgroup a CU: two right-hand sides at 1,000 points, 20,480 panels, 757 us
+// in one loop (181 VGPRs), 655 in two (147).
 template <int P, int R>
-__global__ void __launch_bounds__(kT, P * R > 1 ? 2 : 4)
+__global__ void __launch_bounds__(kT, P > 1 ? 2 : R > 1 ? 3 : 4)
     k_field(const double *__restrict__ pts, int npts, const double *__restrict__ tri,
             const double *__restrict__ geo, const int *__restrict__ perm, int N,
             double k, const double2 *__restrict__ robin,
@@ -56,32 +58,25 @@ __global__ void __launch_bounds__(kT, P * R > 1 ? 2 : 4)
     for (int r = 0; r < R; r++) acc[i][r] = make_double2(0.0, 0.0);
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // panel j's integrals S, K at point i times its values (Robin coefficient, right-hand sides)
-  struct Val {
-    double2 sg, v[R];
-  };
-  auto values = [&](int j) {
-    Val u;
-    u.sg = robin ? robin[j] : make_double2(0.0, 0.0);
-    const int c = perm[j];
-#pragma unroll
-    for (int r = 0; r < R; r++)
-      u.v[r] = r < nr ? x[(size_t)(r0 + r) * N + c] : make_double2(0.0, 0.0);
-    return u;
-  };
-  auto add = [&](int i, const double2 &S, const double2 &K, const Val &u) {
+  // a panel's integrals S, K at point i, Robin coefficient sg, times its values val(r)
+  auto add = [&](int i, const double2 &S, const double2 &K, const double2 &sg, auto val) {
     double2 g = K;
     if (robin) {
-      g.x -= u.sg.x * S.x - u.sg.y * S.y;
-      g.y -= u.sg.x * S.y + u.sg.y * S.x;
+      g.x -= sg.x * S.x - sg.y * S.y;
+      g.y -= sg.x * S.y + sg.y * S.x;
     }
 #pragma unroll
     for (int r = 0; r < R; r++) {
       if (r < nr) {
-        acc[i][r].x += g.x * u.v[r].x - g.y * u.v[r].y;
-        acc[i][r].y += g.x * u.v[r].y + g.y * u.v[r].x;
+        const double2 v = val(r);
+        acc[i][r].x += g.x * v.x - g.y * v.y;
+        acc[i][r].y += g.x * v.y + g.y * v.x;
       }
     }
+  };
+  auto coeff = [&](int j) { return robin ? robin[j] : make_double2(0.0, 0.0); };
+  auto values = [&](int j) {
+    return [=, c = perm[j]](int r) { return x[(size_t)(r0 + r) * N + c]; };
   };
   const double lim2 = ratio * ratio;
   auto is_close = [&](int i, const double *g) {
@@ -90,36 +85,32 @@ __global__ void __launch_bounds__(kT, P * R > 1 ? 2 : 4)
   };
   // panels of the refined rule, a point of the rule a lane (128 points next to a
   // surface of 1,280 panels: 90 us with the rule by the lane of the panel, one
-  // point a workgroup; 137 with four points, one after the other; 64 now)
+  // point a workgroup; 137 with four points, one after the other; 66 now)
   auto refined = [&](int i, int j0, unsigned long long near) {
     for (; near; near &= near - 1) {
       const int j = j0 + __ffsll(near) - 1;
       const double *gj = geo + 8 * (size_t)j;
-      const Val u = values(j);
       for (int q = lane; q < nqn; q += 64) {
         double2 o[4];
         panel_sum(k, y[i], nz, tri + 9 * (size_t)j, gj + 3, gj[6], quadn + 4 * q, 1, o);
-        add(i, o[0], o[1], u);
+        add(i, o[0], o[1], coeff(j), values(j));
       }
     }
   };
   const int first = blockIdx.y * kT + 64 * w;  // the wave's first panel
-  if constexpr (P == 1) {
-    for (int j0 = first; j0 < N; j0 += nsl * kT) {
-      const int j = j0 + lane;
-      const double *gj = geo + 8 * (size_t)min(j, N - 1);
-      const bool close = is_close(0, gj);
-      if (j < N && !close) {
+  static_assert(P == 1 || R == 1, "v is the one right-hand side of several points");
+  bool met = false;
+  for (int j = first + lane; j < N; j += nsl * kT) {
+    if constexpr (P == 1) {
+      const double *gj = geo + 8 * (size_t)j;
+      if (is_close(0, gj)) {
+        met = true;
+      } else {
         double2 o[4];
         panel_sum(k, y[0], nz, tri + 9 * (size_t)j, gj + 3, gj[6], quad, nq, o);
-        add(0, o[0], o[1], values(j));
+        add(0, o[0], o[1], coeff(j), values(j));
       }
-      refined(0, j0, __ballot(j < N && close));
-    }
-  } else {
-    // (the refined rule in a loop of its own: most wavefronts have no use for it)
-    bool met = false;
-    for (int j = first + lane; j < N; j += nsl * kT) {
+    } else {
       const double *gj = geo + 8 * (size_t)j, *tr = tri + 9 * (size_t)j;
       double t[9], g8[8];
       for (int a = 0; a < 9; a++) t[a] = tr[a];
@@ -151,21 +142,21 @@ __global__ void __launch_bounds__(kT, P * R > 1 ? 2 : 4)
           K[i].y += wn * gpi;
         }
       }
-      const Val u = values(j);
+      const double2 sg = coeff(j), v = values(j)(0);
 #pragma unroll
       for (int i = 0; i < P; i++) {
         met |= close[i];
-        if (!close[i]) add(i, S[i], K[i], u);
+        if (!close[i]) add(i, S[i], K[i], sg, [&](int) { return v; });
       }
     }
-    if (__any(met))
-      for (int j0 = first; j0 < N; j0 += nsl * kT) {
-        const int j = j0 + lane;
-#pragma unroll
-        for (int i = 0; i < P; i++)
-          refined(i, j0, __ballot(j < N && is_close(i, geo + 8 * (size_t)min(j, N - 1))));
-      }
   }
+  if (__any(met))  // the refined rule
+    for (int j0 = first; j0 < N; j0 += nsl * kT) {
+      const int j = j0 + lane;
+#pragma unroll
+      for (int i = 0; i < P; i++)
+        refined(i, j0, __ballot(j < N && is_close(i, geo + 8 * (size_t)min(j, N - 1))));
+    }
 #pragma unroll
   for (int i = 0; i < P; i++)
 #pragma unroll
